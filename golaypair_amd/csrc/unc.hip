@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(256) k_unc_filter_fp32(UncTabs tb, int nsides,
                 const bool valid = s < S.p_suf;
                 float mx = 0.f;
                 if (valid) {
-                    const int8_t* e = ent + S.ent_off + s * nent;
+                    const int8_t* e = ent + S.suf_off + s * nent;
                     for (int k = 0; k < S.nch; ++k) {
                         const int t = k >> 4, row = k & 15;
                         float re = xpre[wv][t * 32 + row], im = xpre[wv][t * 32 + 16 + row];
@@ -495,57 +495,6 @@ __global__ void __launch_bounds__(64) k_emit_rows(const UncSide* __restrict__ si
         m, m, [&](int64_t i) { return surv[rows[i]]; }, sides, radix, tup, trig, bound, words, keys, groups, ties);
 }
 
-// One suffix operand table of the split filter: the B fragments of every
-// combination of the suffix positions' tuples (mixed-radix order, last
-// position fastest), laid out [tile][block][lane] as uint4 of 8 BF16 (entry
-// e = 16 block + 8 (lane / 32) + i of combination 32 tile + lane % 32, entry
-// e = x r + i being element i of suffix position x's tuple).  The tile count
-// is rounded up to even (the filter loads tiles in pairs); padding is zero.  `side` is a
-// table side with these positions and letters (its tuple rows are used).
-struct SufJob {
-    int64_t out_off;  // in uint4
-    int32_t side, npos, pos_off, pad;
-};
-
-__global__ void __launch_bounds__(256) k_build_suf(const SufJob* __restrict__ jobs, const int32_t* __restrict__ pos,
-                                                   const UncSide* __restrict__ sides,
-                                                   const int32_t* __restrict__ radix,
-                                                   const int8_t* __restrict__ tup, uint4* __restrict__ sufb) {
-    const SufJob J = jobs[blockIdx.x];
-    const UncSide& S = sides[J.side];
-    const int r = S.r, nent = J.npos * r, nbs = nent > 16 ? (nent + 15) / 16 : 1;
-    const int32_t* sp = pos + J.pos_off;
-    int64_t ps = 1;
-    for (int x = 0; x < J.npos; ++x) ps *= radix[S.radix_off + sp[x]];
-    const int64_t ntiles = (ps + 63) / 64 * 2;
-    uint4* out = sufb + J.out_off;
-    for (int64_t u = threadIdx.x; u < ntiles * nbs * 64; u += blockDim.x) {
-        const int lane = (int)(u & 63), blk = (int)((u >> 6) % nbs);
-        const int64_t tile = (u >> 6) / nbs;
-        const int64_t s0 = tile * 32 + (lane & 31);
-        uint32_t hv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (s0 < ps) {
-            int dg[kMaxN];
-            int64_t rest = s0;
-            for (int x = J.npos - 1; x >= 0; --x) {
-                const int R = radix[S.radix_off + sp[x]];
-                dg[x] = (int)(rest % R);
-                rest /= R;
-            }
-            for (int i8 = 0; i8 < 8; ++i8) {
-                const int e = 16 * blk + 8 * (lane >> 5) + i8;
-                if (e < nent) {
-                    const int x = e / r, i = e % r;
-                    const float v = (float)tup[S.tup_off + ((int64_t)sp[x] * S.rmax + dg[x]) * r + i];
-                    hv[i8] = __float_as_uint(v) >> 16;  // small integers are exact in BF16
-                }
-            }
-        }
-        out[u] = make_uint4(hv[0] | (hv[1] << 16), hv[2] | (hv[3] << 16), hv[4] | (hv[5] << 16),
-                            hv[6] | (hv[7] << 16));
-    }
-}
-
 // Records of one table side (unordered) -> compact list.
 __global__ void k_select_side(const uint64_t* __restrict__ surv, int64_t m, uint64_t sid,
                               unsigned long long* __restrict__ count, uint64_t* __restrict__ out) {
@@ -560,19 +509,6 @@ __global__ void k_select_side(const uint64_t* __restrict__ surv, int64_t m, uint
 
 namespace {
 
-uint16_t bf16_rne_u(float f) {
-    uint32_t u;
-    std::memcpy(&u, &f, 4);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-double bf16_d(uint16_t h) {
-    uint32_t u = (uint32_t)h << 16;
-    float f;
-    std::memcpy(&f, &u, 4);
-    return f;
-}
-
 // Per-side tables (concatenated over the sides of a call), views into the
 // batch's staging buffer.
 struct Tables {
@@ -583,35 +519,30 @@ struct Tables {
     uint64_t* pm1 = nullptr;
     int32_t* pos32 = nullptr;  // per side and position: block offsets into Shared
     int32_t* pos64 = nullptr;
-    int32_t* olist = nullptr;  // per side: outer positions (active, in order)
-    float* fix32 = nullptr;    // per side: FP32 sum of the single-split positions
+    int32_t* olist = nullptr;  // FP32 path, per side: outer positions (active, in order)
+    float* fix32 = nullptr;    // FP32 path, per side: FP32 sum of the single-split positions
     int64_t items = 0;
 };
 
-// Tables shared by every side of a call, content-addressed: the per-(position,
-// letter) DFT contribution blocks (FP32 channel layout and FP64 (Re, Im) pairs),
-// the MFMA A fragments and FP32 weights of each suffix start b, the mid tables of
-// each (a, b, letters at a..b-1) and the suffix operands of each (b, letters at b..L-1).
+// Tables shared by every side of a call: the per-(position, letter) DFT
+// contribution blocks (FP64 (Re, Im) pairs; FP32 path: also in its channel
+// layout) and, on the FP32 path, the weights of each suffix position set, the
+// mid tables and the suffix entries (content-addressed, filled on the host; the
+// split path's tables are built on the device by k_unc_tabs).
 struct Shared {
     std::vector<int> block;  // [position j][letter + 128] -> block id, -1 if absent
     std::vector<int32_t> off32, off64;
     std::vector<float> c32;
     std::vector<double> c64;
-    // suffix weight sets (one per distinct suffix position set): positions,
-    // offset into frags (split path) or w32 (FP32 path), max BF16 split residual
+    // FP32 path: suffix weight sets (one per distinct suffix position set), offset into w32
     std::vector<std::vector<int>> sets;
     std::vector<int64_t> set_off;
-    std::vector<double> set_rho;
-    int64_t n_frags = 0, n_w32 = 0, n_mid = 0, n_suf = 0;
+    int64_t n_w32 = 0, n_mid = 0, n_suf = 0;
     // views into the staging buffer
-    uint4* frags = nullptr;  // MFMA A fragments per suffix position set (split path)
-    float* w32 = nullptr;    // FP32 suffix weights (FP32 path)
+    float* w32 = nullptr;    // FP32 suffix weights
     float* mid = nullptr;    // mid tables
-    uint4* sufb = nullptr;   // suffix B operands (split path)
-    int8_t* ent = nullptr;   // suffix entries (FP32 path)
-    // FP32 filter channels: slot q (row q % 16 of M-tile q / 16) holds k = chan[q]
-    std::vector<int> chan;   // 0: an empty slot of the last M-tile (zero weights)
-    int lr = 8;              // registers per lane read in the last M-tile (8, 4 or 2)
+    int8_t* ent = nullptr;   // suffix entries
+    std::vector<int> chan;   // filter channels: k of channel q (FP32 path: row q % 16 of tile q / 16)
     int mt() const { return ((int)chan.size() + 15) / 16; }
     int id(int j, int letter) const {
         const int b = block[(size_t)j * 256 + (letter + 128)];
@@ -623,20 +554,27 @@ struct Shared {
 // The split of a side's leaf index over its active positions (more than one
 // split; single-split positions add a constant and digit 0 of radix 1, so the
 // leaf index of the DFS order is the mixed-radix number of the active digits):
-// suffix = the last active positions (p_suf >= 64, grown while the entries fit
-// the K blocks already used and p_suf stays <= 1024), mid = the active
-// positions before it (16 <= p_mid <= 4096 where possible), outer = the rest.
+// suffix = the last active positions, mid = the active positions before it,
+// outer = the rest.
 struct Split {
     std::vector<int> out, mid, suf;  // position indices, ascending
     int64_t po = 1, pm = 1, ps = 1;
     int nent = 0;
 };
 
-Split side_split(const SideHost& S) {
-    Split X;
+std::vector<int> active_positions(const SideHost& S) {
     std::vector<int> act;
     for (int j = 0; j < S.L; ++j)
         if (S.R[j] > 1) act.push_back(j);
+    return act;
+}
+
+// FP32 path: the suffix reaches p_suf >= 64 and grows while its entries fit the
+// 16-entry blocks already used and p_suf stays <= 1024; 16 <= p_mid <= 4096
+// where possible.
+Split side_split_fp32(const SideHost& S) {
+    Split X;
+    const std::vector<int> act = active_positions(S);
     int k = (int)act.size();
     while (k > 0) {
         const int j = act[k - 1];
@@ -654,6 +592,43 @@ Split side_split(const SideHost& S) {
     X.mid.assign(act.begin() + a, act.begin() + k);
     X.out.assign(act.begin(), act.begin() + a);
     for (int j : X.out) X.po *= S.R[j];
+    return X;
+}
+
+// Split path: the suffix with the least work of k_unc_filter (in its vector
+// instructions per block, for items of 256 rows: per tile of 32 suffix columns
+// 8 per channel and row tile and about 40 for the decisions; per item about 15
+// per channel and row tile for the row features and 400 to begin), among those
+// of at most 1024 combinations (always at least one position).  The mid
+// table holds at least one position and at most 4096 rows where it can; the
+// outer part takes the rest and the single-split positions.
+Split side_split_quad(const SideHost& S, int chp) {
+    Split X;
+    const std::vector<int> act = active_positions(S);
+    int best = (int)act.size();
+    double best_cost = 0;
+    int64_t ps = 1;
+    for (int k = (int)act.size(); k >= 0; --k) {
+        if (k < (int)act.size()) {
+            ps *= S.R[act[k]];
+            if (ps > 1024 && k + 1 < (int)act.size()) break;
+        }
+        const double rows = (double)S.leaves / (double)ps;
+        const double items = std::ceil(rows / kRowsPerItem), tiles = (double)((ps + 31) / 32);
+        const double cost = items * (tiles * 2.0 * (8.0 * chp + 40.0) + 30.0 * chp + 400.0);
+        if (k == (int)act.size() || k + 1 == (int)act.size() || cost < best_cost) {
+            best = k;
+            best_cost = cost;
+            X.ps = ps;
+        }
+    }
+    X.suf.assign(act.begin() + best, act.end());
+    int a = best;
+    while (a > 0 && (X.pm == 1 || X.pm * S.R[act[a - 1]] <= 4096)) X.pm *= S.R[act[--a]];
+    X.mid.assign(act.begin() + a, act.begin() + best);
+    X.po = (int64_t)(S.leaves / (uint64_t)(X.pm * X.ps));
+    for (int j = 0; j < S.L; ++j)
+        if (S.R[j] == 1 || j < (a < (int)act.size() ? act[a] : S.L)) X.out.push_back(j);
     return X;
 }
 
@@ -683,7 +658,6 @@ void build_mid(const Shared& SH, const SideHost& S, const std::vector<int>& mp, 
         }
         for (size_t q = 0; q < SH.chan.size(); ++q) {
             const int k = SH.chan[q], t = (int)q / 16, row = (int)q % 16;
-            if (k <= 0) continue;  // empty slot
             out[m * mt * 32 + t * 32 + row] = (float)acc[2 * (k - 1)];
             out[m * mt * 32 + t * 32 + 16 + row] = (float)acc[2 * (k - 1) + 1];
         }
@@ -694,75 +668,29 @@ void build_mid(const Shared& SH, const SideHost& S, const std::vector<int>& mp, 
     }
 }
 
-// Suffix operands of (suffix positions, letters): BF16 B fragments
-// [ntiles][nbs][64] (split path) or int8 entries [p_suf][nent] (FP32 path).
-// Entry e = x r + i is element i of the tuple of suffix position x; suffix
+// FP32 path: int8 entries [p_suf][nent] of (suffix positions, letters).  Entry
+// e = x r + i is element i of the tuple of suffix position x; suffix
 // combinations in mixed-radix order, last position fastest.
-void build_suf(const SideHost& S, const std::vector<int>& sp, bool fp32, uint4* sufb, int8_t* ent) {
+void build_ent(const SideHost& S, const std::vector<int>& sp, int8_t* ent) {
     const int r = S.r, nent = (int)sp.size() * r;
     int64_t ps = 1;
     for (int j : sp) ps *= (int64_t)S.R[j];
     std::vector<int> sdg(sp.size(), 0);
-    std::vector<int8_t> vals((size_t)ps * std::max(nent, 1), 0);
     for (int64_t s = 0; s < ps; ++s) {
-        for (int e = 0; e < nent; ++e) vals[s * nent + e] = S.tuple(sp[e / r], sdg[e / r])[e % r];
+        for (int e = 0; e < nent; ++e) ent[s * nent + e] = S.tuple(sp[e / r], sdg[e / r])[e % r];
         for (int x = (int)sp.size() - 1; x >= 0; --x) {
             if (++sdg[x] < S.R[sp[x]]) break;
             sdg[x] = 0;
         }
     }
-    if (fp32) {
-        std::copy(vals.begin(), vals.end(), ent);
-        return;
-    }
-    // BF16 of every int8 value (exact: |v| <= 128 has at most 8 significant bits)
-    static const std::array<uint16_t, 256> bf = [] {
-        std::array<uint16_t, 256> t{};
-        for (int v = -128; v < 128; ++v) t[v + 128] = bf16_rne_u((float)v);
-        return t;
-    }();
-    const int nbs = std::max(1, (nent + 15) / 16);
-    const int ntiles = (int)((ps + 63) / 64 * 2);  // even: tiles go in pairs
-    for (int tile = 0; tile < ntiles; ++tile)
-        for (int blk = 0; blk < nbs; ++blk)
-            for (int lane = 0; lane < 64; ++lane) {
-                uint16_t hv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                const int64_t s = (int64_t)tile * 32 + lane % 32;
-                if (s < ps)
-                    for (int i8 = 0; i8 < 8; ++i8) {
-                        const int e = 16 * blk + 8 * (lane / 32) + i8;
-                        if (e < nent) hv[i8] = bf[vals[s * nent + e] + 128];
-                    }
-                uint4 q;
-                q.x = hv[0] | ((uint32_t)hv[1] << 16);
-                q.y = hv[2] | ((uint32_t)hv[3] << 16);
-                q.z = hv[4] | ((uint32_t)hv[5] << 16);
-                q.w = hv[6] | ((uint32_t)hv[7] << 16);
-                *sufb++ = q;
-            }
-}
-
-// Element counts of the mid and suffix tables of a split (their layouts above).
-int64_t mid_size(const Split& X, int mt) { return X.pm * mt * 32; }
-int64_t suf_size(const Split& X, bool fp32) {
-    if (fp32) return X.ps * std::max(X.nent, 1);
-    return ((X.ps + 63) / 64 * 2) * std::max(1, (X.nent + 15) / 16) * 64;
 }
 
 // FP32 suffix DFT weights of the suffix positions, [nent][mt*32] (FP32 path).
-// Registers a new suffix position set `sp`: its offset and size in w32 (FP32
-// path) or frags (split path); returns its index.
-int add_set(Shared& SH, const std::vector<int>& sp, int r, bool fp32) {
-    const int nent = (int)sp.size() * r, nbs = std::max(1, (nent + 15) / 16);
+// Registers a new suffix position set `sp`; returns its index.
+int add_set(Shared& SH, const std::vector<int>& sp, int r) {
     SH.sets.push_back(sp);
-    SH.set_rho.push_back(0.0);
-    if (fp32) {
-        SH.set_off.push_back(SH.n_w32);
-        SH.n_w32 += (int64_t)nent * SH.mt() * 32;
-    } else {
-        SH.set_off.push_back(SH.n_frags);
-        SH.n_frags += (int64_t)SH.mt() * 2 * nbs * 64;
-    }
+    SH.set_off.push_back(SH.n_w32);
+    SH.n_w32 += (int64_t)sp.size() * r * SH.mt() * 32;
     return (int)SH.sets.size() - 1;
 }
 
@@ -788,9 +716,9 @@ void build_w32(const Shared& SH, int set, int L, int r, int N, const std::vector
 }
 
 // Blocks of every position j < L and every letter of the split table: the DFT
-// contributions of each of the position's tuples (FP64 (Re, Im) for all k, and
-// the FP32 filter channels).
-void add_blocks(Shared& SH, const SplitTable& X, int L, int N, const std::vector<double>& cs,
+// contributions of each of the position's tuples (FP64 (Re, Im) for all k and, on
+// the FP32 path, its filter channels).
+void add_blocks(Shared& SH, const SplitTable& X, int L, int N, bool fp32, const std::vector<double>& cs,
                 const std::vector<double>& sn) {
     const int r = X.r, K = N / 2, mt = SH.mt();
     SH.block.assign((size_t)L * 256, -1);
@@ -801,9 +729,8 @@ void add_blocks(Shared& SH, const SplitTable& X, int L, int N, const std::vector
             SH.block[(size_t)j * 256 + (letter + 128)] = (int)SH.off32.size();
             SH.off32.push_back((int32_t)SH.c32.size());
             SH.off64.push_back((int32_t)SH.c64.size());
-            SH.c32.resize(SH.c32.size() + (size_t)std::max(R, 1) * mt * 32, 0.f);
+            if (fp32) SH.c32.resize(SH.c32.size() + (size_t)std::max(R, 1) * mt * 32, 0.f);
             SH.c64.resize(SH.c64.size() + (size_t)std::max(R, 1) * 2 * K, 0.0);
-            float* c32 = &SH.c32[SH.off32.back()];
             double* c64 = &SH.c64[SH.off64.back()];
             for (int d = 0; d < R; ++d)
                 for (int k = 1; k <= K; ++k) {
@@ -817,76 +744,15 @@ void add_blocks(Shared& SH, const SplitTable& X, int L, int N, const std::vector
                     c64[((int64_t)d * K + (k - 1)) * 2] = re;
                     c64[((int64_t)d * K + (k - 1)) * 2 + 1] = im;
                 }
+            if (!fp32) continue;
+            float* c32 = &SH.c32[SH.off32.back()];
             for (int d = 0; d < R; ++d)
                 for (size_t q = 0; q < SH.chan.size(); ++q) {
                     const int k = SH.chan[q], t = (int)q / 16, row = (int)q % 16;
-                    if (k <= 0) continue;  // empty slot
                     c32[(int64_t)d * mt * 32 + t * 32 + row] = (float)c64[((int64_t)d * K + (k - 1)) * 2];
                     c32[(int64_t)d * mt * 32 + t * 32 + 16 + row] = (float)c64[((int64_t)d * K + (k - 1)) * 2 + 1];
                 }
         }
-}
-
-// Writes the MFMA A fragments of set `set`; returns the largest BF16 split
-// residual |w - hi - lo| of its weights.  32x32x16 layout: lane l holds
-// A[row l % 32][entry 8 (l / 32) + i] (rows 0..15 Re, 16..31 Im of the tile's
-// channel slots).  The last tile of the small-tile class (unc_small_last_tile)
-// is a 16x16x32 operand, lane l holding A[m = l % 16][k = 8 (l / 16) + i]: its
-// B operand is the 32x32 one read as 16x16x32, k = 8 g + i (g = l / 16) being
-// entry 8 (g / 2) + i of leaf 16 (g % 2) + n, so row m = 4 G + c (G = m / 4)
-// holds, for leaves 16 (G % 2) + n only (k groups g with g % 2 == G % 2), the
-// Re (c even) or Im (c odd) weights of channel slot 4 (G / 2) + c / 2.  Output
-// lane l then holds leaf l % 32's two channels of slots 4 (l / 32) + {0, 1}.
-double build_frags(const Shared& SH, int set, int L, int r, int N, const std::vector<double>& cs,
-                   const std::vector<double>& sn) {
-    const std::vector<int>& sp = SH.sets[set];
-    const int mt = SH.mt(), nent = (int)sp.size() * r, nbs = std::max(1, (nent + 15) / 16);
-    const bool small = unc_small_last_tile(nbs, mt, SH.lr);
-    uint4* out = SH.frags + SH.set_off[set];
-    double rho = 0;
-    for (int t = 0; t < mt; ++t)
-        for (int st = 0; st < 2 * nbs; ++st)
-            for (int lane = 0; lane < 64; ++lane) {
-                uint16_t hv[8];
-                for (int i8 = 0; i8 < 8; ++i8) {
-                    int e, slot;
-                    bool im;
-                    if (small && t == mt - 1) {
-                        const int m = lane % 16, G = m / 4, c = m % 4, g = lane / 16;
-                        e = (G % 2 == g % 2) ? 8 * (g / 2) + i8 : nent;  // other half of the leaves: zero
-                        slot = 4 * (G / 2) + c / 2;
-                        im = (c % 2) != 0;
-                    } else {
-                        const int row = lane % 32;
-                        e = 16 * (st % nbs) + 8 * (lane / 32) + i8;
-                        slot = row % 16;
-                        im = row >= 16;
-                    }
-                    const int part = st / nbs;
-                    const size_t qs = 16 * t + slot;
-                    uint16_t v = 0;
-                    if (e < nent && qs < SH.chan.size() && SH.chan[qs] > 0) {
-                        const int k = SH.chan[qs];
-                        const int j = sp[e / r], i = e % r;
-                        const int p = j + L * i;
-                        const int mm = (int)(((int64_t)k * p) % N);
-                        const double w = im ? sn[mm] : cs[mm];
-                        const uint16_t hi = bf16_rne_u((float)w);
-                        const double r1 = w - bf16_d(hi);
-                        const uint16_t lo = bf16_rne_u((float)r1);
-                        rho = std::max(rho, std::fabs(r1 - bf16_d(lo)));
-                        v = part ? lo : hi;
-                    }
-                    hv[i8] = v;
-                }
-                uint4 q;
-                q.x = hv[0] | ((uint32_t)hv[1] << 16);
-                q.y = hv[2] | ((uint32_t)hv[3] << 16);
-                q.z = hv[4] | ((uint32_t)hv[5] << 16);
-                q.w = hv[6] | ((uint32_t)hv[7] << 16);
-                *out++ = q;
-            }
-    return rho;
 }
 
 // Where one side's rows go in the batch tables (filled by add_side on host threads).
@@ -894,7 +760,25 @@ struct SideSlot {
     int sid = 0;
     bool pm1 = false;
     int64_t item_base = 0, radix_off = 0, tup_off = 0, pm1_off = -1, pos_off = 0, olist_off = 0, fix_off = 0;
+    int64_t xout_off = 0;
 };
+
+// max |x_p| sums over the words of a side: the sum over its positions of the
+// largest sum of |entries| of a split.
+double pos_s1(const SideHost& S, int j) {
+    double m = 0;
+    for (int d = 0; d < S.R[j]; ++d) {
+        double ab = 0;
+        for (int i = 0; i < S.r; ++i) ab += std::abs(S.tuple(j, d)[i]);
+        m = std::max(m, ab);
+    }
+    return m;
+}
+double side_s1(const SideHost& S) {
+    double s = 0;
+    for (int j = 0; j < S.L; ++j) s += pos_s1(S, j);
+    return s;
+}
 
 // Whether every tuple entry of the side is +-1 (words then carry +1 bit masks).
 bool side_pm1(const SideHost& S) {
@@ -907,7 +791,7 @@ bool side_pm1(const SideHost& S) {
 }
 
 void add_side(Tables& T, const SideSlot& Z, const Shared& SH, const SideHost& S, const Split& X, int rmax,
-              int order, int paf, int group, bool fp32, int64_t mid_off, int64_t suf_off, int set) {
+              int order, int paf, int group, bool fp32, double scale, int64_t mid_off, int64_t suf_off, int set) {
     UncSide D{};
     D.L = S.L; D.r = S.r; D.N = S.N; D.K = S.N / 2; D.seqflag = S.seqflag; D.rmax = rmax;
     D.group = group;
@@ -918,13 +802,14 @@ void add_side(Tables& T, const SideSlot& Z, const Shared& SH, const SideHost& S,
     D.nout = (int32_t)X.out.size();
     D.nent = X.nent;
     D.p_suf = ps; D.p_mid = pm; D.p_out = po; D.leaves = (int64_t)S.leaves;
-    D.nbs = std::max(1, (X.nent + 15) / 16);
-    D.ntiles = (int)((ps + 31) / 32);
     D.item_base = Z.item_base;
-    D.olist_off = Z.olist_off;
-    for (size_t x = 0; x < X.out.size(); ++x) T.olist[Z.olist_off + x] = X.out[x];
-    // single-split positions: one constant, FP64 sum rounded once to FP32
-    {
+    D.xout_off = Z.xout_off;
+    D.mid_off = mid_off;
+    D.suf_off = suf_off;
+    if (fp32) {
+        D.olist_off = Z.olist_off;
+        for (size_t x = 0; x < X.out.size(); ++x) T.olist[Z.olist_off + x] = X.out[x];
+        // single-split positions: one constant, FP64 sum rounded once to FP32
         const int K = N / 2;
         double acc[2 * kMaxK] = {};
         for (int j = 0; j < L; ++j)
@@ -935,10 +820,10 @@ void add_side(Tables& T, const SideSlot& Z, const Shared& SH, const SideHost& S,
         D.fix_off = Z.fix_off;
         for (size_t q = 0; q < SH.chan.size(); ++q) {
             const int k = SH.chan[q], t = (int)q / 16, row = (int)q % 16;
-            if (k <= 0) continue;  // empty slot
             T.fix32[D.fix_off + t * 32 + row] = (float)acc[2 * (k - 1)];
             T.fix32[D.fix_off + t * 32 + 16 + row] = (float)acc[2 * (k - 1) + 1];
         }
+        D.w32_off = SH.set_off[set];
     }
     D.radix_off = Z.radix_off;
     for (int j = 0; j < L; ++j) T.radix[Z.radix_off + j] = S.R[j];
@@ -960,43 +845,39 @@ void add_side(Tables& T, const SideSlot& Z, const Shared& SH, const SideHost& S,
     D.c64_off = Z.pos_off;
     for (int j = 0; j < L; ++j) {
         const int id = SH.id(j, S.orig[j]);
-        T.pos32[Z.pos_off + j] = SH.off32[id];
+        if (fp32) T.pos32[Z.pos_off + j] = SH.off32[id];
         T.pos64[Z.pos_off + j] = SH.off64[id];
     }
-    D.mid_off = mid_off;
-    D.sufb_off = fp32 ? 0 : suf_off;
-    D.ent_off = fp32 ? suf_off : 0;
-    D.w32_off = fp32 ? SH.set_off[set] : 0;
-    // A fragments (suffix DFT weights, BF16 hi and lo), shared per suffix position set
-    D.frag_off = fp32 ? 0 : SH.set_off[set];
-    const double rho = fp32 ? 0.0 : SH.set_rho[set];
     bool in_suf[kMaxN] = {};
     for (int j : X.suf) in_suf[j] = true;
     // error bound of the filter's Re/Im
     double s1_pre = 0, s1_suf = 0;
-    for (int j = 0; j < L; ++j) {
-        double mxabs = 0;
-        for (int d = 0; d < S.R[j]; ++d) {
-            double ab = 0;
-            for (int i = 0; i < r; ++i) ab += std::abs(S.tuple(j, d)[i]);
-            mxabs = std::max(mxabs, ab);
-        }
-        (in_suf[j] ? s1_suf : s1_pre) += mxabs;
-    }
-    const double u24 = 0x1p-24, u23 = 0x1p-23;
-    double E;
-    if (!fp32)
-        E = (D.nout + 4) * u24 * s1_pre * 1.01                              // fixed + X_outer + Mid rounding (FP32)
-            + s1_suf * rho * 1.0000001                                      // BF16 split residual
-            + 1.004 * (32.0 * D.nbs + 1.0) * u23 * (s1_pre + s1_suf);       // MFMA accumulation
-    else
-        E = (D.nout + 4) * u24 * s1_pre * 1.01 + s1_suf * u24 * 1.01         // FP32 weights
-            + (X.nent + 1.0) * u24 * (s1_pre + s1_suf) * 1.01;              // FP32 FMAs
+    for (int j = 0; j < L; ++j) (in_suf[j] ? s1_suf : s1_pre) += pos_s1(S, j);
+    const double u24 = 0x1p-24, u23 = 0x1p-23, u22 = 0x1p-22;
     const double thr = 2.0 * order - paf + 0.001;
-    const double eps = psd_eps(E, thr);
+    double t = thr, eps;
+    if (!fp32) {
+        // Bound on | P' - |X|^2 | near the threshold (|X| <= R there, so |s| <= s1_suf
+        // and |c| <= R + |s|), all in scaled units: FP32 accumulation of the 12
+        // products (whose magnitudes sum to at most (|c| + |s|)^2), the dropped and
+        // rounded parts of the cross terms, |c|^2 in FP32, the FP32 rounding of the
+        // three sums that make c, and parts below the smallest normal f16.
+        // In these units |X| <= 128 (the choice of `scale`): a threshold above 150^2 accepts
+        // every leaf as 150^2 does, and is below kFeatBig, which no leaf reaches.
+        t = std::min(scale * scale * thr, 150.0 * 150.0);
+        const double R = std::min(std::sqrt(scale * scale * std::max(thr + 1.0, 0.0)), 130.0), sf = scale * s1_suf;
+        const double m = R + 2.0 * sf, c = R + sf;
+        const double d = 4.04 * u24 * scale * (s1_pre + s1_suf) * 1.42;
+        eps = 1.004 * 13.0 * u23 * m * m + 6.06 * u22 * c * sf + 3.03 * u24 * c * c + 2.0 * R * d + d * d +
+              0x1p-20 * (m + 1.0);
+    } else {
+        const double E = (D.nout + 4) * u24 * s1_pre * 1.01 + s1_suf * u24 * 1.01  // FP32 weights
+                         + (X.nent + 1.0) * u24 * (s1_pre + s1_suf) * 1.01;        // FP32 FMAs
+        eps = psd_eps(E, thr);
+    }
     D.thr = thr;
-    D.thr_hi = std::nextafter((float)(thr + eps), INFINITY);
-    D.thr_lo = std::nextafter((float)(thr - eps), -INFINITY);
+    D.thr_hi = std::nextafter((float)(t + eps), INFINITY);
+    D.thr_lo = std::nextafter((float)(t - eps), -INFINITY);
     T.sides[Z.sid] = D;
 }
 
@@ -1012,14 +893,6 @@ V* upload(gp_ctx* ctx, const char* name, const std::vector<V>& v) {
 // ---------------------------------------------------------------------------
 // host: the three stages
 
-// Sides of one operand class of the split filter kernel, contiguous in table order.
-struct UncClass {
-    int nbs = 0, mt = 0;
-    int lr = 8;  // registers per lane read in the last M-tile (8, 4 or 2)
-    int sid_lo = 0, sid_hi = 0;
-    int64_t item_lo = 0, item_hi = 0;
-};
-
 // Host tables of one batch (built without the device, so that the next batch's
 // tables can be prepared while the current batch runs).
 struct UncPrep {
@@ -1030,10 +903,11 @@ struct UncPrep {
     Tables T;
     Shared SH;
     std::vector<int> side_of;
-    std::vector<UncClass> classes;
+    UncChan chan{};        // split path: filter channels
+    double scale = 1.0;    // split path: a power of two that keeps |X|^2 in the range of f16
     uint64_t total_leaves = 0;
     uint64_t dead_leaves = 0;  // leaves of sides rejected by their fixed channels
-    int64_t n_suf_jobs = 0, n_sufb = 0;  // split path: suffix operand jobs and their size (uint4)
+    int64_t n_tab_blocks = 0, n_suf = 0, n_mid = 0, n_xout = 0;  // split path: sizes of the device-built tables
     // every table in one staging buffer (one host-to-device copy): pinned
     // (`stage`) or, when prepared without a pool, `host` until unc_stage
     PinnedBuf* stage = nullptr;
@@ -1051,8 +925,8 @@ namespace {
 
 // Staging buffer regions, in upload order (sizes in bytes).
 enum StageRegion {
-    kStSides, kStRadix, kStTup, kStPm1, kStC64, kStPos64, kStPos32, kStOlist, kStFix32, kStC32,
-    kStMid, kStSufJobs, kStSufPos, kStFrags, kStEnt, kStW32, kStToff, kStCount
+    kStSides, kStItems, kStRadix, kStTup, kStPm1, kStC64, kStPos64, kStTabJobs, kStTabBlocks, kStTabPos, kStToff,
+    kStPos32, kStOlist, kStFix32, kStC32, kStMid, kStEnt, kStW32, kStCount
 };
 
 }  // namespace
@@ -1066,24 +940,21 @@ void unc_stage(UncPrep& U, PinnedPool& pool) {
     U.host.reset();
 }
 
-template <int NBS, int MT, int LR>
-void launch_filter_t(const UncClass& c, int64_t rounds, int cls, int nsub, dim3 grid, hipStream_t st,
-                     const UncTabs& tb, UncCtl* ctl, uint64_t* surv, int64_t scap, uint64_t* band, int64_t bcap) {
-    hipLaunchKernelGGL((k_unc_filter<NBS, MT, LR>), grid, dim3(256), 0, st, tb, c.sid_lo, c.sid_hi, c.item_lo,
-                       c.item_hi, rounds, cls, nsub, ctl, surv, scap, band, bcap);
-}
-
-void launch_filter_class(const UncClass& c, int64_t rounds, int cls, int nsub, dim3 grid, hipStream_t st,
-                         const UncTabs& tb, UncCtl* ctl, uint64_t* surv, int64_t scap, uint64_t* band, int64_t bcap) {
-#define GP_FILTER_CASE(NB, M, LR)                \
-    if (c.nbs == NB && c.mt == M && c.lr == LR) \
-        return launch_filter_t<NB, M, LR>(c, rounds, cls, nsub, grid, st, tb, ctl, surv, scap, band, bcap);
-#define GP_FILTER_LR(NB, M) GP_FILTER_CASE(NB, M, 8) GP_FILTER_CASE(NB, M, 4) GP_FILTER_CASE(NB, M, 2)
-    GP_FILTER_LR(1, 1) GP_FILTER_LR(2, 1) GP_FILTER_LR(3, 1) GP_FILTER_LR(4, 1)
-    GP_FILTER_LR(1, 2) GP_FILTER_LR(2, 2) GP_FILTER_LR(3, 2) GP_FILTER_LR(4, 2)
-#undef GP_FILTER_LR
+// The split filter of `pairs` channel pairs on `grid` blocks.
+void launch_filter(int pairs, dim3 grid, hipStream_t st, const UncTabs& tb, int64_t nitems, int64_t rounds, int nsub,
+                   UncCtl* ctl, uint64_t* surv, int64_t scap, uint64_t* band, int64_t bcap) {
+#define GP_FILTER_CASE(NP)                                                                                       \
+    case NP:                                                                                                     \
+        hipLaunchKernelGGL((k_unc_filter<NP>), grid, dim3(256), 0, st, tb, nitems, rounds, nsub, ctl, surv, scap, \
+                           band, bcap);                                                                          \
+        break;
+    switch (pairs) {
+        GP_FILTER_CASE(1) GP_FILTER_CASE(2) GP_FILTER_CASE(3) GP_FILTER_CASE(4) GP_FILTER_CASE(5) GP_FILTER_CASE(6)
+        GP_FILTER_CASE(7) GP_FILTER_CASE(8) GP_FILTER_CASE(9) GP_FILTER_CASE(10) GP_FILTER_CASE(11)
+        GP_FILTER_CASE(12) GP_FILTER_CASE(13) GP_FILTER_CASE(14) GP_FILTER_CASE(15) GP_FILTER_CASE(16)
+        default: throw ArgError("uncompress: no filter kernel for this number of channels");
+    }
 #undef GP_FILTER_CASE
-    throw ArgError("uncompress: no filter kernel for this operand class");
 }
 
 UncTrig unc_trig(gp_ctx* ctx, int N) {
@@ -1172,43 +1043,29 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         if (all_channels)
             for (size_t i = 0; i < sides.size(); ++i)
                 if (sides[i].leaves != 0) live.push_back(i);
-        // filter channels by slot: full M-tiles in order; in the last M-tile its
-        // c real channels go to rows (i mod lr) + 4 (i / lr), lr the fewest
-        // registers per lane (2, 4 or 8) that hold them, and the other slots hold
-        // 0 (no channel: zero weights, never read)
-        std::vector<int> real;
         for (int k = 1; k <= K; ++k)
-            if (all_channels || k % r != 0) real.push_back(k);
-        const int mtr = ((int)real.size() + 15) / 16;
-        const int last = (int)real.size() - 16 * (mtr - 1);
-        SH.lr = last <= 4 ? 2 : last <= 8 ? 4 : 8;
-        SH.chan.assign(real.begin(), real.begin() + 16 * (mtr - 1));
-        if (SH.lr == 8) {
-            SH.chan.insert(SH.chan.end(), real.begin() + 16 * (mtr - 1), real.end());
-        } else {
-            std::vector<int> tile(8, 0);
-            for (int i = 0; i < last; ++i) tile[(i % SH.lr) + 4 * (i / SH.lr)] = real[16 * (mtr - 1) + i];
-            while (!tile.empty() && tile.back() == 0) tile.pop_back();
-            SH.chan.insert(SH.chan.end(), tile.begin(), tile.end());
-        }
+            if (all_channels || k % r != 0) SH.chan.push_back(k);
+        const int chp = ((int)SH.chan.size() + 1) & ~1;  // split path: channels in pairs
+        U.chan.n = chp;
+        for (size_t q = 0; q < SH.chan.size(); ++q) U.chan.k[q] = (int8_t)SH.chan[q];
         // shared per-(position, letter) blocks; per side its split and table keys
         Phase ph1("tables: splits + keys");
-        if (!live.empty()) add_blocks(SH, *sides[live[0]].tab, sides[live[0]].L, N, cs, sn);
+        if (!live.empty()) add_blocks(SH, *sides[live[0]].tab, sides[live[0]].L, N, fp32, cs, sn);
         std::vector<Split> spl(live.size());
         std::vector<std::string> kmid(live.size()), ksuf(live.size());
         std::vector<char> pm1(live.size());
         parallel(live.size(), [&](size_t q) {
             const SideHost& S = sides[live[q]];
-            spl[q] = side_split(S);
+            spl[q] = fp32 ? side_split_fp32(S) : side_split_quad(S, chp);
             kmid[q] = pos_key(S, spl[q].mid);
             ksuf[q] = pos_key(S, spl[q].suf);
             pm1[q] = side_pm1(S);
         });
         U.all_pm1 = std::all_of(pm1.begin(), pm1.end(), [](char b) { return b != 0; });
         ph1.next("tables: layout");
-        // content-addressed suffix weight sets (key: the suffix positions, the
-        // first half of the suffix key), mid and suffix tables (built below, in
-        // parallel): one per distinct key
+        // content-addressed mid and suffix tables and, on the FP32 path, suffix
+        // weight sets (key: the suffix positions, the first half of the suffix
+        // key): one per distinct key
         std::unordered_map<std::string_view, int> set_of, mid_job, suf_job;
         set_of.reserve(64);
         mid_job.reserve(live.size());
@@ -1216,10 +1073,12 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         std::vector<size_t> mid_rep, suf_rep;  // representative side (index into live) per job
         std::vector<int> side_mid(live.size()), side_suf(live.size()), side_set(live.size());
         for (size_t q = 0; q < live.size(); ++q) {
-            const std::string_view kpos(ksuf[q].data(), ksuf[q].size() / 2);
-            auto it = set_of.find(kpos);
-            if (it == set_of.end()) it = set_of.emplace(kpos, add_set(SH, spl[q].suf, sides[live[q]].r, fp32)).first;
-            side_set[q] = it->second;
+            if (fp32) {
+                const std::string_view kpos(ksuf[q].data(), ksuf[q].size() / 2);
+                auto it = set_of.find(kpos);
+                if (it == set_of.end()) it = set_of.emplace(kpos, add_set(SH, spl[q].suf, sides[live[q]].r)).first;
+                side_set[q] = it->second;
+            }
             auto im = mid_job.emplace(kmid[q], (int)mid_rep.size());
             if (im.second) mid_rep.push_back(q);
             side_mid[q] = im.first->second;
@@ -1233,43 +1092,34 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         std::vector<int64_t> mid_off(mid_rep.size()), suf_off(suf_rep.size());
         for (size_t i = 0; i < mid_rep.size(); ++i) {
             mid_off[i] = SH.n_mid;
-            SH.n_mid += mid_size(spl[mid_rep[i]], SH.mt());
+            SH.n_mid += fp32 ? spl[mid_rep[i]].pm * SH.mt() * 32 : spl[mid_rep[i]].pm * chp;
         }
         for (size_t i = 0; i < suf_rep.size(); ++i) {
             suf_off[i] = SH.n_suf;
-            SH.n_suf += suf_size(spl[suf_rep[i]], fp32);
+            SH.n_suf += fp32 ? spl[suf_rep[i]].ps * std::max(spl[suf_rep[i]].nent, 1)
+                             : (spl[suf_rep[i]].ps + 31) / 32 * chp * 64;
         }
-        // table order: sides grouped by operand class (one kernel instantiation each)
+        // table order: sides by decreasing cost of one work item (its suffix tiles),
+        // the kernel hands the items out in this order to the first free block; equal
+        // ones by suffix table, so that blocks at work together read the same one
         const int mtc = SH.mt();
-        auto cls = [&](size_t q) { return std::max(1, (spl[q].nent + 15) / 16); };
         std::vector<size_t> torder(live.size());
         std::iota(torder.begin(), torder.end(), 0);
-        // within a class, sides by decreasing cost of one work item (mid rows x suffix tile
-        // pairs): the kernel hands the items out in this order to the first free wave
-        auto item_cost = [&](size_t q) { return spl[q].pm * ((spl[q].ps + 63) / 64); };
-        std::stable_sort(torder.begin(), torder.end(), [&](size_t x, size_t y) {
-            if (cls(x) != cls(y)) return cls(x) < cls(y);
-            return item_cost(x) > item_cost(y);
-        });
+        if (!fp32)
+            std::stable_sort(torder.begin(), torder.end(), [&](size_t x, size_t y) {
+                const int64_t tx = (spl[x].ps + 31) / 32, ty = (spl[y].ps + 31) / 32;
+                if (tx != ty) return tx > ty;
+                return side_suf[x] < side_suf[y];
+            });
         std::vector<SideSlot> slot(live.size());
-        int64_t n_radix = 0, n_tup = 0, n_pm1 = 0, n_pos = 0, n_olist = 0, n_fix = 0;
+        int64_t n_radix = 0, n_tup = 0, n_pm1 = 0, n_pos = 0, n_olist = 0, n_fix = 0, n_xout = 0;
         for (size_t x = 0; x < torder.size(); ++x) {
             const size_t q = torder[x];
             const SideHost& S = sides[live[q]];
-            const int nbs = cls(q);
-            if (U.classes.empty() || U.classes.back().nbs != nbs) {
-                UncClass c;
-                c.nbs = nbs;
-                c.mt = mtc;
-                c.lr = SH.lr;
-                c.sid_lo = c.sid_hi = (int)x;
-                c.item_lo = c.item_hi = T.items;
-                U.classes.push_back(c);
-            }
             SideSlot& Z = slot[q];
             Z.sid = (int)x;
             Z.item_base = T.items;
-            T.items += spl[q].po;
+            T.items += fp32 ? spl[q].po : (spl[q].po * spl[q].pm + kRowsPerItem - 1) / kRowsPerItem;
             Z.radix_off = n_radix;
             n_radix += S.L;
             Z.tup_off = n_tup;
@@ -1281,14 +1131,17 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
             }
             Z.pos_off = n_pos;
             n_pos += S.L;
-            Z.olist_off = n_olist;
-            n_olist += (int64_t)spl[q].out.size();
-            Z.fix_off = n_fix;
-            n_fix += (int64_t)mtc * 32;
+            if (fp32) {
+                Z.olist_off = n_olist;
+                n_olist += (int64_t)spl[q].out.size();
+                Z.fix_off = n_fix;
+                n_fix += (int64_t)mtc * 32;
+            } else {
+                Z.xout_off = n_xout;
+                n_xout += spl[q].po * chp;
+            }
             side_of.push_back((int)live[q]);
             total_leaves += S.leaves;
-            U.classes.back().sid_hi = (int)x + 1;
-            U.classes.back().item_hi = T.items;
         }
         T.nsides = (int64_t)live.size();
         if (T.nsides == 0) return prep;
@@ -1300,21 +1153,35 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         bytes[kStPm1] = n_pm1 * sizeof(uint64_t);
         bytes[kStC64] = SH.c64.size() * sizeof(double);
         bytes[kStPos64] = n_pos * sizeof(int32_t);
-        bytes[kStPos32] = n_pos * sizeof(int32_t);
-        bytes[kStOlist] = n_olist * sizeof(int32_t);
-        bytes[kStFix32] = n_fix * sizeof(float);
-        bytes[kStC32] = SH.c32.size() * sizeof(float);
-        bytes[kStMid] = SH.n_mid * sizeof(float);
-        // split path: suffix operands are built on the device from a job list
-        int64_t n_sufpos = 0;
-        if (!fp32)
-            for (size_t i = 0; i < suf_rep.size(); ++i) n_sufpos += (int64_t)spl[suf_rep[i]].suf.size();
-        bytes[kStSufJobs] = fp32 ? 0 : suf_rep.size() * sizeof(SufJob);
-        bytes[kStSufPos] = n_sufpos * sizeof(int32_t);
-        bytes[kStFrags] = SH.n_frags * sizeof(uint4);
-        bytes[kStEnt] = fp32 ? SH.n_suf : 0;
-        bytes[kStW32] = SH.n_w32 * sizeof(float);
         bytes[kStToff] = sizeof(int64_t);
+        // split path: every table is built on the device from a job list
+        std::vector<TabJob> jobs;
+        int64_t n_tabpos = 0;
+        if (!fp32) {
+            auto add = [&](int type, size_t q, const std::vector<int>& pos, int64_t count, int64_t off) {
+                jobs.push_back(TabJob{type, slot[q].sid, (int32_t)pos.size(), (int32_t)n_tabpos, count, off});
+                n_tabpos += (int64_t)pos.size();
+                U.n_tab_blocks += (count + kTabSlice - 1) / kTabSlice;
+            };
+            for (size_t i = 0; i < suf_rep.size(); ++i) add(0, suf_rep[i], spl[suf_rep[i]].suf, spl[suf_rep[i]].ps, suf_off[i]);
+            for (size_t i = 0; i < mid_rep.size(); ++i) add(1, mid_rep[i], spl[mid_rep[i]].mid, spl[mid_rep[i]].pm, mid_off[i]);
+            for (size_t q = 0; q < live.size(); ++q) add(2, q, spl[q].out, spl[q].po, slot[q].xout_off);
+            U.n_suf = SH.n_suf;
+            U.n_mid = SH.n_mid;
+            U.n_xout = n_xout;
+            bytes[kStItems] = T.items * sizeof(UncItem);
+            bytes[kStTabJobs] = jobs.size() * sizeof(TabJob);
+            bytes[kStTabBlocks] = U.n_tab_blocks * sizeof(TabBlock);
+            bytes[kStTabPos] = n_tabpos * sizeof(int32_t);
+        } else {
+            bytes[kStPos32] = n_pos * sizeof(int32_t);
+            bytes[kStOlist] = n_olist * sizeof(int32_t);
+            bytes[kStFix32] = n_fix * sizeof(float);
+            bytes[kStC32] = SH.c32.size() * sizeof(float);
+            bytes[kStMid] = SH.n_mid * sizeof(float);
+            bytes[kStEnt] = SH.n_suf;
+            bytes[kStW32] = SH.n_w32 * sizeof(float);
+        }
         U.stage_off.assign(kStCount, 0);
         size_t total = 0;
         for (int i = 0; i < kStCount; ++i) {
@@ -1323,9 +1190,8 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         }
         U.stage_bytes = total;
         if (std::getenv("GOLAY_PROFILE"))
-            std::fprintf(stderr, "[golay] staging: %.2f MB (suffix operands %.2f MB, mid %.2f MB, sides %.2f MB)\n",
-                         total / 1e6, bytes[kStEnt] / 1e6, bytes[kStMid] / 1e6,
-                         bytes[kStSides] / 1e6);
+            std::fprintf(stderr, "[golay] staging: %.2f MB (sides %.2f MB); suffix features %.2f MB\n", total / 1e6,
+                         bytes[kStSides] / 1e6, fp32 ? 0.0 : SH.n_suf * 16e-6);
         if (pinned) {
             U.stage = pinned->acquire(total);
             U.stage_pool = pinned;
@@ -1344,23 +1210,26 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         T.olist = static_cast<int32_t*>(at(kStOlist));
         T.fix32 = static_cast<float*>(at(kStFix32));
         SH.mid = static_cast<float*>(at(kStMid));
-        U.n_suf_jobs = fp32 ? 0 : (int64_t)suf_rep.size();
-        U.n_sufb = fp32 ? 0 : SH.n_suf;
         if (!fp32) {
-            auto* jobs = static_cast<SufJob*>(at(kStSufJobs));
-            auto* spos = static_cast<int32_t*>(at(kStSufPos));
-            int64_t po = 0;
-            for (size_t i = 0; i < suf_rep.size(); ++i) {
-                const Split& X = spl[suf_rep[i]];
-                jobs[i] = SufJob{suf_off[i], slot[suf_rep[i]].sid, (int32_t)X.suf.size(), (int32_t)po, 0};
-                for (int j : X.suf) spos[po++] = j;
+            auto* items = static_cast<UncItem*>(at(kStItems));
+            for (size_t q : torder) {
+                const int64_t n = (spl[q].po * spl[q].pm + kRowsPerItem - 1) / kRowsPerItem;
+                for (int64_t b = 0; b < n; ++b) *items++ = UncItem{slot[q].sid, (uint32_t)b};
             }
+            std::memcpy(at(kStTabJobs), jobs.data(), bytes[kStTabJobs]);
+            auto* blk = static_cast<TabBlock*>(at(kStTabBlocks));
+            for (size_t i = 0; i < jobs.size(); ++i)
+                for (int64_t b = 0; b * kTabSlice < jobs[i].count; ++b) *blk++ = TabBlock{(int32_t)i, (uint32_t)b};
+            auto* tp = static_cast<int32_t*>(at(kStTabPos));
+            auto put = [&](const std::vector<int>& pos) { tp = std::copy(pos.begin(), pos.end(), tp); };
+            for (size_t q : suf_rep) put(spl[q].suf);
+            for (size_t q : mid_rep) put(spl[q].mid);
+            for (size_t q = 0; q < live.size(); ++q) put(spl[q].out);
         }
-        SH.frags = static_cast<uint4*>(at(kStFrags));
         SH.ent = static_cast<int8_t*>(at(kStEnt));
         SH.w32 = static_cast<float*>(at(kStW32));
         std::memcpy(at(kStC64), SH.c64.data(), bytes[kStC64]);
-        std::memcpy(at(kStC32), SH.c32.data(), bytes[kStC32]);
+        if (fp32) std::memcpy(at(kStC32), SH.c32.data(), bytes[kStC32]);
         std::memcpy(at(kStToff), &U.trig_off, sizeof(int64_t));
         // rows that add_side leaves unwritten: tuples and masks d >= R[j] (never
         // read) and the fixed-sum padding channels (read as 0)
@@ -1372,25 +1241,29 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
             before_fill();
         }
         ph1.next("tables: fill");
-        // every table built in place on host threads: weight sets, mid and suffix
-        // tables, then the per-side rows (which need the sets' BF16 residuals)
+        // FP32 path: every table built in place on host threads
         const size_t nset = SH.sets.size();
         const int r0 = sides[live[0]].r, L0 = sides[live[0]].L;
         auto fill_one = [&](size_t i) {
             if (i < nset) {
-                if (fp32) build_w32(SH, (int)i, L0, r0, N, cs, sn);
-                else SH.set_rho[i] = build_frags(SH, (int)i, L0, r0, N, cs, sn);
+                build_w32(SH, (int)i, L0, r0, N, cs, sn);
             } else if (i < nset + mid_rep.size()) {
                 const size_t k = i - nset, q = mid_rep[k];
                 build_mid(SH, sides[live[q]], spl[q].mid, SH.mid + mid_off[k]);
             } else {
                 const size_t k = i - nset - mid_rep.size(), q = suf_rep[k];
-                build_suf(sides[live[q]], spl[q].suf, true, nullptr, SH.ent + suf_off[k]);
+                build_ent(sides[live[q]], spl[q].suf, SH.ent + suf_off[k]);
             }
         };
-        parallel(nset + mid_rep.size() + (fp32 ? suf_rep.size() : 0), fill_one);
+        if (fp32) parallel(nset + mid_rep.size() + suf_rep.size(), fill_one);
+        // split path: the scale of the features (S1 bounds every |X| of the batch)
+        if (!fp32) {
+            double s1 = 0;
+            for (size_t q = 0; q < live.size(); ++q) s1 = std::max(s1, side_s1(sides[live[q]]));
+            while (U.scale * s1 > 128.0) U.scale *= 0.5;
+        }
         parallel(live.size(), [&](size_t q) {
-            add_side(T, slot[q], SH, sides[live[q]], spl[q], rmax, order, paf, group[live[q]], fp32,
+            add_side(T, slot[q], SH, sides[live[q]], spl[q], rmax, order, paf, group[live[q]], fp32, U.scale,
                      mid_off[side_mid[q]], suf_off[side_suf[q]], side_set[q]);
         });
     }
@@ -1438,26 +1311,33 @@ UncTabs upload_tables(gp_ctx* ctx, UncPrep& U, const std::string& name, UncBatch
     B.d_c64 = static_cast<const double*>(at(kStC64));
     B.d_pos64 = static_cast<const int32_t*>(at(kStPos64));
     *d_toff = static_cast<const int64_t*>(at(kStToff));
-    // split path: the suffix operands, built on the device from the job list
-    uint4* sufb = nullptr;
-    if (U.n_suf_jobs > 0) {
-        sufb = static_cast<uint4*>(ctx->buf(name + ".sufb").ensure((size_t)U.n_sufb * sizeof(uint4)));
-        hipLaunchKernelGGL(k_build_suf, dim3((unsigned)U.n_suf_jobs), dim3(256), 0, ctx->stream,
-                           static_cast<const SufJob*>(at(kStSufJobs)), static_cast<const int32_t*>(at(kStSufPos)),
-                           B.d_sides, B.d_radix, B.d_tup, sufb);
+    UncTabs tb{};
+    tb.sides = B.d_sides;
+    tb.radix = B.d_radix;
+    if (!U.fp32) {
+        // the tables that the device builds from the job list
+        uint4* suf = ctx->dev<uint4>(name + ".suf", (size_t)U.n_suf);
+        float2* mid = ctx->dev<float2>(name + ".mid", (size_t)U.n_mid);
+        float2* xout = ctx->dev<float2>(name + ".xout", (size_t)U.n_xout);
+        hipLaunchKernelGGL(k_unc_tabs, dim3((unsigned)U.n_tab_blocks), dim3(256), 0, ctx->stream,
+                           static_cast<const TabBlock*>(at(kStTabBlocks)), static_cast<const TabJob*>(at(kStTabJobs)),
+                           static_cast<const int32_t*>(at(kStTabPos)), B.d_sides, B.d_radix, B.d_pos64, B.d_c64,
+                           U.chan, U.scale, xout, mid, suf);
         GP_HIP(hipGetLastError());
+        tb.items = static_cast<const UncItem*>(at(kStItems));
+        tb.suf = suf;
+        tb.mid2 = mid;
+        tb.xout = xout;
+    } else {
+        tb.pos32 = static_cast<const int32_t*>(at(kStPos32));
+        tb.olist = static_cast<const int32_t*>(at(kStOlist));
+        tb.c32 = static_cast<const float*>(at(kStC32));
+        tb.mid = static_cast<const float*>(at(kStMid));
+        tb.fix32 = static_cast<const float*>(at(kStFix32));
+        tb.ent = static_cast<const int8_t*>(at(kStEnt));
+        tb.w32 = static_cast<const float*>(at(kStW32));
     }
-    return UncTabs{B.d_sides,
-                   B.d_radix,
-                   static_cast<const int32_t*>(at(kStPos32)),
-                   static_cast<const int32_t*>(at(kStOlist)),
-                   static_cast<const float*>(at(kStC32)),
-                   static_cast<const float*>(at(kStMid)),
-                   static_cast<const float*>(at(kStFix32)),
-                   sufb,
-                   static_cast<const uint4*>(at(kStFrags)),
-                   static_cast<const int8_t*>(at(kStEnt)),
-                   static_cast<const float*>(at(kStW32))};
+    return tb;
 }
 
 // The filter kernels of one batch on the context's stream.
@@ -1465,55 +1345,18 @@ void launch_filters(gp_ctx* ctx, const UncPrep& U, const UncTabs& tb, UncCtl* ct
                     uint64_t* d_band, int64_t bcap) {
     hipStream_t st = ctx->stream;
     if (!U.fp32) {
-        if (U.classes.size() > 4) throw ArgError("uncompress: more than 4 operand classes in a batch");
-        for (size_t ci = 0; ci < U.classes.size(); ++ci) {
-            const UncClass& c = U.classes[ci];
-            // as many waves as the class keeps resident (its occupancy hint, 4 SIMDs per CU)
-            const int cap = unc_waves_per_simd(c.nbs, c.mt, c.lr);
-            const int per_simd = (int)std::clamp<int64_t>(tuned(ctx, "unc_waves/" + std::to_string(U.N), cap), 1, cap);
-            const int64_t waves = std::min<int64_t>(c.item_hi - c.item_lo, (int64_t)ctx->num_cus * 4 * per_simd);
-            const dim3 grid((unsigned)std::max<int64_t>(1, (waves + 3) / 4));
-            // items by wave index for all but the last `tail` rounds, which go out through
-            // the work counters (by default every item goes through them)
-            const int64_t W = (int64_t)grid.x * 4;
-            const int64_t tail = tuned(ctx, "unc_counter_rounds/" + std::to_string(U.N), (int64_t)1 << 40);
-            const int64_t rounds = std::max<int64_t>(0, (c.item_hi - c.item_lo) / W - tail);
-            const int64_t nsub = std::clamp<int64_t>(tuned(ctx, "unc_counter_streams/" + std::to_string(U.N),
-                                                           kSubCounters), 1, std::min<int64_t>(kSubCounters, grid.x));
-            if (std::getenv("GOLAY_PROFILE")) {
-                // leaf-tiles per wave as the kernel hands items out (the fixed rounds, then
-                // each counter stream's items to whichever of its waves is free first):
-                // mean and heaviest wave
-                std::vector<double> cost;
-                for (int sd = c.sid_lo; sd < c.sid_hi; ++sd) {
-                    const UncSide& S = U.T.sides[sd];
-                    cost.insert(cost.end(), (size_t)S.p_out, (double)S.p_mid * (double)(2 * ((S.ntiles + 1) / 2)));
-                }
-                std::vector<double> fixed((size_t)W, 0.0);
-                for (int64_t k = 0; k < rounds; ++k)
-                    for (int64_t w = 0; w < W; ++w) fixed[(size_t)w] += cost[(size_t)(k * W + ((k & 1) ? W - 1 - w : w))];
-                double total = 0, mx = 0;
-                for (size_t k = 0; k < cost.size(); ++k) total += cost[k];
-                for (int64_t j = 0; j < nsub; ++j) {
-                    std::priority_queue<double, std::vector<double>, std::greater<double>> load;
-                    for (int64_t w = 0; w < W; ++w)
-                        if ((w / 4) % nsub == j) load.push(fixed[(size_t)w]);
-                    for (int64_t k = rounds * W + j; k < (int64_t)cost.size(); k += nsub) {
-                        const double l = cost[(size_t)k] + load.top();
-                        load.pop();
-                        load.push(l);
-                    }
-                    while (!load.empty()) {
-                        mx = std::max(mx, load.top());
-                        load.pop();
-                    }
-                }
-                std::fprintf(stderr, "[golay] filter class <%d,%d,%d>: %lld items on %lld waves, tiles per wave mean "
-                             "%.0f, max %.0f (x%.3f)\n", c.nbs, c.mt, c.lr, (long long)(c.item_hi - c.item_lo),
-                             (long long)W, total / (double)W, mx, mx * (double)W / std::max(total, 1.0));
-            }
-            launch_filter_class(c, rounds, (int)ci, (int)nsub, grid, st, tb, ctl, d_surv, scap, d_band, bcap);
-        }
+        // as many blocks (one wave per SIMD each) as stay resident
+        const int pairs = U.chan.n / 2, cap = unc_waves_per_simd(pairs);
+        const int per_cu = (int)std::clamp<int64_t>(tuned(ctx, "unc_waves/" + std::to_string(U.N), cap), 1, cap);
+        const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>(U.T.items, (int64_t)ctx->num_cus * per_cu));
+        // items by block index for all but the last `tail` rounds, which go out through
+        // the work counters (by default every item goes through them)
+        const int64_t tail = tuned(ctx, "unc_counter_rounds/" + std::to_string(U.N), (int64_t)1 << 40);
+        const int64_t rounds = std::max<int64_t>(0, U.T.items / blocks - tail);
+        const int64_t nsub = std::clamp<int64_t>(tuned(ctx, "unc_counter_streams/" + std::to_string(U.N), kSubCounters),
+                                                 1, std::min<int64_t>(kSubCounters, blocks));
+        launch_filter(pairs, dim3((unsigned)blocks), st, tb, U.T.items, rounds, (int)nsub, ctl, d_surv, scap, d_band,
+                      bcap);
     } else {
         const int64_t waves = std::min<int64_t>(U.T.items, (int64_t)ctx->num_cus * 8);
         const dim3 grid((unsigned)std::max<int64_t>(1, (waves + 3) / 4));
@@ -1532,7 +1375,7 @@ void add_filter_stats(gp_stats* stats, const UncPrep& U, const UncCtl& h, float 
     stats->tie_band += h.ties;
     stats->psd_kernel_ms += ms_filter;
     stats->band_kernel_ms += ms_band;
-    stats->psd_launches += U.fp32 ? 1 : U.classes.size();
+    stats->psd_launches += 1;
     stats->kernel_ms += ms_filter + ms_band;
 }
 
@@ -1583,6 +1426,7 @@ UncBatch unc_launch(gp_ctx* ctx, UncPrep& U, gp_stats* stats) {
         if ((int64_t)h.surv > scap) { scap = (int64_t)h.surv + 1024; continue; }
         break;
     }
+    if ((int64_t)h.surv > scap || (int64_t)h.band > bcap) throw std::runtime_error("uncompress: survivor list overflow");
     B.nsurv = (int64_t)h.surv;
     B.d_surv = ctx->buf("u_surv").as<uint64_t>();
     add_filter_stats(stats, U, h, ms_filter, ms_band);

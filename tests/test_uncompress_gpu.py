@@ -290,3 +290,28 @@ def test_uncompress_batch_graph_matches_eager(gpu_ctx, monkeypatch, batch_leaves
         assert "".join(g.pair_line(x, y) + "\n" for x, y in zip(oa, ob)) == want, mode
         assert "".join(l + "\n" for l in ta.lines()) == open(os.path.join(wd, "uncompress_tmp_a")).read()
         assert st.tie_band == 0
+
+
+@pytest.mark.parametrize("L,c,c2,free,paf,seed", [
+    (3, 2, 1, (0, 0, 0), -20, 6),                   # 1 channel pair, fewer rows than a wave
+    (5, 3, 1, (1, -1, 1, -1, 1), -10, 4),           # odd channel count
+    (8, 4, 2, (0, 0, 0, 0, 0), -40, 37),
+    (6, 5, 1, (3, 3, -3, 3, -3, -3), -100, 4),
+    (15, 3, 1, (1, -1, 1, 1, -1, 1, -1, 1), -40, 4),
+    (12, 5, 1, (1, -1, 3, 3, -3), -135, 47),        # 12 channel pairs
+    (9, 7, 1, (1, -3, 3), -129, 41),                # 14
+    (32, 2, 1, (0,) * 11, -20, 23),
+    (15, 3, 1, (1, -1, 1, 1, -1, 1), -165, 51),     # the largest threshold
+    (15, 3, 1, (1, -1, 1, 1, -1, 1), 90, 51),       # the smallest
+])
+def test_uncompress_side_filter_tiles(gpu_ctx, L, c, c2, free, paf, seed):
+    """The filter's tiles of 64 rows and 32 columns with remainders of both and its
+    channel pairs, with thresholds that accept all, some or none of the leaves."""
+    rng = np.random.default_rng(seed)
+    seq = np.where(rng.integers(0, 2, L) == 0, c, -c).astype(np.int8)  # single-split letters
+    seq[rng.permutation(L)[:len(free)]] = free
+    for seqflag in (0, 1):
+        ref_text, ref_leaves = _oracle.uncompress_side(seq, c, c2, paf, seqflag)
+        cands, rot, st = gpu_ctx.uncompress_side(seq, c, c2, paf, seqflag)
+        assert "".join(l + "\n" for l in cands.lines()) == ref_text
+        assert st.psd_decisions == ref_leaves
