@@ -556,8 +556,7 @@ double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nr
 //
 // Everything the call needs beyond the caller's words and pass flags lives in
 // `scratch`, one file-scope device array per GPU, held until the process ends:
-//   [0, 256)                  NaHead: band / tie / pass counters, the row-sum
-//                             bound S1, the thresholds and the table descriptor
+//   [0, 256)                  NaHead: band / tie / pass counters (calls that want stats)
 //   [256, 256 + 16 KiB)       the split-BF16 A fragments of the word length
 //   [.., + 1 KiB)             its FP64 twiddles.
 // Host code refers to it only through the address hipGetSymbolAddress gives
@@ -567,12 +566,8 @@ double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nr
 namespace gp {
 
 struct NaHead {
-    BandCtl ctl;                  // band rows rechecked by k_na_band, FP64 ties
+    BandCtl ctl;                  // band rows settled in FP64, FP64 ties
     unsigned long long passed;    // rows accepted
-    unsigned int s1;              // max over the rows of sum |x_p|
-    unsigned int pad;
-    FilterThr thr;
-    PsdTableDesc desc;            // frag_off = trig_off = 0: the regions below
 };
 constexpr size_t kNaHeadBytes = 256;
 constexpr size_t kNaFragCount = 2 * 8 * 64;  // M-tiles (<= 2) x 2 nb (<= 8) x 64 lanes, n <= 64
@@ -604,60 +599,167 @@ __global__ void k_na_reset(NaHead* h) {
         h->ctl.count = 0;
         h->ctl.ties = 0;
         h->passed = 0;
-        h->s1 = 0;
     }
 }
 
-// S1 = max over the rows of sum |x_p| (the row-sum bound of the error analysis).
-__global__ void __launch_bounds__(256) k_na_s1(const int8_t* __restrict__ words, int stride, int n, int64_t count,
-                                               NaHead* h) {
-    unsigned int best = 0;
-    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < count; r += (int64_t)gridDim.x * blockDim.x) {
-        const int8_t* w = words + r * stride;
-        unsigned int a = 0;
-        for (int p = 0; p < n; ++p) a += (unsigned int)abs((int)w[p]);
-        best = max(best, a);
+// The two thresholds of a row with s1 = sum |x_p|:
+//   hi = hi0 + a s1 + b s1^2,  lo = lo0 - a s1 - b s1^2
+// hold thr +- psd_eps(s1 E1, thr) (E1 = split_bf16_E for s1 = 1) and the FP32
+// rounding of these sums.
+struct NaThr {
+    double thr;
+    float hi0, lo0, a, b;
+};
+
+NaThr na_thr(const PsdTableDesc& d, double thr) {
+    if (thr < 0) return NaThr{thr, -1.f, -1.f, 0.f, 0.f};  // |X|^2 >= 0: every row is rejected
+    const double E1 = split_bf16_E(d, 1.0), r = std::sqrt(2.0 * (thr + 1.0)) * 1.000001;
+    const double b = 2.0 * E1 * E1, a = 2.0 * E1 * r;
+    const double smax = 128.0 * kMaxN, top = thr + 1.0 + a * smax + b * smax * smax;
+    const double eps0 = psd_eps(0.0, thr) + 4.0 * 0x1p-24 * top;
+    return NaThr{thr, std::nextafter((float)(thr + eps0), INFINITY), std::nextafter((float)(thr - eps0), -INFINITY),
+                 std::nextafter((float)a, INFINITY), std::nextafter((float)b, INFINITY)};
+}
+
+// Waves of k_na_filter that stay resident with n's operand class (from its
+// registers: 4, 3 or 2 per SIMD); each streams one run of rows, and more of them
+// would run after the first.
+int64_t na_waves(const PsdTableDesc& d, int num_cus) {
+    return (int64_t)num_cus * 4 * (d.mt == 1 ? 4 : d.nb == 3 ? 3 : 2);
+}
+
+// FP64 max PSD of the row at w by the whole wave: lane q < n / 2 takes k = q + 1
+// in the summation order of fp64_max_psd; the result is in every lane.
+__device__ __forceinline__ double na_wave_max_psd(const int8_t* __restrict__ w, int n, const double* tw, int lane) {
+    const int x = lane < n ? (int)w[lane] : 0;
+    const int k = lane < (n >> 1) ? lane + 1 : 0;  // (idle lanes: k = 0, their value is dropped)
+    double re = 0.0, im = 0.0;
+    int m = 0;
+    for (int p = 0; p < n; ++p) {
+        const double v = (double)__builtin_amdgcn_readlane(x, p);
+        re = __builtin_fma(v, tw[m], re);
+        im = __builtin_fma(v, tw[n + m], im);
+        m += k;
+        if (m >= n) m -= n;
     }
-    for (int o = 32; o; o >>= 1) best = max(best, (unsigned int)__shfl_xor((int)best, o));
-    if ((threadIdx.x & 63) == 0) atomicMax(&h->s1, best);
+    double mx = k ? re * re + im * im : 0.0;
+    for (int o = 32; o; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    return mx;
 }
 
-// Thresholds from S1 as the host path makes them (split_bf16_E, make_thr).
-__global__ void k_na_thr(NaHead* h, double thr) {
-    if (threadIdx.x != 0) return;
-    const double adds = 32.0 * h->desc.nb + 1.0;
-    const double E = (double)h->s1 * ((double)h->desc.rho_max + 1.004 * adds * 0x1p-23);
-    const double eps = psd_eps(E, thr);
-    h->thr.thr = thr;
-    h->thr.hi = nextafterf((float)(thr + eps), INFINITY);
-    h->thr.lo = nextafterf((float)(thr - eps), -INFINITY);
-}
-
-// Rows left in the band by k_psd_mfma are settled in FP64 in place; accepted
-// rows are counted.
-__global__ void __launch_bounds__(256) k_na_band(const int8_t* __restrict__ words, int stride, int64_t count,
-                                                 const double* __restrict__ trig64, NaHead* h,
-                                                 uint8_t* __restrict__ pass) {
-    const int n = h->desc.n;
-    const double t = h->thr.thr;
-    unsigned long long nb = 0, nt = 0, npass = 0;
-    for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < count; base += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = base + threadIdx.x;
-        unsigned long long acc = 0;
-        if (r < count) {
-            uint8_t d = pass[r];
-            if (d == kBand) {
-                const double m = fp64_max_psd(words + r * stride, n, trig64, trig64 + n);
-                ++nb;
-                nt += fabs(m - t) < 1e-9;
-                d = m > t ? kReject : kAccept;
-                pass[r] = d;
-            }
-            acc = d == kAccept;
+// The whole filter of one word length in one pass over the rows, tiles of 32
+// rows in pairs as in k_psd_mfma.  The error bound of a row needs its sum
+// |x_p|: four letters per v_sad_u8 on the letters the wave holds anyway, so a
+// row has its own thresholds and no pass over the rows comes first.  Rows in the
+// band are settled in FP64 at once: one at a time by the whole wave, or, when a
+// pair of tiles holds many, one per lane.
+// Bound by reading the rows.  A call with n = 25 and 8e6 rows of 32 bytes takes
+// 69 us (3.8 TB/s with launch and wait) against 591 us in five kernels, 430 of
+// them for a pass of byte loads that found the largest row sum; one of 4099 rows
+// with n = 10 takes 16 us against 65.
+template <int NB, int MT>
+__global__ void __launch_bounds__(256) k_na_filter(const int8_t* __restrict__ words, int64_t stride, int n,
+                                                   int64_t count, int64_t tpw, const uint4* __restrict__ frags,
+                                                   const double* __restrict__ trig64, NaThr th,
+                                                   uint8_t* __restrict__ pass, NaHead* h) {
+    constexpr int D = NB == 1 ? 8 : NB == 2 ? 4 : 2;  // tiles in flight per wave
+    constexpr int kWaveRows = 12;  // band rows of a tile pair from which lanes settle them in parallel
+    __shared__ double tw[2 * kMaxN];
+    const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+    const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t q0 = wave * tpw, q1 = min(q0 + tpw, (count + 31) / 32);
+    const int64_t last = min(q1 * 32, count) - 1;
+    const int8_t* __restrict__ base = words + 8 * half;
+    // lanes read bytes 16 bl + 8 half .. + 7 of their row; past the end, the wave's last row
+    auto load = [&](int64_t q, uint2 (&raw)[NB]) {
+        const int8_t* w = base + min(q * 32 + col, last) * stride;
+#pragma unroll
+        for (int bl = 0; bl < NB; ++bl) raw[bl] = *reinterpret_cast<const uint2*>(w + 16 * bl);
+    };
+    uint2 ring[D][NB];
+    uint4 a[MT][2 * NB];
+    if (q0 < q1) {
+#pragma unroll
+        for (int g = 0; g < D; ++g) load(q0 + g, ring[g]);
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int s2 = 0; s2 < 2 * NB; ++s2) a[t][s2] = frags[((t * 2 * NB) + s2) * 64 + lane];
+    }
+    for (int i = threadIdx.x; i < 2 * n; i += blockDim.x) tw[i] = trig64[i];
+    __syncthreads();
+    // the last block's letters past n do not count
+    const int left = n - 16 * (NB - 1) - 8 * half;  // letters of this lane's 8 bytes there
+    const uint32_t k0 = left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+    const uint32_t k1 = left >= 8 ? ~0u : left <= 4 ? 0u : (1u << (8 * (left - 4))) - 1u;
+    auto row_sum = [&](const uint2 (&raw)[NB]) {
+        constexpr uint32_t z = 0x80808080u;  // |x| = |(x + 128) - 128| on unsigned bytes
+        uint32_t s = 0;
+#pragma unroll
+        for (int bl = 0; bl < NB; ++bl) {
+            const uint32_t x = bl + 1 < NB ? raw[bl].x : raw[bl].x & k0, y = bl + 1 < NB ? raw[bl].y : raw[bl].y & k1;
+            s = __builtin_amdgcn_sad_u8(x ^ z, z, s);
+            s = __builtin_amdgcn_sad_u8(y ^ z, z, s);
         }
-        npass += acc;
+        return s;
+    };
+    unsigned long long nband = 0, nties = 0, npass = 0;
+    for (int64_t qq = q0; qq < q1; qq += D) {
+#pragma unroll
+        for (int g = 0; g < D; g += 2) {
+            const int64_t q = qq + g;
+            if (q >= q1) break;
+            uint4 b0[NB], b1[NB];
+#pragma unroll
+            for (int bl = 0; bl < NB; ++bl) {
+                b0[bl] = pack8_bf16(ring[g][bl].x, ring[g][bl].y);
+                b1[bl] = pack8_bf16(ring[g + 1][bl].x, ring[g + 1][bl].y);
+            }
+            // lanes 0..31 get the sums of tile q's rows, lanes 32..63 those of tile q + 1
+            const auto sw = __builtin_amdgcn_permlane32_swap(row_sum(ring[g]), row_sum(ring[g + 1]), false, false);
+            const float s1 = (float)((uint32_t)sw[0] + (uint32_t)sw[1]);
+            load(q + D, ring[g]);
+            load(q + 1 + D, ring[g + 1]);
+            f32x16 acc0[MT], acc1[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc0[t] = acc1[t] = f32x16{};
+            mfma_tile_reg<NB, MT>(a, b0, acc0);
+            mfma_tile_reg<NB, MT>(a, b1, acc1);
+            float m = tile_pair_max_psd1(acc0[0], acc1[0]);
+#pragma unroll
+            for (int t = 1; t < MT; ++t) m = fmaxf(m, tile_pair_max_psd1(acc0[t], acc1[t]));
+            const int64_t r = q * 32 + lane;
+            const bool mine = r <= last;
+            const float e = __builtin_fmaf(s1, th.b, th.a) * s1;
+            const bool reject = m > th.hi0 + e;
+            bool accept = m < th.lo0 - e;
+            unsigned long long bb = __ballot(mine && !reject && !accept);
+            if (bb) {
+                const unsigned long long all = bb;
+                if (__popcll(bb) > kWaveRows) {
+                    if (bb >> lane & 1) {
+                        const double v = fp64_max_psd(words + r * stride, n, tw, tw + n);
+                        accept = !(v > th.thr);
+                        nties += fabs(v - th.thr) < 1e-9;
+                    }
+                } else {
+                    while (bb) {
+                        const int l = __ffsll((long long)bb) - 1;
+                        bb &= bb - 1;
+                        const double v = na_wave_max_psd(words + (q * 32 + l) * stride, n, tw, lane);
+                        if (lane == l) {
+                            accept = !(v > th.thr);
+                            nties += fabs(v - th.thr) < 1e-9;
+                        }
+                    }
+                }
+                nband += all >> lane & 1;
+            }
+            if (mine) pass[r] = accept ? kAccept : kReject;
+            npass += mine && accept;
+        }
     }
-    block_atomic_add(&h->passed, npass, &h->ctl.count, nb, &h->ctl.ties, nt);
+    if (h) block_atomic_add(&h->passed, npass, &h->ctl.count, nband, &h->ctl.ties, nties);
 }
 
 }  // namespace gp
@@ -692,57 +794,53 @@ extern "C" int gp_psd_filter_batch_static(gp_ctx* ctx, const int8_t* d_words, in
             std::lock_guard<std::mutex> lk(g_na_mu);
             if (g_na_n[ctx->device] != n) {
                 const int id = ctx->tables.get(n);
-                PsdTableDesc d = ctx->tables.desc[id];
+                const PsdTableDesc& d = ctx->tables.desc[id];
                 const size_t nfrag = (size_t)d.mt * 2 * d.nb * 64;
                 if (nfrag > kNaFragCount) throw ArgError("gp_psd_filter_batch_static: table beyond the scratch");
                 GP_HIP(hipMemcpyAsync(base + kNaFragOff, ctx->tables.frags.data() + d.frag_off, nfrag * sizeof(uint4),
                                       hipMemcpyHostToDevice, st));
                 GP_HIP(hipMemcpyAsync(base + kNaTrigOff, ctx->tables.trig64.data() + d.trig_off,
                                       2 * (size_t)n * sizeof(double), hipMemcpyHostToDevice, st));
-                d.frag_off = 0;
-                d.trig_off = 0;
-                GP_HIP(hipMemcpyAsync(&h->desc, &d, sizeof d, hipMemcpyHostToDevice, st));
                 GP_HIP(hipStreamSynchronize(st));
                 g_na_n[ctx->device] = n;
             }
         }
-        const int blocks = (int)std::min<int64_t>((count + 255) / 256, (int64_t)ctx->num_cus * 8);
-        hipLaunchKernelGGL(k_na_reset, dim3(1), dim3(64), 0, st, h);
-        hipLaunchKernelGGL(k_na_s1, dim3(blocks), dim3(256), 0, st, d_words, stride, n, count, h);
-        hipLaunchKernelGGL(k_na_thr, dim3(1), dim3(64), 0, st, h, 2.0 * order - paf + 0.001);
-        GP_HIP(hipGetLastError());
-        SegTiles T{};
-        T.nseg = 1;
-        T.table[0] = 0;
-        T.stride[0] = stride;
-        T.first_row[0] = 0;
-        T.rows[0] = count;
-        T.byte0[0] = 0;
-        GP_HIP(hipEventRecord(ctx->ev0, st));
-        {
-            // the one table in the scratch, at index 0 of its descriptor array
-            std::vector<PsdTableDesc> dd(1, ctx->tables.desc[ctx->tables.get(n)]);
-            launch_psd_mfma(T, dd, ctx->num_cus, st, d_words, &h->desc, frags, &h->thr, d_pass, nullptr);
+        const PsdTableDesc& d = ctx->tables.desc[ctx->tables.get(n)];
+        const NaThr th = na_thr(d, 2.0 * order - paf + 0.001);
+        // whole tile pairs per wave, at most the resident waves of the class
+        const int64_t pairs = (count + 63) / 64;
+        const int64_t tpw = 2 * ((pairs + na_waves(d, ctx->num_cus) - 1) / na_waves(d, ctx->num_cus));
+        const dim3 grid((unsigned)((2 * pairs + 4 * tpw - 1) / (4 * tpw)));
+        if (stats) {
+            hipLaunchKernelGGL(k_na_reset, dim3(1), dim3(64), 0, st, h);
+            GP_HIP(hipEventRecord(ctx->ev0, st));
         }
-        GP_HIP(hipEventRecord(ctx->ev1, st));
-        hipLaunchKernelGGL(k_na_band, dim3(blocks), dim3(256), 0, st, d_words, stride, count, trig64, h, d_pass);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, d_words, (int64_t)stride, n, count, tpw, frags, trig64,
+                               th, d_pass, stats ? h : nullptr);
+        };
+        if (d.nb == 1) launch(k_na_filter<1, 1>);
+        else if (d.nb == 2) launch(k_na_filter<2, 1>);
+        else if (d.nb == 3 && d.mt == 1) launch(k_na_filter<3, 1>);
+        else if (d.nb == 3) launch(k_na_filter<3, 2>);
+        else launch(k_na_filter<4, 2>);
         GP_HIP(hipGetLastError());
-        GP_HIP(hipEventRecord(ctx->ev2, st));
-        NaHead hh;
-        GP_HIP(hipMemcpyAsync(&hh, h, sizeof hh, hipMemcpyDeviceToHost, st));
+        NaHead hh{};
+        if (stats) {
+            GP_HIP(hipEventRecord(ctx->ev1, st));
+            GP_HIP(hipMemcpyAsync(&hh, h, sizeof hh, hipMemcpyDeviceToHost, st));
+        }
         GP_HIP(hipStreamSynchronize(st));
         if (stats) {
-            float ms_main = 0, ms_band = 0;
-            GP_HIP(hipEventElapsedTime(&ms_main, ctx->ev0, ctx->ev1));
-            GP_HIP(hipEventElapsedTime(&ms_band, ctx->ev1, ctx->ev2));
+            float ms = 0;
+            GP_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
             stats->psd_decisions += (uint64_t)count;
             stats->psd_pass += hh.passed;
             stats->band_rechecks += hh.ctl.count;
             stats->tie_band += hh.ctl.ties;
-            stats->psd_kernel_ms += ms_main;
-            stats->band_kernel_ms += ms_band;
+            stats->psd_kernel_ms += ms;
             stats->psd_launches += 1;
-            stats->kernel_ms += ms_main + ms_band;
+            stats->kernel_ms += ms;
         }
         return GP_OK;
     } catch (const ArgError& e) {

@@ -75,6 +75,27 @@ def test_static_entry_matches_batch_entry(gpu_ctx, calls):
         assert st.tie_band == 0
 
 
+@pytest.mark.parametrize("n,order,paf,count,extra", [
+    (2, 2, 0, 1, 0), (10, 50, 0, 31, 0), (10, 50, 0, 33, 8), (16, 128, 0, 64, 0), (25, 50, 0, 65, 0),
+    (25, 50, 0, 70001, 8), (34, 578, 0, 1000, 0), (36, 18, -1260, 4097, 0), (48, 1152, 0, 129, 24), (64, 2048, 0, 4097, 0),
+])
+def test_static_entry_tiles_bands_and_padding(gpu_ctx, n, order, paf, count, extra):
+    """Row counts around the tiles, each operand class, letters past n that are not
+    zero, strides that only keep 8-byte alignment, and rows at the threshold (an
+    alternating word has PSD n^2 at n / 2), few and many within a pair of tiles."""
+    rng = np.random.default_rng(n + count)
+    w = _words(rng, count, n, 1, 16 * ((n + 15) // 16) + extra)
+    w[:, n:] = rng.integers(-128, 128, size=w[:, n:].shape)
+    hard = rng.random(count) < np.where(np.arange(count) // 64 % 2 == 0, 0.06, 0.6)
+    w[hard, :n] = 1 - 2 * (np.arange(n) % 2)
+    rc, got, st = _static(gpu_ctx, w, n, order, paf)
+    assert rc == g.GP_OK, gpu_ctx.lib.gp_last_error(gpu_ctx.h)
+    want, _, _ = gpu_ctx.psd_filter_batch(w, np.full(count, n, np.int32), np.full(count, order, np.int32),
+                                          np.full(count, paf, np.int32))
+    assert (got == want).all(), np.nonzero(got != want)[0][:10]
+    assert st.psd_pass == want.sum()
+
+
 def test_static_entry_rejects_sizes_beyond_its_scratch(gpu_ctx):
     w = np.zeros((4, 80), np.int8)
     rc, _, _ = _static(gpu_ctx, w, 65, 100, 0)             # longer than the one table it holds
