@@ -541,12 +541,11 @@ __global__ void __launch_bounds__(256) k_gen_emit(const int8_t* __restrict__ wor
 // side << 63 | the letter indices (v - a0) / 2, 4 bits each, first letter
 // most significant (n <= 15).
 __global__ void k_gen_sortkey(const int8_t* __restrict__ ow, const uint8_t* __restrict__ oside, int64_t m, int n,
-                              int a0, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                              int a0, uint64_t* __restrict__ keys) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
         uint64_t k = 0;
         for (int j = 0; j < n; ++j) k = (k << 4) | (uint64_t)((ow[i * n + j] - a0) >> 1);
         keys[i] = ((uint64_t)(oside[i] != 0) << 63) | k;
-        vals[i] = (uint32_t)i;
     }
 }
 
@@ -816,19 +815,15 @@ int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, i
         const int8_t* src_w = d_ow;
         const uint8_t* src_k = d_ok;
         if (acc_n > 1 && n <= 15) {
-            // file order on the device: radix sort of (side, word) keys, rows gathered
+            // file order on the device: sort by (side, word) keys, rows gathered
             uint64_t* d_sk = ctx->dev<uint64_t>("g_sk", (size_t)acc_n);
-            uint32_t* d_sv = ctx->dev<uint32_t>("g_sv", (size_t)acc_n);
-            uint64_t* d_tk = ctx->dev<uint64_t>("g_tk", (size_t)acc_n);
-            uint32_t* d_tv = ctx->dev<uint32_t>("g_tv", (size_t)acc_n);
-            uint32_t* d_hist = static_cast<uint32_t*>(ctx->buf("g_hist").ensure(radix_hist_bytes(acc_n)));
             const unsigned g = (unsigned)std::min<int64_t>((acc_n + 255) / 256, (int64_t)ctx->num_cus * 8);
-            hipLaunchKernelGGL(k_gen_sortkey, dim3(g), dim3(256), 0, st, d_ow, d_os, acc_n, n, a0, d_sk, d_sv);
+            hipLaunchKernelGGL(k_gen_sortkey, dim3(g), dim3(256), 0, st, d_ow, d_os, acc_n, n, a0, d_sk);
             GP_HIP(hipGetLastError());
-            radix_sort_pairs(st, d_sk, d_sv, d_tk, d_tv, d_hist, acc_n, 0, 64);
+            const MergeSorted order = merge_sort(ctx, "g_sort", d_sk, acc_n);
             int8_t* d_w2 = ctx->dev<int8_t>("g_ow2", (size_t)acc_n * n);
             uint8_t* d_k2 = ctx->dev<uint8_t>("g_ok2", (size_t)acc_n * std::max(K, 1));
-            hipLaunchKernelGGL(k_gen_gather, dim3(g), dim3(256), 0, st, d_ow, d_ok, d_sv, acc_n, n, K, d_w2, d_k2);
+            hipLaunchKernelGGL(k_gen_gather, dim3(g), dim3(256), 0, st, d_ow, d_ok, order.idx, acc_n, n, K, d_w2, d_k2);
             GP_HIP(hipGetLastError());
             src_w = d_w2;
             src_k = d_k2;

@@ -1,15 +1,27 @@
-// Device radix sort and the candidate join shared by match and uncompress.
+// Device sort of records by long keys, and the candidate join of match.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <string>
 #include <vector>
 
 struct gp_ctx;
 struct gp_stats;
 
 namespace gp {
+
+// Records in sorted order: first key words and record numbers, in buffers of the
+// context that the next sort of the same name uses again.
+struct MergeSorted {
+    const uint64_t* key;
+    const uint32_t* idx;
+};
+// Sorts n records on the context's stream by keys[i], then by the nrest words at
+// rest + i * nrest, then by i.
+MergeSorted merge_sort(gp_ctx* ctx, const std::string& name, const uint64_t* keys, int64_t n,
+                       const uint64_t* rest = nullptr, int nrest = 0);
 
 // Stable LSD radix sort of (key, value) pairs on bits [begin_bit, end_bit).
 void radix_sort_pairs(hipStream_t st, uint64_t* keys, uint32_t* vals, uint64_t* tmp_keys, uint32_t* tmp_vals,

@@ -74,3 +74,13 @@ def test_sort_gen_files_equal_coreutils(gpu_ctx, order, compress, paf):
             mixed = g.Cands(cands.words[perm], cands.keys[perm])
             got = gpu_ctx.sort_candidates(mixed)
             assert "".join(l + "\n" for l in got.lines()) == ref, side
+
+
+@pytest.mark.parametrize("m", [2047, 2048, 2049, 4097, 10241])
+@pytest.mark.parametrize("key_values", [[7], [7, 70, 77]])
+def test_sort_runs_and_ties(gpu_ctx, m, key_values):
+    """Record counts around the runs of 2048 and their merges, with keys whose first
+    words are mostly equal, so that the other words decide."""
+    rng = np.random.default_rng(m)
+    c = _random_records(rng, m, 15, [-3, -1, 1, 3], key_values)
+    assert gpu_ctx.sort_candidates(c).lines() == sorted(set(c.lines()))
