@@ -8,9 +8,14 @@
 // inverted B key is the A key shifted by the constant BOUND - Q, and two
 // digit strings of tuples that differ by a nonzero constant shift cannot be
 // equal (the first component keeps or changes its decimal length, and either
-// way the strings differ).  The join therefore hashes the key tuples, sorts B
-// by hash (LSD radix sort), and for every A scans the equal-hash range of B,
-// verifying tuple equality and then the integer PAF condition.
+// way the strings differ).  The join therefore hashes the key tuples:
+//   k_join_insert  B records into chains of a hash table
+//   k_join_probe   for every A its slot's chain: equal hash, then equal tuple
+//   k_join_check   the integer PAF condition of the candidate pairs
+// and the accepted pairs are sorted into the reference's emission order.
+// Bound by launches and the copies of the four input buffers.  The files of order
+// 45, 3 -> 1 (at most 53000 records each) take 237 us, against 767 us with B radix
+// sorted by hash (40 launches) and the pairs sorted on the host.
 #include <algorithm>
 
 #include "gp_internal.hpp"
@@ -29,60 +34,97 @@ __device__ __forceinline__ uint64_t key_hash(const uint8_t* __restrict__ k, int 
     return h;
 }
 
-__global__ void k_hash_keys(const uint8_t* __restrict__ keys, int64_t m, int nkey, int kstride,
-                            uint64_t* __restrict__ h, uint32_t* __restrict__ idx) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        h[i] = key_hash(keys + i * kstride, nkey);
-        if (idx) idx[i] = (uint32_t)i;
-    }
-}
+constexpr uint32_t kJoinEnd = 0xFFFFFFFFu;
 
-__device__ bool paf_ok(const int8_t* __restrict__ a, const int8_t* __restrict__ b, int n, int target) {
-    for (int s = 1; s <= n / 2; ++s) {
-        int acc = 0;
-        int j = s;
-        for (int p = 0; p < n; ++p) {
-            acc += (int)a[p] * (int)a[j] + (int)b[p] * (int)b[j];
-            if (++j == n) j = 0;
-        }
-        if (acc != target) return false;
+// B record i in front of the chain of its slot (head: kJoinEnd where empty).
+__global__ void k_join_insert(const uint8_t* __restrict__ keys, int64_t m, int nkey, int kstride,
+                              uint64_t* __restrict__ hash, uint32_t* __restrict__ next, uint32_t* head,
+                              uint32_t mask) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint64_t h = key_hash(keys + i * kstride, nkey);
+        hash[i] = h;
+        next[i] = atomicExch(&head[(uint32_t)h & mask], (uint32_t)i);
     }
-    return true;
 }
 
 struct JoinCtl {
     unsigned long long out;
-    unsigned long long checks;
+    unsigned long long cand;
 };
 
-__global__ void k_join(const int8_t* __restrict__ wa, const uint8_t* __restrict__ ka, int64_t na,
-                       const int8_t* __restrict__ wb, const uint8_t* __restrict__ kb, int64_t nb,
-                       const uint64_t* __restrict__ sh, const uint32_t* __restrict__ sidx, int n, int nkey,
-                       int wstride, int kstride, int target, uint32_t* __restrict__ out_a,
-                       uint32_t* __restrict__ out_b, int64_t cap, JoinCtl* ctl) {
-    unsigned long long checks = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < na; i += (int64_t)gridDim.x * blockDim.x) {
+// Appends x of the lanes with `have` to list (at most cap entries kept) with one
+// atomic per wave; every lane of the wave must call it.
+__device__ __forceinline__ void wave_append(unsigned long long* count, bool have, uint64_t x, uint64_t* list,
+                                            int64_t cap) {
+    const unsigned long long b = __ballot(have);
+    if (!b) return;
+    const int lane = threadIdx.x & 63;
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(count, (unsigned long long)__popcll(b));
+    base = __shfl(base, 0) + __popcll(b & ((1ull << lane) - 1ull));
+    if (have && (int64_t)base < cap) list[base] = x;
+}
+
+// Candidate pairs A << 32 | B with equal key tuples, one A record per lane.
+__global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ ka, int64_t na,
+                                                    const uint8_t* __restrict__ kb, int nkey, int kstride,
+                                                    const uint64_t* __restrict__ hash,
+                                                    const uint32_t* __restrict__ next,
+                                                    const uint32_t* __restrict__ head, uint32_t mask,
+                                                    uint64_t* __restrict__ cand, int64_t cap, JoinCtl* ctl) {
+    for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < na; i0 += (int64_t)gridDim.x * 256) {
+        const int64_t i = i0 + threadIdx.x;
         const uint8_t* k = ka + i * kstride;
-        const uint64_t h = key_hash(k, nkey);
-        int64_t lo = 0, hi = nb;
-        while (lo < hi) {
-            int64_t mid = (lo + hi) >> 1;
-            if (sh[mid] < h) lo = mid + 1; else hi = mid;
+        uint64_t h = 0;
+        uint32_t j = kJoinEnd;
+        if (i < na) {
+            h = key_hash(k, nkey);
+            j = head[(uint32_t)h & mask];
         }
-        for (int64_t j = lo; j < nb && sh[j] == h; ++j) {
-            const uint32_t ib = sidx[j];
-            const uint8_t* k2 = kb + (int64_t)ib * kstride;
-            bool eq = true;
-            for (int q = 0; q < nkey && eq; ++q) eq = k[q] == k2[q];
-            if (!eq) continue;
-            ++checks;
-            if (paf_ok(wa + i * wstride, wb + (int64_t)ib * wstride, n, target)) {
-                unsigned long long o = atomicAdd(&ctl->out, 1ull);
-                if ((int64_t)o < cap) { out_a[o] = (uint32_t)i; out_b[o] = ib; }
+        while (__any(j != kJoinEnd)) {
+            bool eq = false;
+            uint32_t at = j;
+            if (j != kJoinEnd) {
+                eq = hash[j] == h;
+                j = next[j];
             }
+            if (eq) {
+                const uint8_t* k2 = kb + (int64_t)at * kstride;
+                for (int q = 0; q < nkey && eq; ++q) eq = k[q] == k2[q];
+            }
+            wave_append(&ctl->cand, eq, (uint64_t)i << 32 | at, cand, cap);
         }
     }
-    block_atomic_add(&ctl->checks, checks);
+}
+
+// The PAF condition of each candidate by 8 lanes, which take the shifts in turn
+// (a lane that checked its candidate alone had a chain of n^2 / 2 dependent
+// adds, and each accepted pair its own atomic).
+__global__ void __launch_bounds__(256) k_join_check(const int8_t* __restrict__ wa, const int8_t* __restrict__ wb, int n,
+                                                    int wstride, int target, const uint64_t* __restrict__ cand,
+                                                    int64_t cap, uint64_t* __restrict__ out, JoinCtl* ctl) {
+    const int64_t m = min((int64_t)ctl->cand, cap);
+    const int lane = threadIdx.x & 63, sub = lane & 7;
+    for (int64_t c0 = (int64_t)blockIdx.x * 32; c0 < m; c0 += (int64_t)gridDim.x * 32) {
+        const int64_t c = c0 + (threadIdx.x >> 3);
+        const uint64_t x = c < m ? cand[c] : 0;
+        bool ok = c < m;
+        if (ok) {
+            const int8_t* a = wa + (int64_t)(x >> 32) * wstride;
+            const int8_t* b = wb + (int64_t)(uint32_t)x * wstride;
+            for (int s = 1 + sub; s <= n / 2; s += 8) {
+                int acc = 0, j = s;
+                for (int p = 0; p < n; ++p) {
+                    acc += (int)a[p] * (int)a[j] + (int)b[p] * (int)b[j];
+                    if (++j == n) j = 0;
+                }
+                ok = ok && acc == target;
+            }
+        }
+        const unsigned long long all = __ballot(ok);
+        const bool pass = (all >> (lane & 56) & 255ull) == 255ull;
+        wave_append(&ctl->out, pass && sub == 0, x, out, cap);
+    }
 }
 
 JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int64_t na, const int8_t* d_wb,
@@ -92,55 +134,57 @@ JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int6
     if (na <= 0 || nb <= 0) return res;
     if (na > 0xFFFFFFFFll || nb > 0xFFFFFFFFll) throw ArgError("join: more than 2^32 candidates");
     hipStream_t st = ctx->stream;
-    uint64_t* hb = ctx->dev<uint64_t>("j_hb", nb);
-    uint32_t* ib = ctx->dev<uint32_t>("j_ib", nb);
-    uint64_t* tk = ctx->dev<uint64_t>("j_tk", nb);
-    uint32_t* tv = ctx->dev<uint32_t>("j_tv", nb);
-    uint32_t* hist = static_cast<uint32_t*>(ctx->buf("j_hist").ensure(radix_hist_bytes(nb)));
+    uint32_t slots = 64;  // a slot per B record or more
+    while (slots < nb && slots < (1u << 31)) slots <<= 1;
+    uint64_t* hash = ctx->dev<uint64_t>("j_hash", nb);
+    uint32_t* next = ctx->dev<uint32_t>("j_next", nb);
+    uint32_t* head = ctx->dev<uint32_t>("j_head", slots);
     JoinCtl* ctl = ctx->dev<JoinCtl>("j_ctl", 1);
-    GP_HIP(hipEventRecord(ctx->ev2, st));
-    hipLaunchKernelGGL(k_hash_keys, dim3(ctx->num_cus * 4), dim3(256), 0, st, d_kb, nb, nkey, kstride, hb, ib);
+    if (stats) GP_HIP(hipEventRecord(ctx->ev2, st));
+    GP_HIP(hipMemsetAsync(head, 0xFF, (size_t)slots * 4, st));
+    const auto blocks = [&](int64_t n_) { return dim3((unsigned)std::min<int64_t>((n_ + 255) / 256, ctx->num_cus * 8)); };
+    hipLaunchKernelGGL(k_join_insert, blocks(nb), dim3(256), 0, st, d_kb, nb, nkey, kstride, hash, next, head,
+                       slots - 1);
     GP_HIP(hipGetLastError());
-    radix_sort_pairs(st, hb, ib, tk, tv, hist, nb, 0, 64);
     int64_t cap = std::max<int64_t>(1024, 2 * std::max(na, nb));
     JoinCtl h{};
+    uint64_t* out = nullptr;
     for (int attempt = 0; attempt < 2; ++attempt) {
-        uint32_t* oa = ctx->dev<uint32_t>("j_oa", cap);
-        uint32_t* ob = ctx->dev<uint32_t>("j_ob", cap);
+        uint64_t* cand = ctx->dev<uint64_t>("j_cand", cap);
+        out = ctx->dev<uint64_t>("j_out", cap);
         GP_HIP(hipMemsetAsync(ctl, 0, sizeof(JoinCtl), st));
-        hipLaunchKernelGGL(k_join, dim3((unsigned)std::min<int64_t>((na + 255) / 256, ctx->num_cus * 8)), dim3(256), 0,
-                           st, d_wa, d_ka, na, d_wb, d_kb, nb, hb, ib, n, nkey, wstride, kstride, paf_target, oa, ob,
-                           cap, ctl);
+        hipLaunchKernelGGL(k_join_probe, blocks(na), dim3(256), 0, st, d_ka, na, d_kb, nkey, kstride, hash, next, head,
+                           slots - 1, cand, cap, ctl);
+        hipLaunchKernelGGL(k_join_check, blocks(8 * na), dim3(256), 0, st, d_wa, d_wb, n, wstride, paf_target, cand,
+                           cap, out, ctl);
         GP_HIP(hipGetLastError());
         GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
         GP_HIP(hipStreamSynchronize(st));
-        if ((int64_t)h.out <= cap) break;
-        cap = (int64_t)h.out;
+        if ((int64_t)h.cand <= cap) break;
+        cap = (int64_t)h.cand;
     }
-    GP_HIP(hipEventRecord(ctx->ev3, st));
+    // emission order of the reference: A position outer, B position inner
+    std::vector<uint64_t> pairs(h.out);
+    if (h.out) {
+        const MergeSorted s = merge_sort(ctx, "j_sort", out, (int64_t)h.out);
+        GP_HIP(hipMemcpyAsync(pairs.data(), s.key, h.out * 8, hipMemcpyDeviceToHost, st));
+    }
+    if (stats) GP_HIP(hipEventRecord(ctx->ev3, st));
+    GP_HIP(hipStreamSynchronize(st));
+    res.checks = h.cand;
+    if (stats) {
+        float ms = 0;
+        GP_HIP(hipEventElapsedTime(&ms, ctx->ev2, ctx->ev3));
+        stats->pair_checks += h.cand;
+        stats->kernel_ms += ms;
+    }
     res.ia.resize(h.out);
     res.ib.resize(h.out);
-    if (h.out) {
-        GP_HIP(hipMemcpyAsync(res.ia.data(), ctx->buf("j_oa").p, h.out * 4, hipMemcpyDeviceToHost, st));
-        GP_HIP(hipMemcpyAsync(res.ib.data(), ctx->buf("j_ob").p, h.out * 4, hipMemcpyDeviceToHost, st));
+    for (size_t i = 0; i < pairs.size(); ++i) {
+        res.ia[i] = (uint32_t)(pairs[i] >> 32);
+        res.ib[i] = (uint32_t)pairs[i];
     }
-    GP_HIP(hipStreamSynchronize(st));
-    float ms = 0;
-    GP_HIP(hipEventElapsedTime(&ms, ctx->ev2, ctx->ev3));
-    res.checks = h.checks;
-    if (stats) { stats->pair_checks += h.checks; stats->kernel_ms += ms; }
-    // emission order of the reference: A position outer, B position inner
-    std::vector<size_t> order(h.out);
-    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
-    std::sort(order.begin(), order.end(), [&](size_t x, size_t y) {
-        return res.ia[x] != res.ia[y] ? res.ia[x] < res.ia[y] : res.ib[x] < res.ib[y];
-    });
-    JoinResult sorted;
-    sorted.checks = res.checks;
-    sorted.ia.resize(order.size());
-    sorted.ib.resize(order.size());
-    for (size_t i = 0; i < order.size(); ++i) { sorted.ia[i] = res.ia[order[i]]; sorted.ib[i] = res.ib[order[i]]; }
-    return sorted;
+    return res;
 }
 
 }  // namespace gp

@@ -118,3 +118,22 @@ def test_gen_large_matches_golden_digest(gpu_ctx, fixture):
         assert len(c) == fx[side]["lines"]
         assert hashlib.sha256(text.encode()).hexdigest() == fx[side]["sha256"]
     assert st.tie_band == 0
+
+
+@pytest.mark.parametrize("n,ma,mb,nkeys", [(6, 300, 300, 4), (8, 1, 700, 1), (18, 257, 64, 3), (21, 90, 1000, 2)])
+def test_match_many_equal_keys(gpu_ctx, n, ma, mb, nkeys):
+    """Long chains of B records with equal keys (more candidate pairs than the first
+    list holds), shifts beyond one per lane, few records on either side."""
+    rng = np.random.default_rng(n)
+    wa = rng.choice([-1, 1], size=(ma, n)).astype(np.int8)
+    wb = rng.choice([-1, 1], size=(mb, n)).astype(np.int8)
+    wb[: min(ma, mb) // 2] = wa[: min(ma, mb) // 2]
+    kinds = rng.integers(0, 256, size=(nkeys, n // 2)).astype(np.uint8)
+    xa, xb = rng.integers(0, nkeys, ma), rng.integers(0, nkeys, mb)
+    target = 2 * int(wa[0].astype(int) @ np.roll(wa[0], 1)) if n == 6 else 4
+    paf = lambda w: np.stack([(w.astype(int) * np.roll(w, -s, axis=1)).sum(1) for s in range(1, n // 2 + 1)], 1)
+    fa, fb = paf(wa), paf(wb)
+    want = [(i, j) for i in range(ma) for j in range(mb) if xa[i] == xb[j] and (fa[i] + fb[j] == target).all()]
+    rc, pa, pb, st = gpu_ctx.match(n, 1, target, g.Cands(wa, kinds[xa]), g.Cands(wb, kinds[xb]))
+    assert st.pair_checks == int((xa[:, None] == xb[None, :]).sum())
+    assert [(x.tolist(), y.tolist()) for x, y in zip(pa, pb)] == [(wa[i].tolist(), wb[j].tolist()) for i, j in want]
