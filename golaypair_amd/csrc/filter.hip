@@ -14,17 +14,22 @@
 // its swapped-template branch) is this whole group, so its classes are orbits.
 // Walking the pairs in (a, b) order and erasing each survivor's class
 // (filter.cpp:117-144) therefore keeps the lexicographically smallest input
-// member of every orbit.  Here every pair's orbit minimum is computed on the GPU
-// (one pair per wave, as an order-preserving packed key); pairs are then grouped
-// by orbit minimum on the host.
+// member of every orbit.  Here, on the GPU,
+//   k_value_range   the range of the values, which gives the bits per value
+//   k_orbit_bits    every pair's orbit minimum, one pair per wave, with whole
+//   k_orbit_min     words as integers where they fit in 128 bits, else by letters
+//   k_class_insert  a hash table of the minima, each slot with its least pair
+//   k_class_keep    the pairs in the table
+// and the kept pairs are sorted by (a, b) and gathered.
 #include <algorithm>
 #include <cstring>
 #include <functional>
 #include <numeric>
+#include <vector>
 
 #include "gp_host.hpp"
 #include "gp_internal.hpp"
-#include "linesort.hpp"
+#include "gp_sort.hpp"
 
 namespace gp {
 
@@ -35,30 +40,6 @@ struct FilterParams {
     int32_t units[64];
     int32_t mx, sh, B, E;  // value v packs as (v + mx) >> sh in B bits, E = 64 / B values per word
 };
-
-// Packed key of the image s * (-1)^(kappa i) * X[(u i + t) mod n], i = 0..n-1:
-// B bits per value, first value in the most significant bits of word 0, so
-// that unsigned word-by-word order is the signed lexicographic order of images.
-template <int W>
-__device__ __forceinline__ void img_key(const int8_t* X, const FilterParams& P, int u, int t, int kappa, int sg,
-                                        uint64_t (&k)[W]) {
-    const int n = P.n;
-    int idx = t, i = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        uint64_t acc = 0;
-        const int iend = min(n, (w + 1) * P.E);
-        const int cnt = max(0, iend - i);
-        for (; i < iend; ++i) {
-            int v = X[idx] * sg;
-            if (kappa & i & 1) v = -v;
-            acc = (acc << P.B) | (uint64_t)((v + P.mx) >> P.sh);
-            idx += u;
-            if (idx >= n) idx -= n;
-        }
-        k[w] = cnt ? acc << (P.B * (P.E - cnt)) : 0ull;
-    }
-}
 
 template <int W>
 __device__ __forceinline__ bool key_less(const uint64_t (&x)[W], const uint64_t (&y)[W]) {
@@ -231,155 +212,357 @@ __global__ void __launch_bounds__(256) k_orbit_min(FilterParams P, const int8_t*
     }
 }
 
-int filter_pairs(gp_ctx* ctx, int order, int compress, const PairSet& in, PairSet& out, gp_stats* stats) {
+typedef unsigned __int128 u128;
+
+template <class T>
+__device__ __forceinline__ T wave_min_bits(T v) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        T o;
+        if constexpr (sizeof(T) == 16)
+            o = (T)__shfl_xor((unsigned long long)(v >> 64), off) << 64 | __shfl_xor((unsigned long long)v, off);
+        else if constexpr (sizeof(T) == 8)
+            o = __shfl_xor((unsigned long long)v, off);
+        else
+            o = (T)__shfl_xor((int)v, off);
+        v = o < v ? o : v;
+    }
+    return v;
+}
+
+// k_orbit_min for words of n * B bits that fit in T (first letter in the highest
+// field): a rotation is two shifts, a negated word a subtraction from the word of
+// largest fields, and the least rotation the minimum of all n.
+//   The words decimated by every unit, of a and of b, one per lane, go to LDS.
+//   Phase 1: variants (swap, unit, kappa, sign) over the lanes; the wave's least
+//   rotation is the a key.  Phase 2, for each variant that reaches it: the lanes
+//   share the rotations of its b-part words, which are in LDS already.
+// Bound by VALU: about 150 rotation steps of 9 operations per pair at n = 50.
+// 120011 pairs of n = 50 with altnegative take 0.39 ms against 4.95 ms by letters (a
+// least rotation by comparing letters in LDS, one after the other), 18645 pairs of
+// n = 45 0.04 ms against 0.31 ms.
+template <class T>
+__global__ void __launch_bounds__(256) k_orbit_bits(FilterParams P, const int8_t* __restrict__ pa,
+                                                    const int8_t* __restrict__ pb, int64_t m,
+                                                    uint64_t* __restrict__ canon) {
+    constexpr int W = sizeof(T) == 16 ? 2 : 1;
+    __shared__ uint8_t fld[4][2][kMaxN];
+    __shared__ T zl[4][2 * kMaxN];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int n = P.n, B = P.B, nb = n * B, nu = P.nunits;
+    const int nk = P.alt ? 2 : 1, ns = nk, per = nk * ns;
+    T mask = 0, all = 0, odd = 0;  // all bits; the largest value in every field; the fields of odd letters
+    for (int j = 0; j < n; ++j) {
+        const T f = (T)((1u << B) - 1u);
+        mask = mask << B | f;
+        all = all << B | (T)((2 * P.mx) >> P.sh);
+        odd = odd << B | (j & 1 ? f : (T)0);
+    }
+    auto variant = [&](T y, int kappa, int sg) {
+        if (kappa) y = (y & ~odd) | ((all & odd) - (y & odd));
+        return sg ? all - y : y;
+    };
+    for (int64_t q = (int64_t)blockIdx.x * 4 + wv; q < m; q += (int64_t)gridDim.x * 4) {
+        if (lane < n) {
+            fld[wv][0][lane] = (uint8_t)((pa[q * n + lane] + P.mx) >> P.sh);
+            fld[wv][1][lane] = (uint8_t)((pb[q * n + lane] + P.mx) >> P.sh);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int c = lane; c < 2 * nu; c += 64) {
+            const uint8_t* x = fld[wv][c >= nu];
+            const int u = P.units[c >= nu ? c - nu : c];
+            T z = 0;
+            int idx = 0;
+            for (int j = 0; j < n; ++j) {
+                z = z << B | x[idx];
+                idx += u;
+                if (idx >= n) idx -= n;
+            }
+            zl[wv][c] = z;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        T best = ~(T)0;
+        uint32_t bits = 0;  // the lane's variants (c = lane + 64 bit) that reach `best`
+        int round = 0;
+        for (int c = lane; c < 2 * nu * per; c += 64, ++round) {
+            T y = variant(zl[wv][c / per], c % per / ns, c % ns), mn = y;
+            for (int r = 1; r < n; ++r) {
+                y = (y << B | y >> (nb - B)) & mask;
+                mn = y < mn ? y : mn;
+            }
+            if (mn < best) {
+                best = mn;
+                bits = 0;
+            }
+            if (mn == best) bits |= 1u << round;
+        }
+        const T ka = wave_min_bits(best);
+        if (best != ka) bits = 0;
+        T kb = ~(T)0;
+        for (unsigned long long reach; (reach = __ballot(bits != 0)) != 0;) {
+            const int l = __ffsll((long long)reach) - 1;
+            const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)bits, l);
+            const int c = l + 64 * (__ffs((int)lb) - 1);
+            if (lane == l) bits &= bits - 1;
+            const int v = c / per, kappa = c % per / ns, ui = v < nu ? v : v - nu;
+            // candidates (unit u or -u, sign): 64 / (2 ns) lanes each; -u has index nu - 1 - ui
+            const int share = 32 / ns, cand = lane / share;
+            const T y = variant(zl[wv][(v < nu ? nu : 0) + (cand & 1 ? nu - 1 - ui : ui)], kappa, cand >> 1);
+            for (int r = lane % share; r < n; r += share) {
+                const T x = r ? (y << (r * B) | y >> (nb - r * B)) & mask : y;
+                kb = x < kb ? x : kb;
+            }
+        }
+        kb = wave_min_bits(kb);
+        if (lane == 0) {
+            if constexpr (W == 2) {
+                canon[q * 4] = (uint64_t)(ka >> 64);
+                canon[q * 4 + 1] = (uint64_t)ka;
+                canon[q * 4 + 2] = (uint64_t)(kb >> 64);
+                canon[q * 4 + 3] = (uint64_t)kb;
+            } else {
+                canon[q * 2] = (uint64_t)ka;
+                canon[q * 2 + 1] = (uint64_t)kb;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// What the packing needs of the values of a call, and its count of kept pairs.
+struct FilterCtl {
+    uint32_t mx;      // max |v|
+    uint32_t parity;  // bit 0: some value is even, bit 1: some is odd
+    uint32_t kept;
+    uint32_t pad;
+};
+
+__global__ void __launch_bounds__(256) k_value_range(const int8_t* __restrict__ a, const int8_t* __restrict__ b,
+                                                     int64_t count, FilterCtl* ctl) {
+    uint32_t mx = 0, par = 0;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    auto take = [&](int v) {
+        mx = max(mx, (uint32_t)abs(v));
+        par |= v & 1 ? 2u : 1u;
+    };
+    for (int64_t i = t; i < count / 4; i += step) {  // (allocations are aligned)
+        const char4 x = reinterpret_cast<const char4*>(a)[i], y = reinterpret_cast<const char4*>(b)[i];
+        take(x.x); take(x.y); take(x.z); take(x.w);
+        take(y.x); take(y.y); take(y.z); take(y.w);
+    }
+    for (int64_t i = count / 4 * 4 + t; i < count; i += step) {
+        take(a[i]);
+        take(b[i]);
+    }
+    // one atomic of each kind per block (they are applied one at a time, 10 ns apart)
+    __shared__ uint32_t part[2][4];
+    for (int o = 32; o; o >>= 1) {
+        mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+        par |= (uint32_t)__shfl_xor((int)par, o);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        part[0][threadIdx.x >> 6] = mx;
+        part[1][threadIdx.x >> 6] = par;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicMax(&ctl->mx, max(max(part[0][0], part[0][1]), max(part[0][2], part[0][3])));
+        atomicOr(&ctl->parity, part[1][0] | part[1][1] | part[1][2] | part[1][3]);
+    }
+}
+
+constexpr uint32_t kNoPair = 0xFFFFFFFFu;
+
+// Pair i before pair j in (a, b) order (golay.h:25-31)?
+__device__ __forceinline__ bool pair_before(const int8_t* __restrict__ pa, const int8_t* __restrict__ pb, int n,
+                                            uint32_t i, uint32_t j) {
+    for (int p = 0; p < n; ++p) {
+        const int x = pa[(int64_t)i * n + p], y = pa[(int64_t)j * n + p];
+        if (x != y) return x < y;
+    }
+    for (int p = 0; p < n; ++p) {
+        const int x = pb[(int64_t)i * n + p], y = pb[(int64_t)j * n + p];
+        if (x != y) return x < y;
+    }
+    return false;
+}
+
+// Open addressing over the CW words of the orbit minimum (at most half full).  A
+// slot once taken stays with its class, and holds the class's least pair so far.
+__global__ void __launch_bounds__(256) k_class_insert(const uint64_t* __restrict__ canon, int CW,
+                                                      const int8_t* __restrict__ pa, const int8_t* __restrict__ pb,
+                                                      int n, int64_t m, uint32_t* slot, uint64_t mask) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint64_t* k = canon + i * CW;
+        uint64_t h = 0x9e3779b97f4a7c15ull;
+        for (int w = 0; w < CW; ++w) h = splitmix64(h ^ k[w]);
+        for (uint64_t s = h & mask;; s = (s + 1) & mask) {
+            uint32_t j = __hip_atomic_load(&slot[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (j == kNoPair) j = atomicCAS(&slot[s], kNoPair, (uint32_t)i);
+            if (j == kNoPair) break;
+            bool same = true;
+            for (int w = 0; w < CW && same; ++w) same = canon[(int64_t)j * CW + w] == k[w];
+            if (!same) continue;
+            while (pair_before(pa, pb, n, (uint32_t)i, j)) {
+                const uint32_t was = atomicCAS(&slot[s], j, (uint32_t)i);
+                if (was == j) break;
+                j = was;
+            }
+            break;
+        }
+    }
+}
+
+// One block per kKeepSlots slots, with one atomic.
+constexpr int kKeepSlots = 1024;
+__global__ void __launch_bounds__(256) k_class_keep(const uint32_t* __restrict__ slot, uint32_t* __restrict__ keep,
+                                                    FilterCtl* ctl) {
+    __shared__ uint32_t part[4], base;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint4 x = reinterpret_cast<const uint4*>(slot)[(int64_t)blockIdx.x * (kKeepSlots / 4) + t];
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+    uint32_t mine = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mine += v[j] != kNoPair;
+    uint32_t incl = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(incl, d);
+        if (lane >= d) incl += y;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    if (t == 0) base = atomicAdd(&ctl->kept, part[0] + part[1] + part[2] + part[3]);
+    __syncthreads();
+    uint32_t at = base + incl - mine;
+    for (int w = 0; w < wave; ++w) at += part[w];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (v[j] != kNoPair) keep[at++] = v[j];
+}
+
+// Key words of the kept pairs, a then b, as packed for the orbit minima (E values
+// a word, the first one highest): the first word of each pair in a column, the
+// other 2 wn - 1 together.
+__global__ void __launch_bounds__(256) k_keep_keys(FilterParams P, const int8_t* __restrict__ pa,
+                                                   const int8_t* __restrict__ pb, const uint32_t* __restrict__ keep,
+                                                   int64_t kept, int wn, uint64_t* __restrict__ first,
+                                                   uint64_t* __restrict__ rest) {
+    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < kept * 2 * wn;
+         x += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t i = x / (2 * wn);
+        const int w = (int)(x - i * 2 * wn), j0 = (w < wn ? w : w - wn) * P.E, j1 = min(j0 + P.E, P.n);
+        const int8_t* v = (w < wn ? pa : pb) + (int64_t)keep[i] * P.n;
+        uint64_t acc = 0;
+        for (int j = j0; j < j1; ++j) acc = acc << P.B | (uint64_t)((v[j] + P.mx) >> P.sh);
+        if (w == 0) first[i] = acc;
+        else rest[i * (2 * wn - 1) + w - 1] = acc;
+    }
+}
+
+__global__ void __launch_bounds__(256) k_keep_rows(const int8_t* __restrict__ pa, const int8_t* __restrict__ pb, int n,
+                                                   const uint32_t* __restrict__ keep,
+                                                   const uint32_t* __restrict__ order, int64_t kept,
+                                                   int8_t* __restrict__ oa, int8_t* __restrict__ ob) {
+    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < kept * n;
+         x += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t i = x / n, src = (int64_t)keep[order[i]] * n + (x - i * n);
+        oa[x] = pa[src];
+        ob[x] = pb[src];
+    }
+}
+
+int filter_pairs(gp_ctx* ctx, int order, int compress, const gp_pairs& in, PairSet& out, gp_stats* stats) {
     const int n = order / compress;
     out.n = n;
     out.a.clear();
     out.b.clear();
-    const int64_t m = in.size();
+    if (in.count < 0 || (in.count > 0 && (!in.a || !in.b))) throw ArgError("bad pair set");
+    const int64_t m = in.count;
     if (m == 0) return GP_OK;
     if (in.n != n) throw ArgError("filter: pair length != order/compress");
     if (n > kMaxN) throw ArgError("filter: length above 64");
-    Phase ph("filter: packing setup");
+    if (m > 0x7FFFFFFFll) throw ArgError("filter: more than 2^31 pairs");
     FilterParams P{};
     P.n = n;
     P.alt = !(compress > 1 || n % 2 == 1);  // filter.cpp:83-87
     for (int u = 1; u < n || (n == 1 && u == 1); ++u)
         if (std::gcd(u, n) == 1) P.units[P.nunits++] = u;
     if (n == 1) { P.nunits = 1; P.units[0] = 0; }
-    // key packing: the values and their negations lie in [-mx, mx]; halve when all have mx's parity
-    int mx = 0, odd_or = 0, odd_and = 1;  // max |v|; whether some / every value is odd
-    {
-        const int nc = 16;
-        std::vector<int> cmx(nc, 0), cor(nc, 0), cand(nc, 1);
-        const int64_t tot = m * n;
-        pool().parallel_for(nc, [&](size_t c) {
-            int lmx = 0, lor = 0, land = 1;
-            for (int64_t i = tot * (int64_t)c / nc; i < tot * (int64_t)(c + 1) / nc; ++i) {
-                const int a = in.a[i], b = in.b[i];
-                lmx = std::max(lmx, std::max(a < 0 ? -a : a, b < 0 ? -b : b));
-                lor |= (a | b) & 1;
-                land &= a & b & 1;
-            }
-            cmx[c] = lmx;
-            cor[c] = lor;
-            cand[c] = land;
-        });
-        for (int c = 0; c < nc; ++c) {
-            mx = std::max(mx, cmx[c]);
-            odd_or |= cor[c];
-            odd_and &= cand[c];
-        }
-    }
-    // every v + mx even: all values odd with mx odd, or all even with mx even
-    const bool same_parity = (mx & 1) ? odd_and == 1 : odd_or == 0;
+    hipStream_t st = ctx->stream;
+    Phase ph("filter: upload");
+    int8_t* da = ctx->dev<int8_t>("f_a", (size_t)m * n);
+    int8_t* db = ctx->dev<int8_t>("f_b", (size_t)m * n);
+    FilterCtl* ctl = ctx->dev<FilterCtl>("f_ctl", 1);
+    GP_HIP(hipMemsetAsync(ctl, 0, sizeof(FilterCtl), st));
+    GP_HIP(hipMemcpyAsync(da, in.a, (size_t)m * n, hipMemcpyHostToDevice, st));
+    GP_HIP(hipMemcpyAsync(db, in.b, (size_t)m * n, hipMemcpyHostToDevice, st));
+    const auto blocks = [&](int64_t threads, int per_cu) {
+        return dim3((unsigned)std::min<int64_t>((threads + 255) / 256, (int64_t)ctx->num_cus * per_cu));
+    };
+    hipLaunchKernelGGL(k_value_range, blocks((m * n + 15) / 16, 2), dim3(256), 0, st, da, db, m * n, ctl);
+    GP_HIP(hipGetLastError());
+    FilterCtl h{};
+    GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
+    GP_HIP(hipStreamSynchronize(st));
+    ph.next("filter: device");
+    // key packing: the values and their negations lie in [-mx, mx]; halve when all
+    // have mx's parity (every v + mx even)
+    const int mx = (int)h.mx;
     P.mx = mx;
-    P.sh = same_parity ? 1 : 0;
+    P.sh = h.parity == (mx & 1 ? 2u : 1u) ? 1 : 0;
     const int range = (2 * mx) >> P.sh;
     P.B = range <= 1 ? 1 : range <= 3 ? 2 : range <= 15 ? 4 : 8;
     P.E = 64 / P.B;
     const int wneed = (n + P.E - 1) / P.E;
-    const int W = wneed <= 1 ? 1 : wneed <= 2 ? 2 : wneed <= 4 ? 4 : 8;
-    hipStream_t st = ctx->stream;
-    ph.next("filter: device");
-    int8_t* da = ctx->dev<int8_t>("f_a", (size_t)m * n);
-    int8_t* db = ctx->dev<int8_t>("f_b", (size_t)m * n);
-    uint64_t* dc = ctx->dev<uint64_t>("f_c", (size_t)m * 2 * W);
-    GP_HIP(hipMemcpyAsync(da, in.a.data(), (size_t)m * n, hipMemcpyHostToDevice, st));
-    GP_HIP(hipMemcpyAsync(db, in.b.data(), (size_t)m * n, hipMemcpyHostToDevice, st));
-    GP_HIP(hipEventRecord(ctx->ev0, st));
+    // (the letter -128 has no negative in a byte: by letters)
+    const int W = mx > 127 || wneed > 2 ? (wneed <= 4 ? 4 : 8) : wneed <= 1 ? 1 : 2, CW = 2 * W;
+    uint64_t* dc = ctx->dev<uint64_t>("f_c", (size_t)m * CW);
+    uint64_t slots = kKeepSlots;
+    while (slots < 2 * (uint64_t)m) slots <<= 1;
+    uint32_t* slot = ctx->dev<uint32_t>("f_slot", slots);
+    uint32_t* keep = ctx->dev<uint32_t>("f_keep", (size_t)m);
+    if (stats) GP_HIP(hipEventRecord(ctx->ev0, st));
     const dim3 grid((unsigned)std::min<int64_t>((m + 3) / 4, (int64_t)ctx->num_cus * 16));
-    if (W == 1) hipLaunchKernelGGL(k_orbit_min<1>, grid, dim3(256), 0, st, P, da, db, m, dc);
-    else if (W == 2) hipLaunchKernelGGL(k_orbit_min<2>, grid, dim3(256), 0, st, P, da, db, m, dc);
-    else if (W == 4) hipLaunchKernelGGL(k_orbit_min<4>, grid, dim3(256), 0, st, P, da, db, m, dc);
-    else hipLaunchKernelGGL(k_orbit_min<8>, grid, dim3(256), 0, st, P, da, db, m, dc);
+    const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, P, da, db, m, dc); };
+    if (W == 1 && n * P.B <= 32) launch(k_orbit_bits<uint32_t>);
+    else if (W == 1) launch(k_orbit_bits<uint64_t>);
+    else if (W == 2) launch(k_orbit_bits<u128>);
+    else if (W == 4) launch(k_orbit_min<4>);
+    else launch(k_orbit_min<8>);
     GP_HIP(hipGetLastError());
-    GP_HIP(hipEventRecord(ctx->ev1, st));
-    std::vector<uint64_t> canon((size_t)m * 2 * W);
-    GP_HIP(hipMemcpyAsync(canon.data(), dc, canon.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+    if (stats) GP_HIP(hipEventRecord(ctx->ev1, st));
+    GP_HIP(hipMemsetAsync(slot, 0xFF, slots * 4, st));
+    hipLaunchKernelGGL(k_class_insert, blocks(m, 8), dim3(256), 0, st, dc, CW, da, db, n, m, slot, slots - 1);
+    hipLaunchKernelGGL(k_class_keep, dim3((unsigned)(slots / kKeepSlots)), dim3(256), 0, st, slot, keep, ctl);
+    GP_HIP(hipGetLastError());
+    GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
     GP_HIP(hipStreamSynchronize(st));
-    float ms = 0;
-    GP_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-    if (stats) stats->kernel_ms += ms;
-    ph.next("filter: group + order");
-    // Pairs with equal canonical keys form one class; its survivor is the pair
-    // that comes first in (a, b) lexicographic order (golay.h:25-31).  Both orders
-    // use packed big-endian keys (byte v + 128 per entry, a then b).
-    // one row per pair: the canonical key (2W words) then the pair key (PW
-    // words), so that (class, pair order) is one lexicographic word compare
-    const int PW = (2 * n + 7) / 8, CW = 2 * W, RW = CW + PW;
-    std::vector<uint64_t> rk((size_t)m * RW);
-    parallel_chunks(m, [&](int64_t i0, int64_t i1) {
-        for (int64_t i = i0; i < i1; ++i) {
-            uint64_t* r = &rk[i * RW];
-            for (int w = 0; w < CW; ++w) r[w] = canon[i * CW + w];
-            const int8_t* pa = &in.a[i * n];
-            const int8_t* pb = &in.b[i * n];
-            for (int w = 0; w < PW; ++w) {
-                uint64_t acc = 0;
-                for (int j = 8 * w; j < 8 * w + 8; ++j) {
-                    const int v = j < n ? pa[j] : j < 2 * n ? pb[j - n] : -128;  // -128 packs as 0
-                    acc = (acc << 8) | (uint64_t)(uint8_t)(v + 128);
-                }
-                r[CW + w] = acc;
-            }
-        }
-    }, 1024);
-    auto words_less = [&](int64_t x, int64_t y, int w0, int w1) {
-        for (int w = w0; w < w1; ++w)
-            if (rk[x * RW + w] != rk[y * RW + w]) return rk[x * RW + w] < rk[y * RW + w];
-        return false;
-    };
-    auto pair_less = [&](int64_t x, int64_t y) { return words_less(x, y, CW, RW); };
-    auto canon_eq = [&](int64_t x, int64_t y) {
-        for (int w = 0; w < CW; ++w)
-            if (rk[x * RW + w] != rk[y * RW + w]) return false;
-        return true;
-    };
-    // Classes by hashing the canonical key, each keeping its least pair: rows go
-    // to 16 partitions by hash (a counting pass), each partition has its own
-    // open-addressing table on a host thread; the kept pairs are then sorted.
-    constexpr int kParts = 16;
-    std::vector<uint64_t> hsh((size_t)m);
-    parallel_chunks(m, [&](int64_t i0, int64_t i1) {
-        for (int64_t i = i0; i < i1; ++i) {
-            uint64_t h = 0x9e3779b97f4a7c15ull;
-            for (int w = 0; w < CW; ++w) h = (h ^ rk[i * RW + w]) * 0xff51afd7ed558ccdull;
-            hsh[i] = h ^ (h >> 29);
-        }
-    }, 4096);
-    std::vector<int64_t> part_off(kParts + 1, 0), part_rows((size_t)m);
-    for (int64_t i = 0; i < m; ++i) ++part_off[(hsh[i] >> 60) + 1];
-    for (int q = 0; q < kParts; ++q) part_off[q + 1] += part_off[q];
-    {
-        std::vector<int64_t> fill(part_off.begin(), part_off.end() - 1);
-        for (int64_t i = 0; i < m; ++i) part_rows[fill[hsh[i] >> 60]++] = i;
+    if (stats) {
+        float ms = 0;
+        GP_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        stats->kernel_ms += ms;
     }
-    std::vector<std::vector<int64_t>> part_keep(kParts);
-    pool().parallel_for(kParts, [&](size_t q) {
-        const int64_t r0 = part_off[q], r1 = part_off[q + 1];
-        size_t T = 16;
-        while (T < 2 * (size_t)(r1 - r0)) T <<= 1;
-        std::vector<int64_t> slot(T, -1);
-        for (int64_t r = r0; r < r1; ++r) {
-            const int64_t i = part_rows[r];
-            size_t s = hsh[i] & (T - 1);
-            while (slot[s] >= 0 && !canon_eq(slot[s], i)) s = (s + 1) & (T - 1);
-            if (slot[s] < 0 || pair_less(i, slot[s])) slot[s] = i;
-        }
-        for (size_t s = 0; s < T; ++s)
-            if (slot[s] >= 0) part_keep[q].push_back(slot[s]);
-    });
-    std::vector<int64_t> keep;
-    for (const auto& k : part_keep) keep.insert(keep.end(), k.begin(), k.end());
-    parallel_sort(keep, pair_less);
-    out.a.resize(keep.size() * n);
-    out.b.resize(keep.size() * n);
-    for (size_t r = 0; r < keep.size(); ++r) {
-        std::memcpy(&out.a[r * n], &in.a[keep[r] * n], n);
-        std::memcpy(&out.b[r * n], &in.b[keep[r] * n], n);
-    }
-    if (stats) stats->pairs += keep.size();
+    ph.next("filter: order");
+    const int64_t kept = h.kept;
+    uint64_t* first = ctx->dev<uint64_t>("f_first", (size_t)kept);
+    uint64_t* rest = ctx->dev<uint64_t>("f_rest", (size_t)kept * (2 * wneed - 1));
+    hipLaunchKernelGGL(k_keep_keys, blocks(kept * 2 * wneed, 8), dim3(256), 0, st, P, da, db, keep, kept, wneed, first,
+                       rest);
+    GP_HIP(hipGetLastError());
+    const MergeSorted s = merge_sort(ctx, "f_sort", first, kept, rest, 2 * wneed - 1);
+    int8_t* oa = ctx->dev<int8_t>("f_oa", (size_t)kept * n);
+    int8_t* ob = ctx->dev<int8_t>("f_ob", (size_t)kept * n);
+    hipLaunchKernelGGL(k_keep_rows, blocks(kept * n, 8), dim3(256), 0, st, da, db, n, keep, s.idx, kept, oa, ob);
+    GP_HIP(hipGetLastError());
+    out.a.resize((size_t)kept * n);
+    out.b.resize((size_t)kept * n);
+    GP_HIP(hipMemcpyAsync(out.a.data(), oa, out.a.size(), hipMemcpyDeviceToHost, st));
+    GP_HIP(hipMemcpyAsync(out.b.data(), ob, out.b.size(), hipMemcpyDeviceToHost, st));
+    GP_HIP(hipStreamSynchronize(st));
+    if (stats) stats->pairs += (uint64_t)kept;
     return GP_OK;
 }
 
@@ -395,8 +578,8 @@ extern "C" int gp_filter(gp_ctx* ctx, int order, int compress, const gp_pairs* i
     return guarded_call(ctx, [&] {
         GP_HIP(hipSetDevice(ctx->device));
         if (!in || !out || order <= 0 || compress <= 0) throw ArgError("gp_filter: bad arguments");
-        PairSet p = import_pairs(in), o;
-        int rc = filter_pairs(ctx, order, compress, p, o, stats);
+        PairSet o;
+        int rc = filter_pairs(ctx, order, compress, *in, o, stats);
         if (rc != GP_OK) return rc;
         return export_pairs(o, out, false);
     });

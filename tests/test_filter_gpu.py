@@ -178,3 +178,35 @@ def test_filter_length50_altnegative_vs_brute_force(gpu_ctx):
     assert len(want) == len(bases)
     oa, ob = _gpu_filter(gpu_ctx, n, 1, a, b)
     assert [(tuple(int(v) for v in x), tuple(int(v) for v in y)) for x, y in zip(oa, ob)] == want
+
+
+@pytest.mark.parametrize("n,compress,letters", [
+    (1, 2, [-1, 1]), (2, 1, [-1, 1]), (32, 1, [-1, 1]), (33, 1, [-1, 1]), (64, 1, [-1, 1]),   # 1 bit per letter
+    (15, 3, [-3, -1, 1, 3]), (17, 3, [-2, 0, 2]), (32, 2, [-3, -1, 1, 3]),                    # 2 bits, one word
+    (33, 2, [-2, 0, 2]), (18, 5, [-5, -3, -1, 1, 3, 5]), (32, 4, list(range(-7, 8))),         # two words
+    (16, 1, list(range(-100, 101))), (33, 4, list(range(-7, 8))), (61, 2, list(range(-20, 21))),  # by letters
+    (12, 1, [-128, 3]),
+])
+def test_filter_packed_words_and_letters(gpu_ctx, n, compress, letters):
+    """Each width of the packed words and the path by letters: of the images of random
+    pairs under random transforms of the group, the least one of each pair is kept."""
+    rng = np.random.default_rng(n + len(letters))
+    alt = compress == 1 and n % 2 == 0 and min(letters) > -128
+    units = [u for u in range(1, n) if np.gcd(u, n) == 1] or [0]
+    seen, rows = set(), []
+    for _ in range(40):
+        x, y = rng.choice(letters, size=(2, n))
+        members = {(tuple(x), tuple(y))}
+        for _ in range(20):
+            u, e, k = rng.choice(units), rng.choice([1, -1]), (np.arange(n) % 2) * (rng.integers(0, 2) if alt else 0)
+            i, (ta, tb) = np.arange(n), rng.integers(0, n, 2)
+            a, b = (x, y) if rng.integers(0, 2) else (y, x)
+            sa, sb = rng.choice([1, -1], 2) if alt else (1, 1)
+            sgn = 1 - 2 * k
+            members.add((tuple(sa * sgn * a[(u * i + ta) % n]), tuple(sb * sgn * b[(e * u * i + tb) % n])))
+        if n > 8 or not rows:  # short words: random pairs may be images of each other
+            seen.add(min(members))
+            rows += sorted(members)
+    rows = [rows[q] for q in rng.permutation(len(rows))] + rows[:5]
+    oa, ob = _gpu_filter(gpu_ctx, n * compress, compress, np.array([r[0] for r in rows]), np.array([r[1] for r in rows]))
+    assert [(tuple(a), tuple(b)) for a, b in zip(oa.tolist(), ob.tolist())] == [tuple(map(tuple, s)) for s in sorted(seen)]
