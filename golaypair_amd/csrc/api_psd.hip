@@ -1,10 +1,8 @@
 // C ABI: context management and the batched PSD filter entry points.
 #include <algorithm>
 #include <cstring>
-#include <map>
 #include <numeric>
 #include <set>
-#include <tuple>
 
 #include "gp_internal.hpp"
 #include "psd_core.hpp"
@@ -187,84 +185,7 @@ int gp_psd_filter_batch(gp_ctx* ctx, const int8_t* words, int stride, const int3
         if (count < 0 || (count > 0 && (!words || !lens || !orders || !pafs || !pass)))
             throw ArgError("gp_psd_filter_batch: null buffer");
         if (count == 0) return GP_OK;
-        // Group rows by (n, order, paf): one segment per group, its rows at 16
-        // bytes per block of 16 letters (zero padded).
-        std::map<std::tuple<int, int, int>, std::vector<int64_t>> groups;
-        for (int64_t i = 0; i < count; ++i) {
-            if (lens[i] < 2 || lens[i] > kMaxN || lens[i] > stride) throw ArgError("word length out of range");
-            groups[{lens[i], orders[i], pafs[i]}].push_back(i);
-        }
-        int64_t bytes = 0;
-        for (auto& [key, rows] : groups) bytes += (int64_t)rows.size() * 16 * ((std::get<0>(key) + 15) / 16);
-        std::vector<int8_t> packed((size_t)bytes, 0);
-        std::vector<int64_t> row_of(count);
-        std::vector<BatchSeg> segs;
-        std::vector<FilterThr> thr(ctx->tables.desc.size() + groups.size());
-        int64_t r = 0, off = 0;
-        std::vector<FilterThr> seg_thr;
-        for (auto& [key, rows] : groups) {
-            auto [n, order, paf] = key;
-            const int table = ctx->tables.get(n);
-            BatchSeg sg{};
-            sg.first_row = r;
-            sg.rows = (int64_t)rows.size();
-            sg.stride = 16 * ctx->tables.desc[table].nb;
-            sg.byte0 = off;
-            double s1 = 0;
-            for (int64_t i : rows) {
-                double a = 0;
-                for (int p = 0; p < n; ++p) {
-                    int8_t v = words[i * stride + p];
-                    packed[off + p] = v;
-                    a += std::abs((int)v);
-                }
-                s1 = std::max(s1, a);
-                row_of[i] = r++;
-                off += sg.stride;
-            }
-            const PsdTableDesc& d = ctx->tables.desc[table];
-            const double th = 2.0 * order - paf + 0.001;
-            const double E = ctx->psd_mode == GP_PSD_SPLIT_BF16 ? split_bf16_E(d, s1) : fp32_E(n, s1);
-            // Each segment gets its own pseudo-table id so thresholds may differ
-            // between segments of one length.
-            seg_thr.push_back(make_thr(th, E));
-            sg.table = table;
-            segs.push_back(sg);
-        }
-        // Thresholds are indexed by table id; with several (order, paf) per n we
-        // run one batch per distinct threshold set.
-        std::vector<uint8_t> dec((size_t)count);
-        std::vector<float> mx(max_psd ? (size_t)count : 0);
-        int8_t* d_words = static_cast<int8_t*>(ctx->words.ensure((size_t)bytes));
-        uint8_t* d_dec = static_cast<uint8_t*>(ctx->decisions.ensure((size_t)count));
-        float* d_max = max_psd ? static_cast<float*>(ctx->aux4.ensure((size_t)count * sizeof(float))) : nullptr;
-        GP_HIP(hipMemcpyAsync(d_words, packed.data(), packed.size(), hipMemcpyHostToDevice, ctx->stream));
-        size_t si = 0;
-        while (si < segs.size()) {
-            // collect a run of segments with distinct tables
-            std::vector<BatchSeg> run;
-            std::vector<FilterThr> tt(ctx->tables.desc.size());
-            std::set<int> used;
-            size_t sj = si;
-            for (; sj < segs.size() && sj - si < 8 && !used.count(segs[sj].table); ++sj) {
-                used.insert(segs[sj].table);
-                run.push_back(segs[sj]);
-                tt[segs[sj].table] = seg_thr[sj];
-            }
-            run_psd_filter(ctx, d_words, 0, (int64_t)count, run, tt, d_dec, stats, d_max);
-            si = sj;
-        }
-        GP_HIP(hipMemcpyAsync(dec.data(), d_dec, (size_t)count, hipMemcpyDeviceToHost, ctx->stream));
-        if (max_psd)
-            GP_HIP(hipMemcpyAsync(mx.data(), d_max, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-        GP_HIP(hipStreamSynchronize(ctx->stream));
-        uint64_t npass = 0;
-        for (int64_t i = 0; i < count; ++i) {
-            pass[i] = dec[row_of[i]] == kAccept ? 1 : 0;
-            npass += pass[i];
-            if (max_psd) max_psd[i] = mx[row_of[i]];
-        }
-        if (stats) stats->psd_pass += npass;
+        filter_rows(ctx, words, stride, lens, orders, pafs, count, pass, max_psd, stats);
         return GP_OK;
     });
 }

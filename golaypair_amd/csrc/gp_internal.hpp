@@ -265,4 +265,9 @@ double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nr
                       const std::vector<BatchSeg>& segs, const std::vector<FilterThr>& thr_by_table,
                       uint8_t* d_decision, gp_stats* stats, float* d_maxpsd = nullptr);
 
+// gp_psd_filter_batch on checked, non-empty arguments (host buffers); throws on a
+// word length out of range before anything is written.
+void filter_rows(gp_ctx* ctx, const int8_t* words, int stride, const int32_t* lens, const int32_t* orders,
+                 const int32_t* pafs, int64_t count, uint8_t* pass, float* max_psd, gp_stats* stats);
+
 }  // namespace gp

@@ -127,6 +127,40 @@ __device__ inline double fp64_max_psd(const int8_t* __restrict__ w, int n, const
     return mx;
 }
 
+// fp64_max_psd of the row at w by the whole wave: lane q < n / 2 takes k = q + 1 in
+// the same summation order; c and s as there.  The result is in every lane.
+__device__ __forceinline__ double wave_max_psd(const int8_t* __restrict__ w, int n, const double* c, const double* s,
+                                               int lane) {
+    const int x = lane < n ? (int)w[lane] : 0;
+    const int k = lane < (n >> 1) ? lane + 1 : 0;  // (idle lanes: k = 0, their value is dropped)
+    double re = 0.0, im = 0.0;
+    int m = 0;
+    for (int p = 0; p < n; ++p) {
+        const double v = (double)__builtin_amdgcn_readlane(x, p);
+        re = __builtin_fma(v, c[m], re);
+        im = __builtin_fma(v, s[m], im);
+        m += k;
+        if (m >= n) m -= n;
+    }
+    double mx = k ? re * re + im * im : 0.0;
+    for (int o = 32; o; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+    return mx;
+}
+
+// sum |x_p| of the 8 letters in a uint2: |x| = |(x + 128) - 128| on unsigned bytes,
+// four at a time.
+__device__ __forceinline__ uint32_t abs_sum8(uint2 v, uint32_t s) {
+    constexpr uint32_t z = 0x80808080u;
+    return __builtin_amdgcn_sad_u8(v.y ^ z, z, __builtin_amdgcn_sad_u8(v.x ^ z, z, s));
+}
+
+// The letters before position `left` of the 8 in v, the others 0.
+__device__ __forceinline__ uint2 keep_letters(uint2 v, int left) {
+    if (left < 8) v.y &= left <= 4 ? 0u : (1u << (8 * (left - 4))) - 1u;
+    if (left < 4) v.x &= left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+    return v;
+}
+
 // Adds the sum of `v` over the lanes of the calling wave to *p with one
 // atomic (none when the sum is 0).  Every lane of the wave must call it.
 __device__ inline void wave_atomic_add(unsigned long long* p, unsigned long long v) {

@@ -552,6 +552,286 @@ double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nr
 }  // namespace gp
 
 // ---------------------------------------------------------------------------
+// Caller rows of mixed lengths, orders and PAFs (gp_psd_filter_batch), as they lie
+// in the caller's buffers:
+//   k_rows_count   rows of each length
+//   k_rows_order   row numbers grouped by length
+//   k_rows_filter  64 rows of one length at a time, gathered; thresholds per row
+// Bound by the copies of the caller's buffers: 1e5 rows of 9 to 25 letters at 32
+// bytes take 323 us, against 1681 us with the rows grouped and packed on the host
+// (the filter's own kernels took 50 us of that).
+
+namespace gp {
+
+struct RowsCtl {
+    uint32_t rows[kMaxN + 1];  // rows of each length
+    uint32_t used[kMaxN + 1];  // places of each length's group given out
+    BandCtl band;
+    unsigned long long passed;
+};
+struct RowsTables {
+    int16_t id[kMaxN + 1];  // table of each length present
+};
+
+constexpr int kRowsChunk = 1024;  // rows per block of the two grouping kernels
+
+__global__ void __launch_bounds__(256) k_rows_count(const int32_t* __restrict__ lens, int64_t count, RowsCtl* ctl) {
+    __shared__ uint32_t h[kMaxN + 1];
+    if (threadIdx.x <= kMaxN) h[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t end = min(((int64_t)blockIdx.x + 1) * kRowsChunk, count);
+    for (int64_t i = (int64_t)blockIdx.x * kRowsChunk + threadIdx.x; i < end; i += 256) atomicAdd(&h[lens[i]], 1u);
+    __syncthreads();
+    if (threadIdx.x <= kMaxN && h[threadIdx.x]) atomicAdd(&ctl->rows[threadIdx.x], h[threadIdx.x]);
+}
+
+// Lane l of a wave: rows of length l + 1, their first place, and the same in tiles of 64.
+struct RowsBins {
+    uint32_t rows, row0, tiles, tile0;
+    __device__ RowsBins(const RowsCtl* ctl, int lane) {
+        rows = ctl->rows[lane + 1];
+        tiles = (rows + 63) / 64;
+        row0 = rows;
+        tile0 = tiles;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t a = __shfl_up(row0, d), b = __shfl_up(tile0, d);
+            if (lane >= d) {
+                row0 += a;
+                tile0 += b;
+            }
+        }
+        row0 -= rows;
+        tile0 -= tiles;
+    }
+};
+
+__global__ void __launch_bounds__(256) k_rows_order(const int32_t* __restrict__ lens, int64_t count, RowsCtl* ctl,
+                                                    uint32_t* __restrict__ ids) {
+    __shared__ uint32_t h[kMaxN + 1], at[kMaxN + 1];
+    if (threadIdx.x <= kMaxN) h[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t end = min(((int64_t)blockIdx.x + 1) * kRowsChunk, count);
+    for (int64_t i = (int64_t)blockIdx.x * kRowsChunk + threadIdx.x; i < end; i += 256) atomicAdd(&h[lens[i]], 1u);
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const RowsBins b(ctl, threadIdx.x);
+        const uint32_t mine = h[threadIdx.x + 1];
+        at[threadIdx.x + 1] = mine ? b.row0 + atomicAdd(&ctl->used[threadIdx.x + 1], mine) : 0u;
+    }
+    __syncthreads();
+    for (int64_t i = (int64_t)blockIdx.x * kRowsChunk + threadIdx.x; i < end; i += 256)
+        ids[atomicAdd(&at[lens[i]], 1u)] = (uint32_t)i;
+}
+
+// What the tiles of a length need of a call.
+struct RowsCall {
+    const int8_t* words;
+    int64_t stride;
+    const int32_t *orders, *pafs;
+    const uint32_t* ids;
+    const PsdTableDesc* tabs;
+    const uint4* frags;
+    const float* trig32;
+    const double* trig64;
+    uint8_t* pass;
+    float* maxpsd;  // may be null
+};
+struct RowsSums {
+    unsigned long long passed = 0, band = 0, ties = 0;
+};
+
+// Decision of row id with the filter's value m and the error bound E on Re and Im;
+// band rows are settled in FP64, one at a time by the wave, or one per lane when
+// the tile holds many.
+__device__ __forceinline__ void rows_decide(const RowsCall& C, const PsdTableDesc& d, bool mine, uint32_t id, float m,
+                                            double E, int lane, RowsSums& S) {
+    const double thr = 2.0 * C.orders[id] - C.pafs[id] + 0.001, eps = psd_eps(E, thr);
+    const bool reject = m > nextafterf((float)(thr + eps), INFINITY);
+    bool accept = m < nextafterf((float)(thr - eps), -INFINITY);
+    const double* c = C.trig64 + d.trig_off;
+    unsigned long long bb = __ballot(mine && !reject && !accept);
+    if (bb) {
+        const bool in = bb >> lane & 1;
+        double v = 0.0;
+        if (__popcll(bb) > 12) {
+            if (in) v = fp64_max_psd(C.words + (int64_t)id * C.stride, d.n, c, c + d.n);
+        } else {
+            for (; bb; bb &= bb - 1) {
+                const int l = __ffsll((long long)bb) - 1;
+                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)id, l);
+                const double x = wave_max_psd(C.words + (int64_t)r * C.stride, d.n, c, c + d.n, lane);
+                if (lane == l) v = x;
+            }
+        }
+        if (in) {
+            accept = !(v > thr);
+            S.ties += fabs(v - thr) < 1e-9;
+            ++S.band;
+        }
+    }
+    if (mine) {
+        C.pass[id] = accept ? 1 : 0;
+        if (C.maxpsd) C.maxpsd[id] = m;
+    }
+    S.passed += mine && accept;
+}
+
+// `tiles` tiles of 64 rows from place p0 of the group that ends at `end`, in pairs of
+// 32-row tiles as in k_psd_mfma.  Rows may start at any byte.
+template <int NB, int MT>
+__device__ __forceinline__ void rows_tiles(const RowsCall& C, const PsdTableDesc& d, uint32_t p0, uint32_t end,
+                                           int64_t tiles, int lane, RowsSums& S) {
+    const int col = lane & 31, half = lane >> 5, n = d.n;
+    uint4 a[MT][2 * NB];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int s2 = 0; s2 < 2 * NB; ++s2) a[t][s2] = C.frags[d.frag_off + ((t * 2 * NB) + s2) * 64 + lane];
+    const double E1 = (double)d.rho_max + 1.004 * (32.0 * NB + 1.0) * 0x1p-23;  // split_bf16_E
+    for (int64_t q = 0; q < tiles; ++q, p0 += 64) {
+        const uint32_t id0 = C.ids[min(p0 + col, end - 1)], id1 = C.ids[min(p0 + 32 + col, end - 1)];
+        uint32_t sum[2];
+        uint4 b[2][NB];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const int8_t* w = C.words + (int64_t)(g ? id1 : id0) * C.stride + 8 * half;
+            sum[g] = 0;
+#pragma unroll
+            for (int bl = 0; bl < NB; ++bl) {
+                uint2 v;
+                __builtin_memcpy(&v, w + 16 * bl, 8);  // (past the row's end: the next row, or the allocation's slack)
+                if (bl + 1 == NB) v = keep_letters(v, n - 16 * bl - 8 * half);
+                sum[g] = abs_sum8(v, sum[g]);
+                b[g][bl] = pack8_bf16(v.x, v.y);
+            }
+        }
+        f32x16 acc0[MT], acc1[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc0[t] = acc1[t] = f32x16{};
+        mfma_tile_reg<NB, MT>(a, b[0], acc0);
+        mfma_tile_reg<NB, MT>(a, b[1], acc1);
+        float m = tile_pair_max_psd1(acc0[0], acc1[0]);
+#pragma unroll
+        for (int t = 1; t < MT; ++t) m = fmaxf(m, tile_pair_max_psd1(acc0[t], acc1[t]));
+        const auto sw = __builtin_amdgcn_permlane32_swap(sum[0], sum[1], false, false);
+        const double E = (double)((uint32_t)sw[0] + (uint32_t)sw[1]) * E1;
+        rows_decide(C, d, p0 + lane < end, half ? id1 : id0, m, E, lane, S);
+    }
+}
+
+// The same with the plain FP32 DFT, one row per lane.
+__device__ __forceinline__ void rows_fp32(const RowsCall& C, const PsdTableDesc& d, uint32_t p0, uint32_t end,
+                                          int64_t tiles, int lane, RowsSums& S) {
+    const float* c = C.trig32 + d.trig_off;
+    for (int64_t q = 0; q < tiles; ++q, p0 += 64) {
+        const uint32_t id = C.ids[min(p0 + lane, end - 1)];
+        const int8_t* w = C.words + (int64_t)id * C.stride;
+        int sum = 0;
+        for (int p = 0; p < d.n; ++p) sum += abs((int)w[p]);
+        const float m = d.K <= 16 ? fp32_max_psd<16>(w, d.n, d.K, c, c + d.n) : fp32_max_psd<32>(w, d.n, d.K, c, c + d.n);
+        const double E = (double)sum * ((double)(d.n + 2) * 0x1p-24) * 1.01;  // fp32_E
+        rows_decide(C, d, p0 + lane < end, id, m, E, lane, S);
+    }
+}
+
+template <bool FP32>
+__global__ void __launch_bounds__(256) k_rows_filter(RowsCall C, RowsTables T, RowsCtl* ctl, int64_t tpw) {
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const RowsBins bins(ctl, lane);
+    const int64_t total = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)(bins.tile0 + bins.tiles), 63);
+    const int64_t t1 = min((wave + 1) * tpw, total);
+    RowsSums S;
+    for (int64_t t = wave * tpw; t < t1;) {
+        // the length of tile t, and its run of tiles
+        const int l = __ffsll((long long)__ballot((int64_t)bins.tile0 + bins.tiles > t)) - 1;
+        const uint32_t rows = (uint32_t)__builtin_amdgcn_readlane((int)bins.rows, l);
+        const uint32_t row0 = (uint32_t)__builtin_amdgcn_readlane((int)bins.row0, l);
+        const int64_t tile0 = (uint32_t)__builtin_amdgcn_readlane((int)bins.tile0, l);
+        const int64_t run = min(t1, tile0 + (rows + 63) / 64) - t;
+        const PsdTableDesc d = C.tabs[T.id[l + 1]];
+        const uint32_t p0 = row0 + (uint32_t)(64 * (t - tile0)), end = row0 + rows;
+        if (FP32) rows_fp32(C, d, p0, end, run, lane, S);
+        else if (d.nb == 1) rows_tiles<1, 1>(C, d, p0, end, run, lane, S);
+        else if (d.nb == 2) rows_tiles<2, 1>(C, d, p0, end, run, lane, S);
+        else if (d.nb == 3 && d.mt == 1) rows_tiles<3, 1>(C, d, p0, end, run, lane, S);
+        else if (d.nb == 3) rows_tiles<3, 2>(C, d, p0, end, run, lane, S);
+        else rows_tiles<4, 2>(C, d, p0, end, run, lane, S);
+        t += run;
+    }
+    block_atomic_add(&ctl->passed, S.passed, &ctl->band.count, S.band, &ctl->band.ties, S.ties);
+}
+
+void filter_rows(gp_ctx* ctx, const int8_t* words, int stride, const int32_t* lens, const int32_t* orders,
+                 const int32_t* pafs, int64_t count, uint8_t* pass, float* max_psd, gp_stats* stats) {
+    if (count > 0x7FFFFFFFll) throw ArgError("gp_psd_filter_batch: more than 2^31 rows");
+    uint64_t present = 0;  // bit n - 1: length n
+    for (int64_t i = 0; i < count; ++i) {
+        if (lens[i] < 2 || lens[i] > kMaxN || lens[i] > stride) throw ArgError("word length out of range");
+        present |= 1ull << (lens[i] - 1);
+    }
+    RowsTables T{};
+    for (int n = 2; n <= kMaxN; ++n)
+        if (present >> (n - 1) & 1) T.id[n] = (int16_t)ctx->tables.get(n);
+    hipStream_t st = ctx->stream;
+    ctx->tables.upload(st);
+    RowsCall C{};
+    int8_t* d_words = static_cast<int8_t*>(ctx->words.ensure((size_t)count * stride + 64));
+    int32_t* d_int = static_cast<int32_t*>(ctx->aux5.ensure((size_t)count * 4 * 4));
+    uint32_t* ids = reinterpret_cast<uint32_t*>(d_int + 3 * count);
+    RowsCtl* ctl = static_cast<RowsCtl*>(ctx->counters.ensure(sizeof(RowsCtl)));
+    C.words = d_words;
+    C.stride = stride;
+    C.orders = d_int + count;
+    C.pafs = d_int + 2 * count;
+    C.ids = ids;
+    C.tabs = ctx->tables.d_desc.as<PsdTableDesc>();
+    C.frags = ctx->tables.d_frags.as<uint4>();
+    C.trig32 = ctx->tables.d_trig32.as<float>();
+    C.trig64 = ctx->tables.d_trig64.as<double>();
+    C.pass = static_cast<uint8_t*>(ctx->decisions.ensure((size_t)count));
+    C.maxpsd = max_psd ? static_cast<float*>(ctx->aux4.ensure((size_t)count * sizeof(float))) : nullptr;
+    GP_HIP(hipMemsetAsync(ctl, 0, sizeof(RowsCtl), st));
+    GP_HIP(hipMemcpyAsync(d_int, lens, (size_t)count * 4, hipMemcpyHostToDevice, st));
+    GP_HIP(hipMemcpyAsync(d_int + count, orders, (size_t)count * 4, hipMemcpyHostToDevice, st));
+    GP_HIP(hipMemcpyAsync(d_int + 2 * count, pafs, (size_t)count * 4, hipMemcpyHostToDevice, st));
+    GP_HIP(hipMemcpyAsync(d_words, words, (size_t)(count - 1) * stride + lens[count - 1], hipMemcpyHostToDevice, st));
+    const dim3 chunks((unsigned)((count + kRowsChunk - 1) / kRowsChunk));
+    hipLaunchKernelGGL(k_rows_count, chunks, dim3(256), 0, st, d_int, count, ctl);
+    hipLaunchKernelGGL(k_rows_order, chunks, dim3(256), 0, st, d_int, count, ctl, ids);
+    GP_HIP(hipGetLastError());
+    // at most this many tiles; two waves per SIMD stay resident
+    const int64_t tiles = count / 64 + __builtin_popcountll(present);
+    const int64_t waves = std::min<int64_t>(tiles, (int64_t)ctx->num_cus * 8), tpw = (tiles + waves - 1) / waves;
+    const dim3 grid((unsigned)((waves + 3) / 4));
+    if (stats) GP_HIP(hipEventRecord(ctx->ev0, st));
+    if (ctx->psd_mode == GP_PSD_SPLIT_BF16)
+        hipLaunchKernelGGL(k_rows_filter<false>, grid, dim3(256), 0, st, C, T, ctl, tpw);
+    else
+        hipLaunchKernelGGL(k_rows_filter<true>, grid, dim3(256), 0, st, C, T, ctl, tpw);
+    GP_HIP(hipGetLastError());
+    if (stats) GP_HIP(hipEventRecord(ctx->ev1, st));
+    GP_HIP(hipMemcpyAsync(pass, C.pass, (size_t)count, hipMemcpyDeviceToHost, st));
+    if (max_psd) GP_HIP(hipMemcpyAsync(max_psd, C.maxpsd, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, st));
+    RowsCtl h;
+    if (stats) GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
+    GP_HIP(hipStreamSynchronize(st));
+    if (stats) {
+        float ms = 0;
+        GP_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        stats->band_rechecks += h.band.count;
+        stats->tie_band += h.band.ties;
+        stats->psd_decisions += (uint64_t)count;
+        stats->psd_pass += h.passed;
+        stats->psd_kernel_ms += ms;
+        stats->psd_launches += 1;
+        stats->kernel_ms += ms;
+    }
+}
+
+}  // namespace gp
+
+// ---------------------------------------------------------------------------
 // The batched PSD filter without allocation (gp_psd_filter_batch_static).
 //
 // Everything the call needs beyond the caller's words and pass flags lives in
@@ -628,25 +908,6 @@ int64_t na_waves(const PsdTableDesc& d, int num_cus) {
     return (int64_t)num_cus * 4 * (d.mt == 1 ? 4 : d.nb == 3 ? 3 : 2);
 }
 
-// FP64 max PSD of the row at w by the whole wave: lane q < n / 2 takes k = q + 1
-// in the summation order of fp64_max_psd; the result is in every lane.
-__device__ __forceinline__ double na_wave_max_psd(const int8_t* __restrict__ w, int n, const double* tw, int lane) {
-    const int x = lane < n ? (int)w[lane] : 0;
-    const int k = lane < (n >> 1) ? lane + 1 : 0;  // (idle lanes: k = 0, their value is dropped)
-    double re = 0.0, im = 0.0;
-    int m = 0;
-    for (int p = 0; p < n; ++p) {
-        const double v = (double)__builtin_amdgcn_readlane(x, p);
-        re = __builtin_fma(v, tw[m], re);
-        im = __builtin_fma(v, tw[n + m], im);
-        m += k;
-        if (m >= n) m -= n;
-    }
-    double mx = k ? re * re + im * im : 0.0;
-    for (int o = 32; o; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
-    return mx;
-}
-
 // The whole filter of one word length in one pass over the rows, tiles of 32
 // rows in pairs as in k_psd_mfma.  The error bound of a row needs its sum
 // |x_p|: four letters per v_sad_u8 on the letters the wave holds anyway, so a
@@ -688,19 +949,11 @@ __global__ void __launch_bounds__(256) k_na_filter(const int8_t* __restrict__ wo
     }
     for (int i = threadIdx.x; i < 2 * n; i += blockDim.x) tw[i] = trig64[i];
     __syncthreads();
-    // the last block's letters past n do not count
-    const int left = n - 16 * (NB - 1) - 8 * half;  // letters of this lane's 8 bytes there
-    const uint32_t k0 = left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
-    const uint32_t k1 = left >= 8 ? ~0u : left <= 4 ? 0u : (1u << (8 * (left - 4))) - 1u;
+    const int left = n - 16 * (NB - 1) - 8 * half;  // letters of this lane's last 8 bytes: those past n do not count
     auto row_sum = [&](const uint2 (&raw)[NB]) {
-        constexpr uint32_t z = 0x80808080u;  // |x| = |(x + 128) - 128| on unsigned bytes
-        uint32_t s = 0;
+        uint32_t s = abs_sum8(keep_letters(raw[NB - 1], left), 0);
 #pragma unroll
-        for (int bl = 0; bl < NB; ++bl) {
-            const uint32_t x = bl + 1 < NB ? raw[bl].x : raw[bl].x & k0, y = bl + 1 < NB ? raw[bl].y : raw[bl].y & k1;
-            s = __builtin_amdgcn_sad_u8(x ^ z, z, s);
-            s = __builtin_amdgcn_sad_u8(y ^ z, z, s);
-        }
+        for (int bl = 0; bl + 1 < NB; ++bl) s = abs_sum8(raw[bl], s);
         return s;
     };
     unsigned long long nband = 0, nties = 0, npass = 0;
@@ -746,7 +999,7 @@ __global__ void __launch_bounds__(256) k_na_filter(const int8_t* __restrict__ wo
                     while (bb) {
                         const int l = __ffsll((long long)bb) - 1;
                         bb &= bb - 1;
-                        const double v = na_wave_max_psd(words + (q * 32 + l) * stride, n, tw, lane);
+                        const double v = wave_max_psd(words + (q * 32 + l) * stride, n, tw, tw + n, lane);
                         if (lane == l) {
                             accept = !(v > th.thr);
                             nties += fabs(v - th.thr) < 1e-9;

@@ -160,6 +160,36 @@ def test_psd_edge_cases(gpu_ctx, name, mode):
     assert (gp_pass == ref_pass).all()
 
 
+@pytest.mark.parametrize("name,mode", MODES)
+@pytest.mark.parametrize("stride,groups", [
+    (2, [(2, 1)]), (9, [(9, 64), (3, 65), (5, 1), (8, 63)]), (17, [(16, 129), (17, 2), (2, 1000)]),
+    (33, [(33, 700), (32, 31), (25, 4000)]), (64, [(64, 100), (48, 65), (36, 63), (50, 130), (10, 3)]),
+])
+def test_psd_rows_tiles_and_strides(gpu_ctx, name, mode, stride, groups):
+    """Lengths with 1, 63, 64, 65 rows in mixed order, rows at any byte, letters past a
+    row's length that are not zero, thresholds of their own, and rows at the
+    threshold (an alternating word has PSD n^2 at n / 2), few and many in a tile."""
+    rng = np.random.default_rng(stride)
+    lens = np.concatenate([np.full(k, n, np.int32) for n, k in groups])
+    words = rng.integers(-3, 4, size=(len(lens), stride)).astype(np.int8)
+    orders = (lens * rng.integers(1, 6, len(lens))).astype(np.int32)
+    pafs = rng.integers(-3, 4, len(lens)).astype(np.int32)
+    hard = rng.random(len(lens)) < np.where(lens % 4 == 0, 0.05, 0.6)
+    words[hard] = 1 - 2 * (np.arange(stride) % 2)
+    orders[hard], pafs[hard] = 0, -(lens[hard] ** 2)
+    at = rng.permutation(len(lens))
+    words, lens, orders, pafs = words[at], lens[at], orders[at], pafs[at]
+    gpu_ctx.set_mode(mode)
+    try:
+        got, mx, st = gpu_ctx.psd_filter_batch(words, lens, orders, pafs, want_max=True)
+    finally:
+        gpu_ctx.set_mode(g.GP_PSD_SPLIT_BF16)
+    want, ref = _oracle.psd_filter_batch(words, lens, orders, pafs)
+    assert (got == want).all(), np.nonzero(got != want)[0][:10]
+    assert (np.abs(mx - ref) <= _row_bounds(words, lens, orders, pafs, mode, mx)).all()
+    assert st.psd_pass == want.sum() and st.psd_decisions == len(lens)
+
+
 MIX_SMALL = [  # n, c, order, paf, share  (the microbenchmark mix at 1/64 scale)
     [9, 10, 90, 0, 1 << 19],
     [10, 5, 50, 0, 1 << 18],
