@@ -19,10 +19,6 @@ std::vector<std::pair<int, int>> getdecomps(int k);
 // every job enumerates everything (proc_num == 1 or no prefix length < n
 // reaches proc_num * 10^4 necklaces).
 int shard_prefix_len(int n, int k, int proc_num);
-// Digit-index values (base k, first digit most significant) of the
-// prenecklaces of length `len` whose 1-based FKM count is = proc_id mod proc_num.
-std::vector<uint64_t> shard_prefixes(int len, const std::vector<int>& alphabet, int proc_id, int proc_num);
-
 // Host copy of a candidate set: words (count x n) and key digits (count x nkey).
 struct CandSet {
     int n = 0, nkey = 0;

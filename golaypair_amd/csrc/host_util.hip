@@ -48,36 +48,6 @@ int shard_prefix_len(int n, int k, int proc_num) {
     return i < n ? i : 0;
 }
 
-std::vector<uint64_t> shard_prefixes(int len, const std::vector<int>& alphabet, int proc_id, int proc_num) {
-    // FKM prenecklace recursion over letter indices, lexicographic order.
-    const int k = (int)alphabet.size();
-    std::vector<int> d(len, 0);
-    std::vector<uint64_t> out;
-    uint64_t count = 0;
-    std::function<void(int, int)> rec = [&](int index, int period) {
-        if (index == len) {
-            ++count;
-            if ((int64_t)(count % (uint64_t)proc_num) == proc_id) {
-                uint64_t v = 0;
-                for (int p = 0; p < len; ++p) v = v * (uint64_t)k + (uint64_t)d[p];
-                out.push_back(v);
-            }
-            return;
-        }
-        d[index] = d[index - period];
-        rec(index + 1, period);
-        for (int c = d[index - period] + 1; c < k; ++c) {
-            d[index] = c;
-            rec(index + 1, index + 1);
-        }
-    };
-    for (int c = 0; c < k; ++c) {
-        d[0] = c;
-        rec(1, 1);
-    }
-    return out;
-}
-
 int export_cands(const CandSet& s, gp_cands* out) {
     if (!out) return GP_ERR_ARG;
     const int64_t m = s.size();

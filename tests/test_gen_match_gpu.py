@@ -137,3 +137,40 @@ def test_match_many_equal_keys(gpu_ctx, n, ma, mb, nkeys):
     rc, pa, pb, st = gpu_ctx.match(n, 1, target, g.Cands(wa, kinds[xa]), g.Cands(wb, kinds[xb]))
     assert st.pair_checks == int((xa[:, None] == xb[None, :]).sum())
     assert [(x.tolist(), y.tolist()) for x, y in zip(pa, pb)] == [(wa[i].tolist(), wb[j].tolist()) for i, j in want]
+
+
+@pytest.mark.parametrize("order,compress,paf,njobs", [
+    (8, 2, 0, 1), (26, 1, 0, 1), (26, 2, 0, 7), (34, 2, 0, 5), (45, 3, -2, 40), (50, 5, 0, 3), (50, 5, 0, 1000),
+])
+def test_gen_jobs_and_word_widths(gpu_ctx, order, compress, paf, njobs):
+    """The shards of a level together are the level (each is the level where the job
+    split has no prefix length), and the 2-bit and 4-bit packed words agree (the FP32
+    path packs every level in 4 bits)."""
+    rows = lambda c: sorted(c.lines())
+    a, b, _ = gpu_ctx.generate(order, compress, paf)
+    gpu_ctx.set_mode(g.GP_PSD_FP32)
+    try:
+        fa, fb, _ = gpu_ctx.generate(order, compress, paf)
+        ja, jb, _ = gpu_ctx.generate(order, compress, paf, njobs - 1, njobs)
+    finally:
+        gpu_ctx.set_mode(g.GP_PSD_SPLIT_BF16)
+    assert fa.lines() == a.lines() and fb.lines() == b.lines()
+    parts = [gpu_ctx.generate(order, compress, paf, j, njobs)[:2] for j in range(min(njobs, 40))]
+    if njobs <= 40:
+        assert ja.lines() == parts[-1][0].lines() and jb.lines() == parts[-1][1].lines()
+    if all(p[0].lines() == a.lines() and p[1].lines() == b.lines() for p in parts):
+        return
+    assert njobs <= 40
+    assert sorted(sum((p[0].lines() for p in parts), [])) == rows(a)
+    assert sorted(sum((p[1].lines() for p in parts), [])) == rows(b)
+
+
+def test_gen_wide_words(gpu_ctx):
+    """Words of more than 64 bits (17 letters of an alphabet of 5): one shard of many."""
+    a, b, _ = gpu_ctx.generate(68, 4, 0, 7, 1000)
+    gpu_ctx.set_mode(g.GP_PSD_FP32)
+    try:
+        fa, fb, _ = gpu_ctx.generate(68, 4, 0, 7, 1000)
+    finally:
+        gpu_ctx.set_mode(g.GP_PSD_SPLIT_BF16)
+    assert len(a) + len(b) > 0 and a.lines() == fa.lines() and b.lines() == fb.lines()
