@@ -105,11 +105,11 @@ int gp_sort_candidates(gp_ctx* ctx, gp_cands* c) {
         uint8_t* dk = ctx->dev<uint8_t>("s_k", (size_t)m * K);
         int8_t* ow = ctx->dev<int8_t>("s_ow", (size_t)m * n);
         uint8_t* ok = ctx->dev<uint8_t>("s_ok", (size_t)m * K + 1);
-        GP_HIP(hipMemcpyAsync(dw, c->words, (size_t)m * n, hipMemcpyHostToDevice, st));
-        GP_HIP(hipMemcpyAsync(dk, c->keys, (size_t)m * K, hipMemcpyHostToDevice, st));
+        copy_to_device(ctx, dw, c->words, (size_t)m * n);
+        copy_to_device(ctx, dk, c->keys, (size_t)m * K);
         const int64_t kept = sort_uniq_cands(ctx, dw, dk, m, n, K, ow, ok);
-        GP_HIP(hipMemcpyAsync(c->words, ow, (size_t)kept * n, hipMemcpyDeviceToHost, st));
-        if (K > 0) GP_HIP(hipMemcpyAsync(c->keys, ok, (size_t)kept * K, hipMemcpyDeviceToHost, st));
+        copy_to_host(ctx, c->words, ow, (size_t)kept * n);
+        copy_to_host(ctx, c->keys, ok, (size_t)kept * K);
         GP_HIP(hipStreamSynchronize(st));
         c->count = kept;
         return GP_OK;
@@ -126,16 +126,15 @@ int gp_match(gp_ctx* ctx, int order, int compress, int paf, const gp_cands* a_so
         const int n = order / compress;
         if (a_sorted->n != n || b_sorted->n != n) throw ArgError("gp_match: word length != order/compress");
         if (a_sorted->nkey != n / 2 || b_sorted->nkey != n / 2) throw ArgError("gp_match: nkey must be n/2");
-        hipStream_t st = ctx->stream;
         const int64_t na = a_sorted->count, nb = b_sorted->count;
         int8_t* wa = ctx->dev<int8_t>("m_wa", (size_t)na * n);
         int8_t* wb = ctx->dev<int8_t>("m_wb", (size_t)nb * n);
         uint8_t* ka = ctx->dev<uint8_t>("m_ka", (size_t)na * (n / 2));
         uint8_t* kb = ctx->dev<uint8_t>("m_kb", (size_t)nb * (n / 2));
-        GP_HIP(hipMemcpyAsync(wa, a_sorted->words, (size_t)na * n, hipMemcpyHostToDevice, st));
-        GP_HIP(hipMemcpyAsync(wb, b_sorted->words, (size_t)nb * n, hipMemcpyHostToDevice, st));
-        GP_HIP(hipMemcpyAsync(ka, a_sorted->keys, (size_t)na * (n / 2), hipMemcpyHostToDevice, st));
-        GP_HIP(hipMemcpyAsync(kb, b_sorted->keys, (size_t)nb * (n / 2), hipMemcpyHostToDevice, st));
+        copy_to_device(ctx, wa, a_sorted->words, (size_t)na * n);
+        copy_to_device(ctx, wb, b_sorted->words, (size_t)nb * n);
+        copy_to_device(ctx, ka, a_sorted->keys, (size_t)na * (n / 2));
+        copy_to_device(ctx, kb, b_sorted->keys, (size_t)nb * (n / 2));
         JoinResult jr = join_pairs(ctx, wa, ka, na, wb, kb, nb, n, n / 2, n, n / 2, paf * compress, stats);
         PairSet ps;
         ps.n = n;
@@ -165,13 +164,13 @@ int gp_psd_keys(gp_ctx* ctx, const int8_t* words, int stride, int n, int64_t cou
         int8_t* dw = ctx->dev<int8_t>("k_w", (size_t)count * stride);
         uint8_t* dk = ctx->dev<uint8_t>("k_k", (size_t)count * (n / 2));
         unsigned int* bad = ctx->dev<unsigned int>("k_bad", 1);
-        GP_HIP(hipMemcpyAsync(dw, words, (size_t)count * stride, hipMemcpyHostToDevice, st));
+        copy_to_device(ctx, dw, words, (size_t)count * stride);
         GP_HIP(hipMemsetAsync(bad, 0, 4, st));
         hipLaunchKernelGGL(k_keys_all, dim3(ctx->num_cus * 4), dim3(256), 0, st, dw, stride, count, n,
                            ctx->tables.d_trig64.as<double>() + d.trig_off, bound, inverted, dk, n / 2, bad);
         GP_HIP(hipGetLastError());
         unsigned int hb = 0;
-        GP_HIP(hipMemcpyAsync(keys, dk, (size_t)count * (n / 2), hipMemcpyDeviceToHost, st));
+        copy_to_host(ctx, keys, dk, (size_t)count * (n / 2));
         GP_HIP(hipMemcpyAsync(&hb, bad, 4, hipMemcpyDeviceToHost, st));
         GP_HIP(hipStreamSynchronize(st));
         if (hb) throw ArgError("gp_psd_keys: key digit outside [0, 255]");

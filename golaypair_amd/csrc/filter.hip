@@ -497,8 +497,8 @@ int filter_pairs(gp_ctx* ctx, int order, int compress, const gp_pairs& in, PairS
     int8_t* db = ctx->dev<int8_t>("f_b", (size_t)m * n);
     FilterCtl* ctl = ctx->dev<FilterCtl>("f_ctl", 1);
     GP_HIP(hipMemsetAsync(ctl, 0, sizeof(FilterCtl), st));
-    GP_HIP(hipMemcpyAsync(da, in.a, (size_t)m * n, hipMemcpyHostToDevice, st));
-    GP_HIP(hipMemcpyAsync(db, in.b, (size_t)m * n, hipMemcpyHostToDevice, st));
+    copy_to_device(ctx, da, in.a, (size_t)m * n);
+    copy_to_device(ctx, db, in.b, (size_t)m * n);
     const auto blocks = [&](int64_t threads, int per_cu) {
         return dim3((unsigned)std::min<int64_t>((threads + 255) / 256, (int64_t)ctx->num_cus * per_cu));
     };
@@ -559,8 +559,8 @@ int filter_pairs(gp_ctx* ctx, int order, int compress, const gp_pairs& in, PairS
     GP_HIP(hipGetLastError());
     out.a.resize((size_t)kept * n);
     out.b.resize((size_t)kept * n);
-    GP_HIP(hipMemcpyAsync(out.a.data(), oa, out.a.size(), hipMemcpyDeviceToHost, st));
-    GP_HIP(hipMemcpyAsync(out.b.data(), ob, out.b.size(), hipMemcpyDeviceToHost, st));
+    copy_to_host(ctx, out.a.data(), oa, out.a.size());
+    copy_to_host(ctx, out.b.data(), ob, out.b.size());
     GP_HIP(hipStreamSynchronize(st));
     if (stats) stats->pairs += (uint64_t)kept;
     return GP_OK;

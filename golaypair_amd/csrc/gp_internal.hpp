@@ -229,6 +229,13 @@ struct gp_ctx {
 
 namespace gp {
 
+// Copies on the context's stream (copies.hip): from the caller's memory, which may
+// be changed after the return; and to it, complete after the next synchronization
+// of the stream.
+constexpr size_t kStagedCopy = 8 << 20;  // from this size on through the pinned pool
+void copy_to_device(gp_ctx* ctx, void* dst, const void* src, size_t bytes);
+void copy_to_host(gp_ctx* ctx, void* dst, const void* src, size_t bytes);
+
 // Tuning table (tuning.hip): loaded from the tuning file when a context is
 // created; tuned(ctx, key, dflt) is the table's value or dflt.
 void load_tuning(gp_ctx* ctx);

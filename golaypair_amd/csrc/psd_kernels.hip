@@ -792,10 +792,10 @@ void filter_rows(gp_ctx* ctx, const int8_t* words, int stride, const int32_t* le
     C.pass = static_cast<uint8_t*>(ctx->decisions.ensure((size_t)count));
     C.maxpsd = max_psd ? static_cast<float*>(ctx->aux4.ensure((size_t)count * sizeof(float))) : nullptr;
     GP_HIP(hipMemsetAsync(ctl, 0, sizeof(RowsCtl), st));
-    GP_HIP(hipMemcpyAsync(d_int, lens, (size_t)count * 4, hipMemcpyHostToDevice, st));
-    GP_HIP(hipMemcpyAsync(d_int + count, orders, (size_t)count * 4, hipMemcpyHostToDevice, st));
-    GP_HIP(hipMemcpyAsync(d_int + 2 * count, pafs, (size_t)count * 4, hipMemcpyHostToDevice, st));
-    GP_HIP(hipMemcpyAsync(d_words, words, (size_t)(count - 1) * stride + lens[count - 1], hipMemcpyHostToDevice, st));
+    copy_to_device(ctx, d_int, lens, (size_t)count * 4);
+    copy_to_device(ctx, d_int + count, orders, (size_t)count * 4);
+    copy_to_device(ctx, d_int + 2 * count, pafs, (size_t)count * 4);
+    copy_to_device(ctx, d_words, words, (size_t)(count - 1) * stride + lens[count - 1]);
     const dim3 chunks((unsigned)((count + kRowsChunk - 1) / kRowsChunk));
     hipLaunchKernelGGL(k_rows_count, chunks, dim3(256), 0, st, d_int, count, ctl);
     hipLaunchKernelGGL(k_rows_order, chunks, dim3(256), 0, st, d_int, count, ctl, ids);
@@ -811,8 +811,8 @@ void filter_rows(gp_ctx* ctx, const int8_t* words, int stride, const int32_t* le
         hipLaunchKernelGGL(k_rows_filter<true>, grid, dim3(256), 0, st, C, T, ctl, tpw);
     GP_HIP(hipGetLastError());
     if (stats) GP_HIP(hipEventRecord(ctx->ev1, st));
-    GP_HIP(hipMemcpyAsync(pass, C.pass, (size_t)count, hipMemcpyDeviceToHost, st));
-    if (max_psd) GP_HIP(hipMemcpyAsync(max_psd, C.maxpsd, (size_t)count * sizeof(float), hipMemcpyDeviceToHost, st));
+    copy_to_host(ctx, pass, C.pass, (size_t)count);
+    if (max_psd) copy_to_host(ctx, max_psd, C.maxpsd, (size_t)count * sizeof(float));
     RowsCtl h;
     if (stats) GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
     GP_HIP(hipStreamSynchronize(st));

@@ -102,6 +102,18 @@ def test_psd_keys_match_oracle_lines(gpu_ctx):
         assert [g.cand_line(w, k) for w, k in zip(words, keys)] == lines
 
 
+@pytest.mark.parametrize("count", [524287, 524288, 1048577, 1300001])
+def test_psd_keys_of_large_buffers(gpu_ctx, count):
+    """Caller buffers on both sides of the size from which copies go through pinned
+    memory in chunks (8 MiB: 524288 words, the keys of 1048576), against small calls."""
+    rng = np.random.default_rng(count)
+    words = rng.choice(np.array([-1, 1], np.int8), size=(count, 16))
+    words[:, 0] = 0  # every PSD below 256
+    got = gpu_ctx.psd_keys(words, 255, False)
+    want = np.concatenate([gpu_ctx.psd_keys(words[i:i + 100000], 255, False) for i in range(0, count, 100000)])
+    assert (got == want).all()
+
+
 def _golden(name):
     p = os.path.join(GOLDEN, name)
     if not os.path.exists(p):
