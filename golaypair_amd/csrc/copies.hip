@@ -1,7 +1,7 @@
 // Copies between the caller's ordinary memory and the device.  The runtime's copy
 // of unpinned memory runs at 30 GB/s to the device and 18 GB/s back, one thread
 // filling or emptying its staging memory.  A large copy goes through pinned
-// buffers of the context's pool instead, filled or emptied by the host threads
+// buffers of the context instead, filled or emptied by the host threads
 // while the DMA of the chunks before runs (57 GB/s).  Sorting 4e6 records of 22
 // bytes, 88 MB each way, takes 5.0 ms instead of 8.5 ms; chunks of 1 MB give 7.5 ms
 // (the threads' start and end shows), of 8 MB 4.9 ms.  Copies below kStagedCopy gain
@@ -46,7 +46,7 @@ void copy_to_device(gp_ctx* ctx, void* dst, const void* src, size_t bytes) {
         if (bytes) GP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
         return;
     }
-    Ring ring(ctx->pinned);
+    Ring ring(ctx->copy_pinned);
     int i = 0;
     for (size_t at = 0; at < bytes; at += kChunk, i = (i + 1) % kBufs) {
         PinnedBuf& b = *ring.b[i];
@@ -64,7 +64,7 @@ void copy_to_host(gp_ctx* ctx, void* dst, const void* src, size_t bytes) {
         if (bytes) GP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
         return;
     }
-    Ring ring(ctx->pinned);
+    Ring ring(ctx->copy_pinned);
     size_t sent = 0, at = 0;  // bytes whose DMA is queued; bytes delivered
     int is = 0, ia = 0;
     while (at < bytes) {

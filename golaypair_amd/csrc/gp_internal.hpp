@@ -214,7 +214,11 @@ struct gp_ctx {
     gp::PairSet unc_cache_out;
     gp::CandSet unc_cache_ta, unc_cache_tb;
     gp_stats unc_cache_stats{};
-    gp::PinnedPool pinned;  // staging for batch uploads
+    gp::PinnedPool pinned;  // staging for batch uploads, taken by the threads that prepare batches
+    // staging of copies.hip, whose events are recorded on `stream`: a pool of its own,
+    // as another thread that waits for such an event while a batch is being captured on
+    // `stream` would end the capture
+    gp::PinnedPool copy_pinned;
     // named scratch buffers of the pipeline stages
     std::map<std::string, std::unique_ptr<gp::DevBuf>> pool;
     gp::DevBuf& buf(const std::string& name) {

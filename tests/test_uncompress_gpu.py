@@ -315,3 +315,20 @@ def test_uncompress_side_filter_tiles(gpu_ctx, L, c, c2, free, paf, seed):
         cands, rot, st = gpu_ctx.uncompress_side(seq, c, c2, paf, seqflag)
         assert "".join(l + "\n" for l in cands.lines()) == ref_text
         assert st.psd_decisions == ref_leaves
+
+
+def test_uncompress_after_large_copies(gpu_ctx, monkeypatch):
+    """A call whose buffers go through the staging memory of large copies, then an
+    uncompression in many batches (graph captures beside the threads that prepare
+    the next batches), again and again on one context."""
+    order, compress, paf = 26, [2, 1], 0
+    wd = _oracle_dir(order, compress, paf, ["gen", "sort", "match", "uncompress"])
+    pa, pb = _read_pairs(os.path.join(wd, "%d-pairs-%d" % (order, 2)), order // 2)
+    want = open(os.path.join(wd, "%d-pairs-%d" % (order, 1))).read()
+    monkeypatch.setenv("GOLAY_UNC_BATCH_LEAVES", "64")
+    words = np.random.default_rng(5).choice(np.array([-1, 1], np.int8), size=(1100000, 16))
+    words[:, 0] = 0
+    for _ in range(3):
+        gpu_ctx.psd_keys(words, 255, False)  # 17 MB up, 8.8 MB back
+        oa, ob, _, _, _ = gpu_ctx.uncompress(order, 2, 1, paf, pa, pb)
+        assert "".join(g.pair_line(x, y) + "\n" for x, y in zip(oa, ob)) == want
