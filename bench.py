@@ -7,8 +7,7 @@ compression 5 -> 1, on the GPU through the C ABI:
   canonical, PSD filter), sort + match at c=5 (4 691 pairs), uncompression 5 -> 1
   of every matched pair (9.2e11 length-50 words over {-1,1}: PSD filter + keys +
   re-match with exact PAF), equivalence filter at length 50 with altnegative.
-value = PSD-filter decisions of the step / wall time of the step (split-BF16 MFMA
-path).  Beside it: the plain FP32 path on a fixed slice of the v=50 pairs (same
+value = PSD-filter decisions of the step / wall time of the step (the MFMA path).  Beside it: the plain FP32 path on a fixed slice of the v=50 pairs (same
 output required), the mixed-length PSD microbenchmark, and the CPU oracle on P
 processes.
 
@@ -29,8 +28,10 @@ sys.path.insert(0, ROOT)
 
 ORDER, C0, C1, PAF = 50, 5, 1, 0
 N1 = ORDER // C1
-FLOPS_PER_LEAF = 4 * N1 * (N1 // 2) + 3 * (N1 // 2)   # algorithmic: real DFT k=1..25 of n=50 + |X|^2 = 5075
-MFMA_PEAK_TFLOPS = 2500.0                             # MI355X dense BF16
+# the filter's matrix product per leaf: 16 multiply-adds (12 features, padded) for each of the 20 channels that
+# the compressed word does not fix = 640 (a direct real DFT at k = 1..25 with |X|^2 would take 5075)
+FLOPS_PER_LEAF = 2 * 16 * (N1 // 2 - N1 // (2 * C0))
+MFMA_PEAK_TFLOPS = 2500.0                             # MI355X dense f16 / BF16
 HBM_PEAK = 8e12                                       # MI355X HBM3E, bytes/s
 FP32_SLICE = (0, 64)                                  # matched c=5 pairs [0, 64) in file order
 PROFILE = "k_unc_filter_v50_golay_search.md"
@@ -394,13 +395,13 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "bf16",
+        "dtype": "fp16",
         "data": "synthetic",
         "config": {"workload": "v=50 Golay-pair search (paf 0): gen at c=5, sort, match, uncompress 5->1 of all "
                                "matched pairs, equivalence filter at length 50 with altnegative; exhaustive, "
                                "no input data",
-                   "order": ORDER, "compress": [C0, C1], "paf": PAF, "psd": "split-BF16 MFMA, FP32 accumulate, "
-                   "FP64 band recheck and keys"},
+                   "order": ORDER, "compress": [C0, C1], "paf": PAF, "psd": "f16 feature MFMA (split-BF16 in gen), FP32 "
+                   "accumulate, FP64 band recheck and keys"},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / MFMA_PEAK_TFLOPS, "traffic": profiled_traffic(),
                      "traffic_source": "profiles/%s (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this workload, "
