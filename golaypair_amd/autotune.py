@@ -6,11 +6,11 @@ table every context loads (gp_create; keys in golaypair_amd/csrc/tuning.hip).
 
 Per workload (order, compression pair, PAF constant):
   gen_ranks_per_lane/<n>/<k>   ranks per lane of the gen kernel at word length
-                               n over k letters: candidates 16 .. 256, timed by
+                               n over k letters: candidates 4 .. 64, timed by
                                gp_generate at the coarse compression;
   unc_waves/<N>                waves per SIMD of the uncompression filter at
-                               finer length N (capped by each operand class's
-                               occupancy): candidates 1 .. 5;
+                               finer length N (capped by the registers of its
+                               number of channels): candidates 1 .. 3;
   unc_leaf_budget/<N>          leaves per uncompression device batch:
                                candidates 2^27 .. 2^31;
   unc_counter_rounds/<N>       rounds of filter work items handed out by the
@@ -42,8 +42,8 @@ WORKLOADS = {
     "v45": (45, 3, 1, -2, (0, 2500)),
     "v90": (90, 10, 5, 0, (0, 156)),
 }
-GEN_RANKS = [16, 32, 64, 128, 256]
-UNC_WAVES = [1, 2, 3, 4, 5]
+GEN_RANKS = [4, 8, 16, 32, 64]
+UNC_WAVES = [1, 2, 3]
 UNC_BUDGET = [1 << 27, 1 << 28, 1 << 29, 1 << 30, 1 << 31]
 UNC_COUNTER_ROUNDS = [0, 1, 2, 4]
 UNC_COUNTER_STREAMS = [1, 2, 4]
