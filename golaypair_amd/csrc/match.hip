@@ -52,18 +52,38 @@ struct JoinCtl {
     unsigned long long cand;
 };
 
-// Appends x of the lanes with `have` to list (at most cap entries kept) with one
-// atomic per wave; every lane of the wave must call it.
-__device__ __forceinline__ void wave_append(unsigned long long* count, bool have, uint64_t x, uint64_t* list,
-                                            int64_t cap) {
-    const unsigned long long b = __ballot(have);
-    if (!b) return;
-    const int lane = threadIdx.x & 63;
-    unsigned long long base = 0;
-    if (lane == 0) base = atomicAdd(count, (unsigned long long)__popcll(b));
-    base = __shfl(base, 0) + __popcll(b & ((1ull << lane) - 1ull));
-    if (have && (int64_t)base < cap) list[base] = x;
-}
+// Entries that a wave appends to a list (at most cap kept), collected in LDS so that
+// about 200 take one atomic: atomics on one address are applied one at a time, and
+// one per step of a wave made the probe of 2^21 records a side with 2^20 candidates
+// take 1.63 ms instead of 0.20 ms.  Every lane of the wave must call push and flush.
+struct WaveQueue {
+    static constexpr int kCap = 256;
+    uint64_t* q;
+    unsigned long long* count;
+    uint64_t* list;
+    int64_t cap;
+    int n = 0;
+    __device__ void push(bool have, uint64_t x) {
+        const unsigned long long b = __ballot(have);
+        if (have) q[n + __popcll(b & ((1ull << (threadIdx.x & 63)) - 1ull))] = x;
+        n += __popcll(b);
+        if (n > kCap - 64) flush();
+    }
+    __device__ void flush() {
+        if (n == 0) return;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the other lanes' writes
+        __builtin_amdgcn_wave_barrier();
+        const int lane = threadIdx.x & 63;
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(count, (unsigned long long)n);
+        base = __shfl(base, 0);
+        for (int x = lane; x < n; x += 64)
+            if ((int64_t)(base + x) < cap) list[base + x] = q[x];
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        n = 0;
+    }
+};
 
 // Candidate pairs A << 32 | B with equal key tuples, one A record per lane.
 __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ ka, int64_t na,
@@ -72,6 +92,8 @@ __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ 
                                                     const uint32_t* __restrict__ next,
                                                     const uint32_t* __restrict__ head, uint32_t mask,
                                                     uint64_t* __restrict__ cand, int64_t cap, JoinCtl* ctl) {
+    __shared__ uint64_t queue[4][WaveQueue::kCap];
+    WaveQueue out{queue[threadIdx.x >> 6], &ctl->cand, cand, cap};
     for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < na; i0 += (int64_t)gridDim.x * 256) {
         const int64_t i = i0 + threadIdx.x;
         const uint8_t* k = ka + i * kstride;
@@ -92,9 +114,10 @@ __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ 
                 const uint8_t* k2 = kb + (int64_t)at * kstride;
                 for (int q = 0; q < nkey && eq; ++q) eq = k[q] == k2[q];
             }
-            wave_append(&ctl->cand, eq, (uint64_t)i << 32 | at, cand, cap);
+            out.push(eq, (uint64_t)i << 32 | at);
         }
     }
+    out.flush();
 }
 
 // The PAF condition of each candidate by 8 lanes, which take the shifts in turn
@@ -103,6 +126,8 @@ __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ 
 __global__ void __launch_bounds__(256) k_join_check(const int8_t* __restrict__ wa, const int8_t* __restrict__ wb, int n,
                                                     int wstride, int target, const uint64_t* __restrict__ cand,
                                                     int64_t cap, uint64_t* __restrict__ out, JoinCtl* ctl) {
+    __shared__ uint64_t queue[4][WaveQueue::kCap];
+    WaveQueue pairs{queue[threadIdx.x >> 6], &ctl->out, out, cap};
     const int64_t m = min((int64_t)ctl->cand, cap);
     const int lane = threadIdx.x & 63, sub = lane & 7;
     for (int64_t c0 = (int64_t)blockIdx.x * 32; c0 < m; c0 += (int64_t)gridDim.x * 32) {
@@ -123,8 +148,9 @@ __global__ void __launch_bounds__(256) k_join_check(const int8_t* __restrict__ w
         }
         const unsigned long long all = __ballot(ok);
         const bool pass = (all >> (lane & 56) & 255ull) == 255ull;
-        wave_append(&ctl->out, pass && sub == 0, x, out, cap);
+        pairs.push(pass && sub == 0, x);
     }
+    pairs.flush();
 }
 
 JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int64_t na, const int8_t* d_wb,
