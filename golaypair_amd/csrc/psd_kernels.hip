@@ -764,11 +764,17 @@ __global__ void __launch_bounds__(256) k_rows_filter(RowsCall C, RowsTables T, R
 
 void filter_rows(gp_ctx* ctx, const int8_t* words, int stride, const int32_t* lens, const int32_t* orders,
                  const int32_t* pafs, int64_t count, uint8_t* pass, float* max_psd, gp_stats* stats) {
-    if (count > 0x7FFFFFFFll) throw ArgError("gp_psd_filter_batch: more than 2^31 rows");
     uint64_t present = 0;  // bit n - 1: length n
     for (int64_t i = 0; i < count; ++i) {
         if (lens[i] < 2 || lens[i] > kMaxN || lens[i] > stride) throw ArgError("word length out of range");
         present |= 1ull << (lens[i] - 1);
+    }
+    constexpr int64_t kMost = 1 << 30;  // rows of one pass: row numbers are 32 bits
+    if (count > kMost) {
+        for (int64_t i = 0; i < count; i += kMost)
+            filter_rows(ctx, words + i * stride, stride, lens + i, orders + i, pafs + i, std::min(kMost, count - i),
+                        pass + i, max_psd ? max_psd + i : nullptr, stats);
+        return;
     }
     RowsTables T{};
     for (int n = 2; n <= kMaxN; ++n)
