@@ -32,8 +32,9 @@ extern "C" {
 #define GP_ERR_CAPACITY (-3)
 #define GP_ERR_UNSUPPORTED (-4)
 
-/* PSD filter arithmetic: split-BF16 MFMA contraction (FP32 accumulate, FP64
- * recheck inside the error band) or the plain FP32 direct DFT on the vector ALUs.
+/* PSD filter arithmetic: matrix products of 16-bit parts (split BF16 in gen and the
+ * row filters, f16 parts in uncompression; FP32 accumulate, FP64 recheck inside the
+ * error band) or the plain FP32 direct DFT on the vector ALUs.
  * Both give identical decisions and keys. */
 #define GP_PSD_SPLIT_BF16 0
 #define GP_PSD_FP32 1
@@ -66,7 +67,7 @@ typedef struct gp_stats {
     uint64_t words;          /* words enumerated / leaves expanded              */
     uint64_t psd_decisions;  /* PSD filter decisions made                       */
     uint64_t psd_pass;       /* decisions that accepted                         */
-    uint64_t band_rechecks;  /* split-BF16 decisions settled in FP64            */
+    uint64_t band_rechecks;  /* decisions inside the error band, settled in FP64 */
     uint64_t key_rechecks;   /* keys whose rint was settled in FP64             */
     uint64_t canonical;      /* words kept by the canonical check               */
     uint64_t pair_checks;    /* exact integer PAF checks run                    */
