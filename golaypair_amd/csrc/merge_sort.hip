@@ -1,6 +1,8 @@
 // Merge sort of records by a first key word (uint64) and, where two first words
 // are equal, by `nrest` further words per record and then by record number.
 //   k_ms_block  runs of one tile of records, sorted in LDS
+//   k_ms_rank   places of all records of some runs at once (up to 2^16 records, or
+//               2^18 without further words), k_ms_place moves them there
 //   k_ms_merge  one round of pairwise merges: a block makes one tile of
 //               consecutive records of the output
 // What moves is the first word and the record number (12 bytes, read and written
@@ -11,7 +13,8 @@
 // which 19 bytes vary in the records of order 45, 3 -> 1 (19 passes of 5 launches
 // each), while the first 64 bits tell nearly all records apart, and a level's
 // files hold 1e4 .. 1e5 records, where the number of launches is the time: 1 + 6
-// launches and 0.12 ms for 6e4 records against 95 launches and 0.74 ms.  The rounds
+// launches and 0.12 ms for 6e4 records against 95 launches and 0.74 ms (1 + 4 with
+// k_ms_rank).  The rounds
 // grow with the logarithm of the records, so a large sort gains as well: 0.45 ms
 // for 4e6 records against 1.4 ms.  A round is bound by its chain of dependent
 // reads (the split of the two runs, the merge in LDS), at 4e6 records by memory.
@@ -28,6 +31,18 @@ constexpr int kMsThreads = 256;
 // other: a round of 6e4 records takes 15 us with 4 and 21 us with 8.  The larger
 // tile saves a round where a round is bound by memory.
 constexpr int64_t kMsSmall = 1 << 18;
+// Rounds over runs of a few tiles are one step (k_ms_rank, k_ms_place): each record's
+// place among `ms_rank_runs` runs, all searched at once, two per block.  A record is
+// searched in every run where a round of merges passes it once, but the searches do
+// not wait for each other.  Calls of gp_sort_candidates on random records of n = 15,
+// merges against ranks of 32 runs: 18 000 records 190 and 159 us, 32 768 216 and 187;
+// 61 000 283 and 250, and with 16 runs and the rounds over those 257.  Where all first
+// words are equal each search reads further words: 32 768 records 331 and 302 us, but
+// 61 000 408 and 469 (32 runs) or 405 (16 runs), 100 000 553 and 619 (16 runs).  Without
+// further words an equal first word costs nothing more.
+__host__ __device__ constexpr int64_t ms_rank_runs(int64_t n, bool rest) {
+    return !rest || n <= 1 << 15 ? 32 : n <= 1 << 16 ? 16 : 0;
+}
 constexpr uint32_t kMsNone = 0xFFFFFFFFu;  // a place past the last record: after every record
 
 struct MsRec {
@@ -230,16 +245,109 @@ __global__ void __launch_bounds__(kMsThreads) k_ms_merge(const uint64_t* __restr
     }
 }
 
+// Places of the records of a tile (blockIdx.x) in the sort of all tiles, as far as
+// the runs blockIdx.y, blockIdx.y + gridDim.y, ... decide them: how many of their
+// records come before each, into part[blockIdx.y][record].  A run is searched in
+// LDS, by first words; the records of a first word that the run has too are
+// searched by all words.  The next run's loads are in flight during the search.
+template <bool REST, int I>
+__global__ void __launch_bounds__(kMsThreads) k_ms_rank(const uint64_t* __restrict__ kin,
+                                                        const uint32_t* __restrict__ iin, int64_t n,
+                                                        const uint64_t* __restrict__ rest, int nrest,
+                                                        int runs, uint32_t* __restrict__ part) {
+    constexpr int kTile = kMsThreads * I;
+    __shared__ uint64_t sk[kTile];
+    __shared__ uint32_t si[kTile];
+    const int t = threadIdx.x, own = blockIdx.x, seg = own / runs * runs, run0 = seg + blockIdx.y;
+    const int tiles = min((int)((n + kTile - 1) / kTile), seg + runs);
+    MsRec r[I], next[I];
+    uint32_t place[I] = {};
+    auto load = [&](int tile, MsRec (&v)[I]) {
+#pragma unroll
+        for (int j = 0; j < I; ++j) {
+            const int64_t x = (int64_t)tile * kTile + j * kMsThreads + t;
+            v[j] = x < n ? MsRec{kin[x], iin[x]} : MsRec{~0ull, kMsNone};
+        }
+    };
+    load(own, r);
+    load(run0, next);
+    for (int run = run0; run < tiles; run += gridDim.y) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < I; ++j) {
+            sk[j * kMsThreads + t] = next[j].k;
+            si[j * kMsThreads + t] = next[j].i;
+        }
+        __syncthreads();
+        if (run + (int)gridDim.y < tiles) load(run + gridDim.y, next);
+        if (run == own) {
+#pragma unroll
+            for (int j = 0; j < I; ++j) place[j] += j * kMsThreads + t;
+            continue;
+        }
+        const int len = (int)min<int64_t>(kTile, n - (int64_t)run * kTile);
+        int lo[I] = {};
+#pragma unroll
+        for (int step = kTile / 2; step; step /= 2)
+#pragma unroll
+            for (int j = 0; j < I; ++j)
+                if (sk[lo[j] + step - 1] < r[j].k) lo[j] += step;
+#pragma unroll
+        for (int j = 0; j < I; ++j) {
+            if (sk[lo[j]] < r[j].k) ++lo[j];
+            int a = lo[j];
+            if (a < len && sk[a] == r[j].k && r[j].i != kMsNone) {
+                int b = len;
+                while (a < b) {  // records after a of a larger first word compare as such
+                    const int mid = (a + b) >> 1;
+                    if (ms_less<REST>(MsRec{sk[mid], si[mid]}, r[j], rest, nrest)) a = mid + 1;
+                    else b = mid;
+                }
+            }
+            place[j] += (uint32_t)a;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < I; ++j) {
+        const int64_t x = (int64_t)own * kTile + j * kMsThreads + t;
+        if (x < n) part[(int64_t)blockIdx.y * n + x] = place[j];
+    }
+}
+
+__global__ void k_ms_place(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ iin, int64_t n,
+                           const uint32_t* __restrict__ part, int groups, int64_t seg, uint64_t* __restrict__ kout,
+                           uint32_t* __restrict__ iout) {
+    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x >= n) return;
+    int64_t at = x / seg * seg;
+#pragma unroll 8
+    for (int g = 0; g < groups; ++g) at += part[(int64_t)g * n + x];
+    kout[at] = kin[x];
+    iout[at] = iin[x];
+}
+
 namespace {
 
 template <bool REST, int I>
 MergeSorted run_merge_sort(hipStream_t st, const uint64_t* keys, int64_t n, const uint64_t* rest, int nrest,
-                           uint64_t* const (&kb)[2], uint32_t* const (&ib)[2]) {
+                           uint64_t* const (&kb)[2], uint32_t* const (&ib)[2], uint32_t* part) {
     constexpr int64_t kTile = kMsThreads * I;
     const dim3 grid((unsigned)((n + kTile - 1) / kTile));
     hipLaunchKernelGGL((k_ms_block<REST, I>), grid, dim3(kMsThreads), 0, st, keys, n, rest, nrest, kb[0], ib[0]);
     int at = 0;
-    for (int64_t run = kTile; run < n; run *= 2, at ^= 1)
+    int64_t run = kTile;
+    if constexpr (I == 4) {
+        if (part) {
+            const int runs = (int)ms_rank_runs(n, REST);
+            hipLaunchKernelGGL((k_ms_rank<REST, I>), dim3(grid.x, runs / 2), dim3(kMsThreads), 0, st, kb[0], ib[0], n, rest,
+                               nrest, runs, part);
+            run *= runs;
+            hipLaunchKernelGGL(k_ms_place, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, kb[0], ib[0], n, part,
+                               runs / 2, run, kb[1], ib[1]);
+            at = 1;
+        }
+    }
+    for (; run < n; run *= 2, at ^= 1)
         hipLaunchKernelGGL((k_ms_merge<REST, I>), grid, dim3(kMsThreads), 0, st, kb[at], ib[at], n, run, rest, nrest,
                            kb[at ^ 1], ib[at ^ 1]);
     GP_HIP(hipGetLastError());
@@ -254,11 +362,13 @@ MergeSorted merge_sort(gp_ctx* ctx, const std::string& name, const uint64_t* key
     if (n <= 0) return MergeSorted{nullptr, nullptr};
     uint64_t* const kb[2] = {ctx->dev<uint64_t>(name + ".k0", (size_t)n), ctx->dev<uint64_t>(name + ".k1", (size_t)n)};
     uint32_t* const ib[2] = {ctx->dev<uint32_t>(name + ".i0", (size_t)n), ctx->dev<uint32_t>(name + ".i1", (size_t)n)};
+    const int64_t runs = n > 2 * kMsThreads * 4 && n <= kMsSmall ? ms_rank_runs(n, nrest > 0) : 0;  // two tiles: a merge
+    uint32_t* const part = runs ? ctx->dev<uint32_t>(name + ".rank", (size_t)(n * runs / 2)) : nullptr;
     if (n <= kMsSmall)
-        return nrest > 0 ? run_merge_sort<true, 4>(ctx->stream, keys, n, rest, nrest, kb, ib)
-                         : run_merge_sort<false, 4>(ctx->stream, keys, n, rest, nrest, kb, ib);
-    return nrest > 0 ? run_merge_sort<true, 8>(ctx->stream, keys, n, rest, nrest, kb, ib)
-                     : run_merge_sort<false, 8>(ctx->stream, keys, n, rest, nrest, kb, ib);
+        return nrest > 0 ? run_merge_sort<true, 4>(ctx->stream, keys, n, rest, nrest, kb, ib, part)
+                         : run_merge_sort<false, 4>(ctx->stream, keys, n, rest, nrest, kb, ib, part);
+    return nrest > 0 ? run_merge_sort<true, 8>(ctx->stream, keys, n, rest, nrest, kb, ib, part)
+                     : run_merge_sort<false, 8>(ctx->stream, keys, n, rest, nrest, kb, ib, part);
 }
 
 }  // namespace gp

@@ -84,3 +84,12 @@ def test_sort_runs_and_ties(gpu_ctx, m, key_values):
     rng = np.random.default_rng(m)
     c = _random_records(rng, m, 15, [-3, -1, 1, 3], key_values)
     assert gpu_ctx.sort_candidates(c).lines() == sorted(set(c.lines()))
+
+
+@pytest.mark.parametrize("m", [2050, 3073, 32768, 32769, 49153, 65536, 65537])
+@pytest.mark.parametrize("key_values", [[7], list(range(0, 93))])
+def test_sort_ranked_runs(gpu_ctx, m, key_values):
+    """Record counts around the sizes up to which runs are ranked all at once (2^15:
+    32 runs of 1024; 2^16: 16 runs and merges), with distinct and equal first words."""
+    c = _random_records(np.random.default_rng(m), m, 15, [-3, -1, 1, 3], key_values)
+    assert gpu_ctx.sort_candidates(c).lines() == sorted(set(c.lines()))
