@@ -332,3 +332,32 @@ def test_uncompress_after_large_copies(gpu_ctx, monkeypatch):
         gpu_ctx.psd_keys(words, 255, False)  # 17 MB up, 8.8 MB back
         oa, ob, _, _, _ = gpu_ctx.uncompress(order, 2, 1, paf, pa, pb)
         assert "".join(g.pair_line(x, y) + "\n" for x, y in zip(oa, ob)) == want
+
+
+def _golay(n):
+    """An aperiodic Golay pair of length 2^k or 10 * 2^k, by doubling."""
+    a, b = (np.array([1, 1, -1, 1, -1, 1, -1, -1, 1, 1]), np.array([1, 1, -1, 1, 1, 1, 1, 1, -1, -1])) if n % 5 == 0 \
+        else (np.array([1]), np.array([1]))
+    while len(a) < n:
+        a, b = np.concatenate([a, b]), np.concatenate([a, -b])
+    return a.astype(np.int8), b.astype(np.int8)
+
+
+@pytest.mark.parametrize("n", [4, 8, 10, 16, 20, 32, 40, 64])
+def test_uncompress_pairs_of_known_words(gpu_ctx, n):
+    """Words of 2 to 32 PAF values (the re-match takes them eight at a time): the pairs
+    that the re-match finds are those of the two sides' words whose PAFs sum to zero."""
+    a, b = _golay(n)
+    pa, pb = (w.reshape(2, n // 2).sum(0, dtype=np.int8)[None] for w in (a, b))
+    oa, ob, _, _, _ = gpu_ctx.uncompress(n, 2, 1, 0, pa, pb)
+    sides = []
+    for flag, seq in ((0, pa[0]), (1, pb[0])):
+        w = gpu_ctx.uncompress_side(seq, 2, 1, 0, flag)[0].words.astype(np.int32)
+        sides.append((w, np.stack([(w * np.roll(w, s, axis=1)).sum(1) for s in range(1, n // 2 + 1)], 1)))
+    by_paf = {}
+    for w, p in zip(*sides[1]):
+        by_paf.setdefault(tuple(-p), []).append(tuple(w))
+    want = {(tuple(w), x) for w, p in zip(*sides[0]) for x in by_paf.get(tuple(p), [])}
+    assert len(want) > 0
+    assert {(tuple(map(int, x)), tuple(map(int, y))) for x, y in zip(oa, ob)} == \
+        {(tuple(map(int, x)), tuple(map(int, y))) for x, y in want}
