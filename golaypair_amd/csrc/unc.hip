@@ -1319,23 +1319,20 @@ void batch_header(const UncPrep& U, UncBatch& B) {
 int64_t surv_cap(uint64_t leaves) { return (int64_t)std::min<uint64_t>(leaves * 3 / 5 + (1 << 20), (uint64_t)3 << 30); }
 int64_t band_cap(uint64_t leaves) { return (int64_t)std::min<uint64_t>(leaves / 64 + (1 << 16), (uint64_t)1 << 28); }
 
-// Uploads the staged tables into the device buffer `name` (one copy: on the
-// context's stream, or, with `uploaded`, on the copy stream, which the
-// context's stream then waits for, so that the copy overlaps earlier kernels),
-// points B's table fields there and returns the filter kernels' view of them.
+// Uploads the staged tables into the device buffer `name` (one copy, on the copy
+// stream, which the context's stream then waits for, so that it overlaps earlier
+// kernels), points B's table fields there and returns the filter kernels' view of
+// them.  The staging buffer's event is recorded on the copy stream alone: a thread
+// that takes the buffer for a later batch waits for that event, and a wait for an
+// event of the context's stream while a batch is captured there ends the capture.
 UncTabs upload_tables(gp_ctx* ctx, UncPrep& U, const std::string& name, UncBatch& B, const int64_t** d_toff,
-                      hipEvent_t uploaded = nullptr) {
+                      hipEvent_t uploaded) {
     unc_stage(U, ctx->pinned);
     char* base = static_cast<char*>(ctx->buf(name).ensure(U.stage_bytes));
-    if (uploaded) {
-        GP_HIP(hipMemcpyAsync(base, U.base, U.stage_bytes, hipMemcpyHostToDevice, ctx->copy_stream));
-        GP_HIP(hipEventRecord(uploaded, ctx->copy_stream));
-        GP_HIP(hipStreamWaitEvent(ctx->stream, uploaded, 0));
-        if (U.stage) U.stage->record_upload(ctx->copy_stream);
-    } else {
-        GP_HIP(hipMemcpyAsync(base, U.base, U.stage_bytes, hipMemcpyHostToDevice, ctx->stream));
-        if (U.stage) U.stage->record_upload(ctx->stream);
-    }
+    GP_HIP(hipMemcpyAsync(base, U.base, U.stage_bytes, hipMemcpyHostToDevice, ctx->copy_stream));
+    GP_HIP(hipEventRecord(uploaded, ctx->copy_stream));
+    GP_HIP(hipStreamWaitEvent(ctx->stream, uploaded, 0));
+    if (U.stage) U.stage->record_upload(ctx->copy_stream);
     auto at = [&](int i) { return static_cast<void*>(base + U.stage_off[i]); };
     B.d_sides = static_cast<const UncSide*>(at(kStSides));
     B.d_radix = static_cast<const int32_t*>(at(kStRadix));
@@ -1428,7 +1425,10 @@ UncBatch unc_launch(gp_ctx* ctx, UncPrep& U, gp_stats* stats) {
     if (U.T.nsides == 0) return B;
     Phase ph2("unc_filter: upload");
     const int64_t* d_toff = nullptr;
-    const UncTabs tb = upload_tables(ctx, U, "u_stage", B, &d_toff);
+    // the copy comes after what a call before this one left on the stream
+    GP_HIP(hipEventRecord(ctx->ev3, st));
+    GP_HIP(hipStreamWaitEvent(ctx->copy_stream, ctx->ev3, 0));
+    const UncTabs tb = upload_tables(ctx, U, "u_stage", B, &d_toff, ctx->slot_ev[0][4]);
     UncCtl* ctl = ctx->dev<UncCtl>("u_ctl", 1);
     int64_t scap = surv_cap(U.total_leaves);
     int64_t bcap = band_cap(U.total_leaves);

@@ -361,3 +361,21 @@ def test_uncompress_pairs_of_known_words(gpu_ctx, n):
     assert len(want) > 0
     assert {(tuple(map(int, x)), tuple(map(int, y))) for x, y in zip(oa, ob)} == \
         {(tuple(map(int, x)), tuple(map(int, y))) for x, y in want}
+
+
+@pytest.mark.parametrize("pairs,batch_leaves", [(4000, 1 << 22)])
+def test_uncompress_reruns_beside_graph_captures(gpu_ctx, monkeypatch, pairs, batch_leaves):
+    """A threshold that nearly every leaf passes: the survivor list of each batch
+    overflows and its filter runs again on the synchronous path, while threads take
+    staging memory for later batches and the next batch's re-match is captured."""
+    a, b, _ = gpu_ctx.generate(45, 3, -2)
+    _, pa, pb, _ = gpu_ctx.match(45, 3, -2, gpu_ctx.sort_candidates(a), gpu_ctx.sort_candidates(b))
+    monkeypatch.setenv("GOLAY_UNC_BATCH_LEAVES", str(batch_leaves))
+    monkeypatch.setenv("GOLAY_UNC_GRAPH", "0")
+    want = gpu_ctx.uncompress(45, 3, 1, -165, pa[:pairs], pb[:pairs])
+    assert want[4].psd_pass > 0.9 * want[4].psd_decisions
+    monkeypatch.setenv("GOLAY_UNC_GRAPH", "1")
+    for _ in range(4):
+        got = gpu_ctx.uncompress(45, 3, 1, -165, pa[:pairs], pb[:pairs])
+        assert (got[0] == want[0]).all() and (got[1] == want[1]).all()
+        assert got[4].psd_pass == want[4].psd_pass
