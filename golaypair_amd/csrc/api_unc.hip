@@ -26,7 +26,8 @@ namespace {
 
 // Leaves per device batch.  A batch costs about 0.2 ms besides its filter (the
 // re-match kernels and their gaps): order 50, 401 pairs, 2^30, 2^31, 2^32 leaves take
-// 81.0, 75.5, 73.0 ms, with 5, 10, 20 GB of survivor space in each of two slots.
+// 81.0, 75.5, 73.0 ms.  Two batches are in flight, each with at most 5.2 GB of survivor
+// space, 2.1 GB of join partitions and 0.3 GB for the band list.
 constexpr uint64_t kLeafBudget = 1ull << 31;
 
 }  // namespace

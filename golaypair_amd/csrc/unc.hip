@@ -1317,6 +1317,16 @@ void batch_header(const UncPrep& U, UncBatch& B) {
 
 // Survivor and band list capacities for a batch of `leaves` leaves.
 int64_t surv_cap(uint64_t leaves) { return (int64_t)std::min<uint64_t>(leaves * 3 / 5 + (1 << 20), (uint64_t)3 << 30); }
+// The same for a batch in flight, at most what 2^30 leaves get (5.2 GB in each of two
+// slots): of a full batch of 2^31 leaves 0.17 % survive at order 50, and one of which
+// more than 30 % do has its filter run again with the room that it needs.
+int64_t slot_surv_cap(uint64_t leaves) { return surv_cap(std::min<uint64_t>(leaves, (uint64_t)1 << 30)); }
+// Survivors that a batch in flight joins: 2^26 and so 2^17 partitions (2.1 GB) for a
+// full batch; one with more is joined again on the synchronous path.
+int64_t slot_join_cap(uint64_t leaves) {
+    const uint64_t rows = leaves / 32, full = (uint64_t)1 << 26;
+    return (int64_t)(rows >= full ? rows : std::min<uint64_t>(rows + (1 << 20), full));
+}
 int64_t band_cap(uint64_t leaves) { return (int64_t)std::min<uint64_t>(leaves / 64 + (1 << 16), (uint64_t)1 << 28); }
 
 // Uploads the staged tables into the device buffer `name` (one copy, on the copy
@@ -1553,7 +1563,7 @@ std::shared_ptr<UncInflight> unc_enqueue(gp_ctx* ctx, std::shared_ptr<UncPrep> p
     const std::string sfx = "#" + std::to_string(slot);
     const int64_t* d_toff = nullptr;
     const UncTabs tb = upload_tables(ctx, U, "u_stage" + sfx, B, &d_toff, ev[4]);
-    F->scap = surv_cap(U.total_leaves);
+    F->scap = slot_surv_cap(U.total_leaves);
     F->bcap = band_cap(U.total_leaves);
     F->ctl = ctx->dev<UncCtl>("u_ctl" + sfx, 1);
     uint64_t* d_surv = ctx->dev<uint64_t>("u_surv" + sfx, (size_t)F->scap);
@@ -1566,7 +1576,7 @@ std::shared_ptr<UncInflight> unc_enqueue(gp_ctx* ctx, std::shared_ptr<UncPrep> p
     // join over at most rcap survivors (the batch is joined again synchronously
     // when more survive); the part of the table in use is sized on the device
     // from the B rows counted by k_unc_rows and stays at most half full
-    F->rcap = std::min<int64_t>(F->scap, (int64_t)(U.total_leaves / 32) + (1 << 20));
+    F->rcap = std::min(F->scap, slot_join_cap(U.total_leaves));
     int64_t pmax = 64;
     while (pmax * 512 < F->rcap) pmax <<= 1;
     const int q_target = B.bound + paf_target;

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import golaypair_amd as g
-from tests import _oracle
+from tests import _device, _oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -379,3 +379,13 @@ def test_uncompress_reruns_beside_graph_captures(gpu_ctx, monkeypatch, pairs, ba
         got = gpu_ctx.uncompress(45, 3, 1, -165, pa[:pairs], pb[:pairs])
         assert (got[0] == want[0]).all() and (got[1] == want[1]).all()
         assert got[4].psd_pass == want[4].psd_pass
+
+
+def test_uncompress_device_memory(gpu_ctx):
+    """A call of several full batches (order 50, 5 -> 1: 2e10 leaves) keeps its device
+    memory within 17 GB."""
+    a, b, _ = gpu_ctx.generate(50, 5, 0)
+    _, pa, pb, _ = gpu_ctx.match(50, 5, 0, gpu_ctx.sort_candidates(a), gpu_ctx.sort_candidates(b))
+    out, held = _device.held_by(lambda ctx: ctx.uncompress(50, 5, 1, 0, pa[:100], pb[:100]))
+    assert out[4].psd_decisions > 1.5e10
+    assert held < 17e9
