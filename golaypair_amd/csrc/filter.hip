@@ -480,7 +480,7 @@ int filter_pairs(gp_ctx* ctx, int order, int compress, const gp_pairs& in, PairS
     out.a.clear();
     out.b.clear();
     if (in.count < 0 || (in.count > 0 && (!in.a || !in.b))) throw ArgError("bad pair set");
-    const int64_t m = in.count;
+    const int64_t m = in.n == 0 ? 0 : in.count;  // (pairs of no letters: none)
     if (m == 0) return GP_OK;
     if (in.n != n) throw ArgError("filter: pair length != order/compress");
     if (n > kMaxN) throw ArgError("filter: length above 64");

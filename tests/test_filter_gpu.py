@@ -210,3 +210,13 @@ def test_filter_packed_words_and_letters(gpu_ctx, n, compress, letters):
     rows = [rows[q] for q in rng.permutation(len(rows))] + rows[:5]
     oa, ob = _gpu_filter(gpu_ctx, n * compress, compress, np.array([r[0] for r in rows]), np.array([r[1] for r in rows]))
     assert [(tuple(a), tuple(b)) for a, b in zip(oa.tolist(), ob.tolist())] == [tuple(map(tuple, s)) for s in sorted(seen)]
+
+
+@pytest.mark.parametrize("order,compress,n", [(1, 2, 0), (6, 1, 0), (3, 4, 0)])
+def test_filter_pairs_of_no_letters(gpu_ctx, order, compress, n):
+    """Pairs of length 0 hold no records, whatever their count says."""
+    a = np.zeros(8, np.int8)
+    inp = g.GpPairs(n, 3, 3, g.ptr(a, g.ctypes.c_int8), g.ptr(a, g.ctypes.c_int8))
+    out = g.GpPairs(n, 7, 8, g.ptr(a, g.ctypes.c_int8), g.ptr(a, g.ctypes.c_int8))
+    assert gpu_ctx.lib.gp_filter(gpu_ctx.h, order, compress, g.ctypes.byref(inp), g.ctypes.byref(out), None) == g.GP_OK
+    assert out.count == 0
