@@ -484,7 +484,8 @@ int filter_pairs(gp_ctx* ctx, int order, int compress, const gp_pairs& in, PairS
     if (m == 0) return GP_OK;
     if (in.n != n) throw ArgError("filter: pair length != order/compress");
     if (n > kMaxN) throw ArgError("filter: length above 64");
-    if (m > 0x7FFFFFFFll) throw ArgError("filter: more than 2^31 pairs");
+    // (pair numbers are 32 bits, all ones an empty slot)
+    if (m >= (int64_t)kNoPair) throw ArgError("filter: more than 2^32 - 2 pairs");
     FilterParams P{};
     P.n = n;
     P.alt = !(compress > 1 || n % 2 == 1);  // filter.cpp:83-87

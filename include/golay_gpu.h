@@ -158,7 +158,7 @@ int gp_uncompress(gp_ctx* ctx, int order, int compress, int new_compress, int pa
                   gp_stats* stats);
 
 /* Equivalence filter: keep the lexicographically smallest input pair of each
- * class, output in (a, b) lexicographic order.
+ * class, output in (a, b) lexicographic order.  At most 2^32 - 2 pairs.
  * Replaces int cache_filter(int ORDER, int COMPRESS, const std::string& PATH_IN,
  *   const std::string& PATH_OUT) (src/core/filter/filter.h:1,
  *   filter.cpp:18-163). */

@@ -220,3 +220,20 @@ def test_filter_pairs_of_no_letters(gpu_ctx, order, compress, n):
     out = g.GpPairs(n, 7, 8, g.ptr(a, g.ctypes.c_int8), g.ptr(a, g.ctypes.c_int8))
     assert gpu_ctx.lib.gp_filter(gpu_ctx.h, order, compress, g.ctypes.byref(inp), g.ctypes.byref(out), None) == g.GP_OK
     assert out.count == 0
+
+
+def test_filter_more_than_2_31_pairs(gpu_ctx):
+    """2^31 + 5 pairs of one letter: their classes are those of the letters."""
+    m = (1 << 31) + 5
+    a = np.ones(m, np.int8)
+    a[-1] = -1
+    a[-3] = 3
+    oa, ob = np.zeros((8, 1), np.int8), np.zeros((8, 1), np.int8)
+    inp = g.GpPairs(1, m, m, g.ptr(a, g.ctypes.c_int8), g.ptr(a, g.ctypes.c_int8))
+    out = g.GpPairs(1, 0, 8, g.ptr(oa, g.ctypes.c_int8), g.ptr(ob, g.ctypes.c_int8))
+    ctx = g.Context(0)  # its buffers go with it
+    try:
+        ctx.check(ctx.lib.gp_filter(ctx.h, 1, 1, g.ctypes.byref(inp), g.ctypes.byref(out), None), "gp_filter")
+    finally:
+        ctx.close()
+    assert oa[:out.count, 0].tolist() == [-1, 1, 3] and ob[:out.count, 0].tolist() == [-1, 1, 3]
