@@ -9,8 +9,8 @@
 // digit strings of tuples that differ by a nonzero constant shift cannot be
 // equal (the first component keeps or changes its decimal length, and either
 // way the strings differ).  The join therefore hashes the key tuples:
-//   k_join_insert  B records into chains of a hash table
-//   k_join_probe   for every A its slot's chain: equal hash, then equal tuple
+//   k_join_insert  B records into a hash table, a chain per key
+//   k_join_probe   for every A its key's chain: equal tuples
 //   k_join_check   the integer PAF condition of the candidate pairs
 // and the accepted pairs are sorted into the reference's emission order.
 // Bound by launches and the copies of the four input buffers.  The files of order
@@ -34,16 +34,46 @@ __device__ __forceinline__ uint64_t key_hash(const uint8_t* __restrict__ k, int 
     return h;
 }
 
-constexpr uint32_t kJoinEnd = 0xFFFFFFFFu;
+// A slot of the hash table: the tag of the keys it holds (0: free) and the first of
+// their B records, numbered from 1 (0: none).  Records of one key are chained in one
+// slot, others in the slots after it, so that an A record walks the records of its own
+// key only (tags that collide apart): chains of all that share a slot index made 2e5 A
+// records beside 1e5 B records of one other key take 21 ms, the longest chain's walk.
+struct JoinSlot {
+    uint32_t tag, head;
+};
 
-// B record i in front of the chain of its slot (head: kJoinEnd where empty).
+__device__ __forceinline__ uint32_t join_tag(uint64_t h) { return (uint32_t)(h >> 32) | 1u; }
+
+// The slot of a key of hash h, or a free one where the table lacks it.
+__device__ __forceinline__ uint64_t join_find(const JoinSlot* __restrict__ slot, uint64_t mask, uint64_t h) {
+    uint64_t s = h & mask;
+    for (uint32_t t; (t = slot[s].tag) != 0 && t != join_tag(h);) s = (s + 1) & mask;
+    return s;
+}
+
+// B record i in front of the chain of its key.  Of the lanes with the hash of the
+// wave's first one, which link up among themselves, that one alone goes to the table
+// (atomics on one address are applied one at a time).
 __global__ void k_join_insert(const uint8_t* __restrict__ keys, int64_t m, int nkey, int kstride,
-                              uint64_t* __restrict__ hash, uint32_t* __restrict__ next, uint32_t* head,
-                              uint32_t mask) {
+                              uint32_t* __restrict__ next, JoinSlot* slot, uint64_t mask) {
+    const int lane = threadIdx.x & 63;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t h = key_hash(keys + i * kstride, nkey);
-        hash[i] = h;
-        next[i] = atomicExch(&head[(uint32_t)h & mask], (uint32_t)i);
+        const uint64_t h0 = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(h >> 32)) << 32 |
+                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)h);
+        const unsigned long long same = __ballot(h == h0), mine = h == h0 ? same : 1ull << lane;
+        const int first = __ffsll((long long)mine) - 1, last = 63 - __clzll((long long)mine);
+        const unsigned long long after = mine >> lane >> 1;
+        if (after) next[i] = (uint32_t)i + (uint32_t)__ffsll((long long)after) + 1;  // (lanes hold records in a row)
+        if (lane != first) continue;
+        uint64_t s = h & mask;
+        for (;; s = (s + 1) & mask) {  // (the table is at most half full)
+            uint32_t t = __hip_atomic_load(&slot[s].tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (t == 0) t = atomicCAS(&slot[s].tag, 0u, join_tag(h));
+            if (t == 0 || t == join_tag(h)) break;
+        }
+        next[i + last - first] = atomicExch(&slot[s].head, (uint32_t)i + 1);
     }
 }
 
@@ -88,29 +118,21 @@ struct WaveQueue {
 // Candidate pairs A << 32 | B with equal key tuples, one A record per lane.
 __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ ka, int64_t na,
                                                     const uint8_t* __restrict__ kb, int nkey, int kstride,
-                                                    const uint64_t* __restrict__ hash,
                                                     const uint32_t* __restrict__ next,
-                                                    const uint32_t* __restrict__ head, uint32_t mask,
+                                                    const JoinSlot* __restrict__ slot, uint64_t mask,
                                                     uint64_t* __restrict__ cand, int64_t cap, JoinCtl* ctl) {
     __shared__ uint64_t queue[4][WaveQueue::kCap];
     WaveQueue out{queue[threadIdx.x >> 6], &ctl->cand, cand, cap};
     for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < na; i0 += (int64_t)gridDim.x * 256) {
         const int64_t i = i0 + threadIdx.x;
         const uint8_t* k = ka + i * kstride;
-        uint64_t h = 0;
-        uint32_t j = kJoinEnd;
-        if (i < na) {
-            h = key_hash(k, nkey);
-            j = head[(uint32_t)h & mask];
-        }
-        while (__any(j != kJoinEnd)) {
-            bool eq = false;
-            uint32_t at = j;
-            if (j != kJoinEnd) {
-                eq = hash[j] == h;
-                j = next[j];
-            }
+        uint32_t j = 0;
+        if (i < na) j = slot[join_find(slot, mask, key_hash(k, nkey))].head;
+        while (__any(j != 0)) {
+            bool eq = j != 0;
+            const uint32_t at = j - 1;
             if (eq) {
+                j = next[at];
                 const uint8_t* k2 = kb + (int64_t)at * kstride;
                 for (int q = 0; q < nkey && eq; ++q) eq = k[q] == k2[q];
             }
@@ -160,17 +182,16 @@ JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int6
     if (na <= 0 || nb <= 0) return res;
     if (na > 0xFFFFFFFFll || nb > 0xFFFFFFFFll) throw ArgError("join: more than 2^32 candidates");
     hipStream_t st = ctx->stream;
-    uint32_t slots = 64;  // a slot per B record or more
-    while (slots < nb && slots < (1u << 31)) slots <<= 1;
-    uint64_t* hash = ctx->dev<uint64_t>("j_hash", nb);
+    uint64_t slots = 64;  // two slots per B record or more
+    while (slots < 2 * (uint64_t)nb) slots <<= 1;
+    const uint64_t mask = slots - 1;
     uint32_t* next = ctx->dev<uint32_t>("j_next", nb);
-    uint32_t* head = ctx->dev<uint32_t>("j_head", slots);
+    JoinSlot* slot = ctx->dev<JoinSlot>("j_slot", slots);
     JoinCtl* ctl = ctx->dev<JoinCtl>("j_ctl", 1);
     if (stats) GP_HIP(hipEventRecord(ctx->ev2, st));
-    GP_HIP(hipMemsetAsync(head, 0xFF, (size_t)slots * 4, st));
+    GP_HIP(hipMemsetAsync(slot, 0, slots * sizeof(JoinSlot), st));
     const auto blocks = [&](int64_t n_) { return dim3((unsigned)std::min<int64_t>((n_ + 255) / 256, ctx->num_cus * 8)); };
-    hipLaunchKernelGGL(k_join_insert, blocks(nb), dim3(256), 0, st, d_kb, nb, nkey, kstride, hash, next, head,
-                       slots - 1);
+    hipLaunchKernelGGL(k_join_insert, blocks(nb), dim3(256), 0, st, d_kb, nb, nkey, kstride, next, slot, mask);
     GP_HIP(hipGetLastError());
     int64_t cap = std::max<int64_t>(1024, 2 * std::max(na, nb));
     JoinCtl h{};
@@ -179,8 +200,8 @@ JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int6
         uint64_t* cand = ctx->dev<uint64_t>("j_cand", cap);
         out = ctx->dev<uint64_t>("j_out", cap);
         GP_HIP(hipMemsetAsync(ctl, 0, sizeof(JoinCtl), st));
-        hipLaunchKernelGGL(k_join_probe, blocks(na), dim3(256), 0, st, d_ka, na, d_kb, nkey, kstride, hash, next, head,
-                           slots - 1, cand, cap, ctl);
+        hipLaunchKernelGGL(k_join_probe, blocks(na), dim3(256), 0, st, d_ka, na, d_kb, nkey, kstride, next, slot, mask,
+                           cand, cap, ctl);
         hipLaunchKernelGGL(k_join_check, blocks(8 * na), dim3(256), 0, st, d_wa, d_wb, n, wstride, paf_target, cand,
                            cap, out, ctl);
         GP_HIP(hipGetLastError());

@@ -186,3 +186,17 @@ def test_gen_wide_words(gpu_ctx):
     finally:
         gpu_ctx.set_mode(g.GP_PSD_SPLIT_BF16)
     assert len(a) + len(b) > 0 and a.lines() == fa.lines() and b.lines() == fb.lines()
+
+
+def test_match_chain_of_equal_keys_beside_other_records(gpu_ctx):
+    """2^16 B records of one key: A records of other keys do not walk them all."""
+    rng, n, m = np.random.default_rng(3), 16, 1 << 16
+    wa, wb = (rng.choice([-1, 1], size=(m, n)).astype(np.int8) for _ in range(2))
+    ka = rng.integers(0, 256, size=(m, n // 2)).astype(np.uint8)
+    one, other = np.repeat(ka[:1] ^ 255, m, 0), rng.integers(0, 256, size=(m, n // 2)).astype(np.uint8)
+    ms = []
+    for kb in (other, one):
+        runs = [gpu_ctx.match(n, 1, 0, g.Cands(wa, ka), g.Cands(wb, kb))[3] for _ in range(4)]
+        assert all(r.pair_checks == 0 for r in runs)
+        ms.append(min(r.kernel_ms for r in runs[1:]))
+    assert ms[1] < 8 * ms[0]
