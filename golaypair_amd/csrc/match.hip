@@ -12,9 +12,10 @@
 //   k_join_insert  B records into a hash table, a chain per key
 //   k_join_probe   for every A its key's chain: equal tuples
 //   k_join_check   the integer PAF condition of the candidate pairs
+// (or, of many candidates, k_join_slots, k_join_runs, k_join_scan: see there)
 // and the accepted pairs are sorted into the reference's emission order.
 // Bound by launches and the copies of the four input buffers.  The files of order
-// 45, 3 -> 1 (at most 53000 records each) take 237 us, against 767 us with B radix
+// 45, 3 -> 1 (at most 53000 records each) take 225 us, against 767 us with B radix
 // sorted by hash (40 launches) and the pairs sorted on the host.
 #include <algorithm>
 
@@ -85,7 +86,8 @@ struct JoinCtl {
 // Entries that a wave appends to a list (at most cap kept), collected in LDS so that
 // about 200 take one atomic: atomics on one address are applied one at a time, and
 // one per step of a wave made the probe of 2^21 records a side with 2^20 candidates
-// take 1.63 ms instead of 0.20 ms.  Every lane of the wave must call push and flush.
+// take 1.63 ms instead of 0.20 ms.  Every lane of the wave must call push, and every
+// thread of the block finish, which takes one atomic for what the 4 waves still hold.
 struct WaveQueue {
     static constexpr int kCap = 256;
     uint64_t* q;
@@ -93,6 +95,7 @@ struct WaveQueue {
     uint64_t* list;
     int64_t cap;
     int n = 0;
+    bool full = false;  // the list had no room for some of the last entries
     __device__ void push(bool have, uint64_t x) {
         const unsigned long long b = __ballot(have);
         if (have) q[n + __popcll(b & ((1ull << (threadIdx.x & 63)) - 1ull))] = x;
@@ -109,13 +112,38 @@ struct WaveQueue {
         base = __shfl(base, 0);
         for (int x = lane; x < n; x += 64)
             if ((int64_t)(base + x) < cap) list[base + x] = q[x];
+        full = (int64_t)base + n > cap;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
         n = 0;
     }
+    __device__ void finish() {
+        __shared__ int held[4];
+        __shared__ unsigned long long base;
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        if (lane == 0) held[wave] = n;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int sum = held[0] + held[1] + held[2] + held[3];
+            base = sum ? atomicAdd(count, (unsigned long long)sum) : 0ull;
+        }
+        __syncthreads();
+        unsigned long long at = base;
+        for (int w = 0; w < wave; ++w) at += (unsigned long long)held[w];
+        for (int x = lane; x < n; x += 64)
+            if ((int64_t)(at + x) < cap) list[at + x] = q[x];
+        n = 0;
+    }
 };
 
-// Candidate pairs A << 32 | B with equal key tuples, one A record per lane.
+__device__ __forceinline__ bool same_keys(const uint8_t* __restrict__ x, const uint8_t* __restrict__ y, int nkey) {
+    uint32_t d = 0;
+    for (int q = 0; q < nkey; ++q) d |= x[q] ^ y[q];  // (a loop that ends early waits for each byte)
+    return d == 0;
+}
+
+// Candidate pairs A << 32 | B with equal key tuples, one A record per lane.  A wave
+// that finds the list full stops: ctl->cand is above cap then.
 __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ ka, int64_t na,
                                                     const uint8_t* __restrict__ kb, int nkey, int kstride,
                                                     const uint32_t* __restrict__ next,
@@ -123,23 +151,22 @@ __global__ void __launch_bounds__(256) k_join_probe(const uint8_t* __restrict__ 
                                                     uint64_t* __restrict__ cand, int64_t cap, JoinCtl* ctl) {
     __shared__ uint64_t queue[4][WaveQueue::kCap];
     WaveQueue out{queue[threadIdx.x >> 6], &ctl->cand, cand, cap};
-    for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < na; i0 += (int64_t)gridDim.x * 256) {
+    for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < na && !out.full; i0 += (int64_t)gridDim.x * 256) {
         const int64_t i = i0 + threadIdx.x;
         const uint8_t* k = ka + i * kstride;
         uint32_t j = 0;
         if (i < na) j = slot[join_find(slot, mask, key_hash(k, nkey))].head;
-        while (__any(j != 0)) {
+        while (__any(j != 0) && !out.full) {
             bool eq = j != 0;
             const uint32_t at = j - 1;
             if (eq) {
                 j = next[at];
-                const uint8_t* k2 = kb + (int64_t)at * kstride;
-                for (int q = 0; q < nkey && eq; ++q) eq = k[q] == k2[q];
+                eq = same_keys(k, kb + (int64_t)at * kstride, nkey);
             }
             out.push(eq, (uint64_t)i << 32 | at);
         }
     }
-    out.flush();
+    out.finish();
 }
 
 // The PAF condition of each candidate by 8 lanes, which take the shifts in turn
@@ -172,7 +199,76 @@ __global__ void __launch_bounds__(256) k_join_check(const int8_t* __restrict__ w
         const bool pass = (all >> (lane & 56) & 255ull) == 255ull;
         pairs.push(pass && sub == 0, x);
     }
-    pairs.flush();
+    pairs.finish();
+}
+
+// Where there are more candidates than the list holds (a few per record), none are
+// listed: the B records are sorted by slot, and a wave checks an A record's run of them,
+// one per lane.  3000 records of one key on either side: 0.59 ms, against 13.3 ms with a
+// list of all 9e6 candidates, made in a second walk of the chains.
+__global__ void k_join_slots(const uint8_t* __restrict__ keys, int64_t m, int nkey, int kstride,
+                             const JoinSlot* __restrict__ slot, uint64_t mask, uint64_t* __restrict__ at) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x)
+        at[i] = join_find(slot, mask, key_hash(keys + i * kstride, nkey));
+}
+
+// A slot's run of the sorted records: its first place, from 1, as the slot's head, and
+// the place after its last as `next` of the first.
+__global__ void k_join_runs(const uint64_t* __restrict__ at, int64_t m, uint32_t* __restrict__ next,
+                            JoinSlot* __restrict__ slot) {
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < m; p += (int64_t)gridDim.x * blockDim.x)
+        if (p == 0 || at[p - 1] != at[p]) {
+            slot[at[p]].head = (uint32_t)p + 1;
+            int64_t lo = p + 1, hi = m;
+            while (lo < hi) {
+                const int64_t mid = (lo + hi) >> 1;
+                if (at[mid] > at[p]) hi = mid;
+                else lo = mid + 1;
+            }
+            next[p] = (uint32_t)lo;
+        }
+}
+
+__global__ void __launch_bounds__(256) k_join_scan(const int8_t* __restrict__ wa, const uint8_t* __restrict__ ka,
+                                                   int64_t na, const int8_t* __restrict__ wb,
+                                                   const uint8_t* __restrict__ kb, int n, int nkey, int wstride,
+                                                   int kstride, int target, const uint32_t* __restrict__ idx,
+                                                   const uint32_t* __restrict__ next,
+                                                   const JoinSlot* __restrict__ slot, uint64_t mask,
+                                                   uint64_t* __restrict__ out, int64_t cap, JoinCtl* ctl) {
+    __shared__ uint64_t queue[4][WaveQueue::kCap];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    WaveQueue pairs{queue[wave], &ctl->out, out, cap};
+    unsigned long long checks = 0;
+    for (int64_t i = (int64_t)blockIdx.x * 4 + wave; i < na; i += (int64_t)gridDim.x * 4) {
+        const uint8_t* k = ka + i * kstride;
+        const int8_t* a = wa + i * wstride;
+        const uint32_t head = slot[join_find(slot, mask, key_hash(k, nkey))].head;
+        const int64_t end = head ? next[head - 1] : 0;
+        for (int64_t p0 = (int64_t)head - 1; head && p0 < end; p0 += 64) {
+            bool ok = p0 + lane < end;
+            uint32_t j = 0;
+            if (ok) {
+                j = idx[p0 + lane];
+                ok = same_keys(k, kb + (int64_t)j * kstride, nkey);
+            }
+            checks += ok;
+            if (ok) {
+                const int8_t* b = wb + (int64_t)j * wstride;
+                for (int s = 1; s <= n / 2 && ok; ++s) {
+                    int acc = 0, q = s;
+                    for (int p = 0; p < n; ++p) {
+                        acc += (int)a[p] * (int)a[q] + (int)b[p] * (int)b[q];
+                        if (++q == n) q = 0;
+                    }
+                    ok = acc == target;
+                }
+            }
+            pairs.push(ok, (uint64_t)i << 32 | j);
+        }
+    }
+    pairs.finish();
+    block_atomic_add(&ctl->cand, checks);
 }
 
 JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int64_t na, const int8_t* d_wb,
@@ -195,20 +291,33 @@ JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int6
     GP_HIP(hipGetLastError());
     int64_t cap = std::max<int64_t>(1024, 2 * std::max(na, nb));
     JoinCtl h{};
-    uint64_t* out = nullptr;
-    for (int attempt = 0; attempt < 2; ++attempt) {
-        uint64_t* cand = ctx->dev<uint64_t>("j_cand", cap);
-        out = ctx->dev<uint64_t>("j_out", cap);
-        GP_HIP(hipMemsetAsync(ctl, 0, sizeof(JoinCtl), st));
-        hipLaunchKernelGGL(k_join_probe, blocks(na), dim3(256), 0, st, d_ka, na, d_kb, nkey, kstride, next, slot, mask,
-                           cand, cap, ctl);
-        hipLaunchKernelGGL(k_join_check, blocks(8 * na), dim3(256), 0, st, d_wa, d_wb, n, wstride, paf_target, cand,
-                           cap, out, ctl);
+    uint64_t* out = ctx->dev<uint64_t>("j_out", cap);
+    uint64_t* cand = ctx->dev<uint64_t>("j_cand", cap);
+    const auto read = [&]() {
         GP_HIP(hipGetLastError());
         GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
         GP_HIP(hipStreamSynchronize(st));
-        if ((int64_t)h.cand <= cap) break;
-        cap = (int64_t)h.cand;
+    };
+    GP_HIP(hipMemsetAsync(ctl, 0, sizeof(JoinCtl), st));
+    hipLaunchKernelGGL(k_join_probe, blocks(na), dim3(256), 0, st, d_ka, na, d_kb, nkey, kstride, next, slot, mask,
+                       cand, cap, ctl);
+    hipLaunchKernelGGL(k_join_check, blocks(8 * na), dim3(256), 0, st, d_wa, d_wb, n, wstride, paf_target, cand, cap,
+                       out, ctl);
+    read();
+    if ((int64_t)h.cand > cap) {
+        uint64_t* at = ctx->dev<uint64_t>("j_at", nb);
+        hipLaunchKernelGGL(k_join_slots, blocks(nb), dim3(256), 0, st, d_kb, nb, nkey, kstride, slot, mask, at);
+        const MergeSorted s = merge_sort(ctx, "j_runs", at, nb);
+        hipLaunchKernelGGL(k_join_runs, blocks(nb), dim3(256), 0, st, s.key, nb, next, slot);
+        for (int attempt = 0; attempt < 2; ++attempt) {
+            GP_HIP(hipMemsetAsync(ctl, 0, sizeof(JoinCtl), st));
+            hipLaunchKernelGGL(k_join_scan, blocks(64 * na), dim3(256), 0, st, d_wa, d_ka, na, d_wb, d_kb, n, nkey,
+                               wstride, kstride, paf_target, s.idx, next, slot, mask, out, cap, ctl);
+            read();
+            if ((int64_t)h.out <= cap) break;
+            cap = (int64_t)h.out;
+            out = ctx->dev<uint64_t>("j_out", cap);
+        }
     }
     // emission order of the reference: A position outer, B position inner
     std::vector<uint64_t> pairs(h.out);

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import golaypair_amd as g
-from tests import _oracle
+from tests import _device, _oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -200,3 +200,23 @@ def test_match_chain_of_equal_keys_beside_other_records(gpu_ctx):
         assert all(r.pair_checks == 0 for r in runs)
         ms.append(min(r.kernel_ms for r in runs[1:]))
     assert ms[1] < 8 * ms[0]
+
+
+def test_match_many_candidates_few_pairs(gpu_ctx):
+    """20000 x 20000 records of one key: 4e8 candidate pairs are checked without a
+    list of them all."""
+    rng, n, m = np.random.default_rng(4), 12, 20000
+    wa, wb = (rng.choice([-1, 1], size=(m, n)).astype(np.int8) for _ in range(2))
+    k = np.full((m, n // 2), 9, np.uint8)
+    paf = lambda w: np.stack([(w.astype(int) * np.roll(w, -s, axis=1)).sum(1) for s in range(1, n // 2 + 1)], 1)
+    fa, fb = paf(wa), paf(wb)
+    target = 24
+    by = {}
+    for j, f in enumerate(map(tuple, fb)):
+        by.setdefault(f, []).append(j)
+    want = [(i, j) for i in range(m) for j in by.get(tuple(target - fa[i]), [])]
+    assert 0 < len(want) < 100000
+    (rc, pa, pb, st), held = _device.held_by(lambda ctx: ctx.match(n, 1, target, g.Cands(wa, k), g.Cands(wb, k)))
+    assert st.pair_checks == m * m
+    assert (pa == wa[[i for i, _ in want]]).all() and (pb == wb[[j for _, j in want]]).all() and len(pa) == len(want)
+    assert held < 1 << 28
