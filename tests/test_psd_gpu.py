@@ -19,7 +19,7 @@ import numpy as np
 import pytest
 
 import golaypair_amd as g
-from tests import _oracle
+from tests import _device, _oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -219,3 +219,28 @@ def test_microbench_pass_set_equals_oracle(gpu_ctx, name, mode):
         assert acc[k] == ref_pass[kinds == k].sum()
         assert (kinds == k).sum() == mix[k, 4]
     assert st.tie_band == 0
+
+
+@pytest.mark.parametrize("name,mode", MODES)
+@pytest.mark.parametrize("rows,stride", [(1003, 1 << 22), (5000, 129), (5000, 128), (1, 1000)])
+def test_psd_batch_rows_far_apart(name, mode, rows, stride):
+    """Rows at strides on both sides of the one from which they are gathered: the results
+    of rows side by side, and device memory that goes with the rows, not with the bytes
+    between them."""
+    rng = np.random.default_rng(rows + stride)
+    lens = rng.integers(2, 65, rows).astype(np.int32)
+    words = np.zeros((rows, stride), np.int8)  # (pages are touched where the rows are)
+    near = rng.choice([-1, 1], size=(rows, 64)).astype(np.int8)
+    words[:, :64] = near
+    orders, pafs = np.where(lens > 30, 50, lens).astype(np.int32), np.zeros(rows, np.int32)
+    ref, _ = _oracle.psd_filter_batch(near, lens, orders, pafs)
+
+    def both(ctx):
+        ctx.set_mode(mode)
+        return ctx.psd_filter_batch(words, lens, orders, pafs, want_max=True), \
+            ctx.psd_filter_batch(near, lens, orders, pafs, want_max=True)
+
+    ((got, gmax, _), (want, wmax, _)), held = _device.held_by(both)
+    assert (got == ref).all() and (want == ref).all() and (gmax == wmax).all()
+    assert rows == 1 or 0 < ref.sum() < rows
+    assert held < 1 << 28
