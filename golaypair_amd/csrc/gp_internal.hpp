@@ -200,6 +200,7 @@ struct gp_ctx {
     hipGraphExec_t unc_graph[2] = {};   // per batch slot: the band recheck + re-match chain
     std::map<std::string, int64_t> tuning;  // measured launch / batch parameters (tuning.hip)
     uint64_t unc_graph_launches = 0, unc_graph_instantiations = 0;
+    bool sort_ctl_clear = false;  // the sort's control record is zero (sort_cands.hip)
     std::vector<unsigned char> unc_side_buf;  // storage of the uncompress sides (reused across calls)
     int psd_mode = GP_PSD_SPLIT_BF16;
     std::string err;

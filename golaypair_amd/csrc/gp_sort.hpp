@@ -18,10 +18,17 @@ struct MergeSorted {
     const uint64_t* key;
     const uint32_t* idx;
 };
+// Key words of a sort as they turn out on the device: `words` of each record (the
+// first one and the rest), of which all records share those before the last `live`.
+struct MergeShape {
+    uint32_t words, live;
+};
 // Sorts n records on the context's stream by keys[i], then by the nrest words at
-// rest + i * nrest, then by i.
+// rest + i * nrest, then by i.  With `shape` (device memory, words <= nrest + 1) the rest
+// words lie at rest + i * (words - 1), and the shared ones are passed over: the sorted
+// keys are the words that come first after them.
 MergeSorted merge_sort(gp_ctx* ctx, const std::string& name, const uint64_t* keys, int64_t n,
-                       const uint64_t* rest = nullptr, int nrest = 0);
+                       const uint64_t* rest = nullptr, int nrest = 0, const MergeShape* shape = nullptr);
 
 // Sort + uniq of m candidate records (int8 words of n, uint8 keys of K = n/2)
 // held on the device, in the byte order of their text lines; the kept records

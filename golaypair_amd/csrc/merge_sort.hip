@@ -55,17 +55,35 @@ struct MsRec {
 template <int I>
 __device__ __forceinline__ int ms_at(int x) { return x + x / I; }
 
+// The further words, and with `shape` their number and the shared ones among them.
+struct MsRest {
+    const uint64_t* p;
+    int n;
+    const MergeShape* shape;
+    // the first key word after the shared ones, given the very first
+    __device__ uint64_t first(const uint64_t* __restrict__ keys, int64_t x) const {
+        if (!shape) return keys[x];
+        const int words = (int)shape->words, skip = words - (int)shape->live;
+        return skip == 0 ? keys[x] : skip < words ? p[x * (words - 1) + skip - 1] : 0;
+    }
+};
+
 template <bool REST>
-__device__ __forceinline__ bool ms_less(const MsRec& a, const MsRec& b, const uint64_t* __restrict__ rest, int nrest) {
+__device__ __forceinline__ bool ms_less(const MsRec& a, const MsRec& b, const MsRest& rest) {
     if (a.k != b.k) return a.k < b.k;
     if (REST && a.i != kMsNone && b.i != kMsNone) {
-        const uint64_t* x = rest + (int64_t)a.i * nrest;
-        const uint64_t* y = rest + (int64_t)b.i * nrest;
-        for (int w = 0; w < nrest; w += 4) {  // four words at a time: their reads do not wait for each other
+        int n = rest.n, from = 0;
+        if (rest.shape) {  // (read here: most comparisons do not come this far)
+            n = (int)rest.shape->words - 1;
+            from = (int)(rest.shape->words - rest.shape->live);
+        }
+        const uint64_t* x = rest.p + (int64_t)a.i * n;
+        const uint64_t* y = rest.p + (int64_t)b.i * n;
+        for (int w = from; w < n; w += 4) {  // four words at a time: their reads do not wait for each other
             uint64_t u[4], v[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int at = min(w + j, nrest - 1);
+                const int at = min(w + j, n - 1);
                 u[j] = x[at];
                 v[j] = y[at];
             }
@@ -81,14 +99,13 @@ __device__ __forceinline__ bool ms_less(const MsRec& a, const MsRec& b, const ui
 // [b0, b1) (fewer at the end: the others get kMsNone).
 template <bool REST, int I>
 __device__ __forceinline__ void ms_merge_items(const uint64_t* sk, const uint32_t* si, int a0, int a1, int b0, int b1,
-                                               int d, const uint64_t* __restrict__ rest, int nrest,
-                                               MsRec (&out)[I]) {
+                                               int d, const MsRest& rest, MsRec (&out)[I]) {
     auto rec = [&](int x) { return MsRec{sk[ms_at<I>(x)], si[ms_at<I>(x)]}; };
     const int na = a1 - a0, nb = b1 - b0;
     int lo = max(0, d - nb), hi = min(d, na);
     while (lo < hi) {  // records of the first range among the first d
         const int mid = (lo + hi) >> 1;
-        if (!ms_less<REST>(rec(b0 + d - 1 - mid), rec(a0 + mid), rest, nrest)) lo = mid + 1;
+        if (!ms_less<REST>(rec(b0 + d - 1 - mid), rec(a0 + mid), rest)) lo = mid + 1;
         else hi = mid;
     }
     int a = a0 + min(lo, na), b = b0 + min(max(d - lo, 0), nb);
@@ -96,7 +113,7 @@ __device__ __forceinline__ void ms_merge_items(const uint64_t* sk, const uint32_
     MsRec x = a < a1 ? rec(a) : none, y = b < b1 ? rec(b) : none;
 #pragma unroll
     for (int j = 0; j < I; ++j) {
-        const bool first = b >= b1 || (a < a1 && !ms_less<REST>(y, x, rest, nrest));
+        const bool first = b >= b1 || (a < a1 && !ms_less<REST>(y, x, rest));
         out[j] = first ? x : y;
         if (first) {
             ++a;
@@ -110,22 +127,24 @@ __device__ __forceinline__ void ms_merge_items(const uint64_t* sk, const uint32_
 
 template <bool REST, int I>
 __global__ void __launch_bounds__(kMsThreads) k_ms_block(const uint64_t* __restrict__ keys, int64_t n,
-                                                         const uint64_t* __restrict__ rest, int nrest,
-                                                         uint64_t* __restrict__ kout, uint32_t* __restrict__ iout) {
+                                                         const uint64_t* __restrict__ restp, int nrest,
+                                                         const MergeShape* shape, uint64_t* __restrict__ kout,
+                                                         uint32_t* __restrict__ iout) {
     constexpr int kTile = kMsThreads * I;
     __shared__ uint64_t sk[kTile + kMsThreads];
     __shared__ uint32_t si[kTile + kMsThreads];
     const int t = threadIdx.x;
     const int64_t base = (int64_t)blockIdx.x * kTile;
+    const MsRest rest{restp, nrest, shape};
     MsRec r[I];
 #pragma unroll
     for (int j = 0; j < I; ++j) {  // any I records: the loads of a wave are consecutive
         const int64_t x = base + j * kMsThreads + t;
-        r[j] = x < n ? MsRec{keys[x], (uint32_t)x} : MsRec{~0ull, kMsNone};
+        r[j] = x < n ? MsRec{REST ? rest.first(keys, x) : keys[x], (uint32_t)x} : MsRec{~0ull, kMsNone};
     }
     // a thread's records: Batcher's networks of 5 and 19 exchanges
     auto exchange = [&](int x, int y) {
-        if (ms_less<REST>(r[y], r[x], rest, nrest)) {
+        if (ms_less<REST>(r[y], r[x], rest)) {
             const MsRec z = r[x];
             r[x] = r[y];
             r[y] = z;
@@ -152,7 +171,7 @@ __global__ void __launch_bounds__(kMsThreads) k_ms_block(const uint64_t* __restr
         }
         __syncthreads();
         const int o = t * I, a0 = o & ~(2 * run - 1);
-        ms_merge_items<REST, I>(sk, si, a0, a0 + run, a0 + run, a0 + 2 * run, o - a0, rest, nrest, r);
+        ms_merge_items<REST, I>(sk, si, a0, a0 + run, a0 + run, a0 + 2 * run, o - a0, rest, r);
     }
     __syncthreads();
 #pragma unroll
@@ -176,15 +195,15 @@ __global__ void __launch_bounds__(kMsThreads) k_ms_block(const uint64_t* __restr
 // memory find the place in 2^18 records.
 template <bool REST>
 __device__ __forceinline__ int64_t ms_split(const uint64_t* __restrict__ k, const uint32_t* __restrict__ i, int64_t a0,
-                                            int64_t na, int64_t b0, int64_t nb, int64_t d,
-                                            const uint64_t* __restrict__ rest, int nrest, int lane) {
+                                            int64_t na, int64_t b0, int64_t nb, int64_t d, const MsRest& rest,
+                                            int lane) {
     int64_t lo = max<int64_t>(0, d - nb), hi = min(d, na);
     while (lo < hi) {
         const int64_t step = (hi - lo + 63) / 64, at = lo + lane * step;
         bool first = false;  // the record at a0 + at comes before the one at b0 + d - 1 - at
         if (at < hi) {
             const int64_t b = b0 + d - 1 - at;
-            first = !ms_less<REST>(MsRec{k[b], i[b]}, MsRec{k[a0 + at], i[a0 + at]}, rest, nrest);
+            first = !ms_less<REST>(MsRec{k[b], i[b]}, MsRec{k[a0 + at], i[a0 + at]}, rest);
         }
         const int c = __popcll(__ballot(first));  // true for the first places, then false
         if (c == 0) return lo;
@@ -197,19 +216,20 @@ __device__ __forceinline__ int64_t ms_split(const uint64_t* __restrict__ k, cons
 template <bool REST, int I>
 __global__ void __launch_bounds__(kMsThreads) k_ms_merge(const uint64_t* __restrict__ kin,
                                                          const uint32_t* __restrict__ iin, int64_t n, int64_t run,
-                                                         const uint64_t* __restrict__ rest, int nrest,
-                                                         uint64_t* __restrict__ kout, uint32_t* __restrict__ iout) {
+                                                         const uint64_t* __restrict__ restp, int nrest,
+                                                         const MergeShape* shape, uint64_t* __restrict__ kout,
+                                                         uint32_t* __restrict__ iout) {
     constexpr int kTile = kMsThreads * I;
     __shared__ uint64_t sk[kTile + kMsThreads];
     __shared__ uint32_t si[kTile + kMsThreads];
     __shared__ int64_t split[2];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const MsRest rest{restp, nrest, shape};
     const int64_t out0 = (int64_t)blockIdx.x * kTile, base = out0 / (2 * run) * (2 * run);
     const int64_t amax = min(base + run, n), bmax = min(base + 2 * run, n);
     const int64_t d0 = out0 - base, d1 = min(d0 + kTile, bmax - base);
     if (wave < 2) {
-        const int64_t s = ms_split<REST>(kin, iin, base, amax - base, amax, bmax - amax, wave ? d1 : d0, rest, nrest,
-                                         lane);
+        const int64_t s = ms_split<REST>(kin, iin, base, amax - base, amax, bmax - amax, wave ? d1 : d0, rest, lane);
         if (lane == 0) split[wave] = s;
     }
     __syncthreads();
@@ -227,7 +247,7 @@ __global__ void __launch_bounds__(kMsThreads) k_ms_merge(const uint64_t* __restr
     __syncthreads();
     MsRec r[I];
     const int d = min(t * I, total);
-    ms_merge_items<REST, I>(sk, si, 0, na, na, total, d, rest, nrest, r);
+    ms_merge_items<REST, I>(sk, si, 0, na, na, total, d, rest, r);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < I; ++j) {
@@ -253,12 +273,14 @@ __global__ void __launch_bounds__(kMsThreads) k_ms_merge(const uint64_t* __restr
 template <bool REST, int I>
 __global__ void __launch_bounds__(kMsThreads) k_ms_rank(const uint64_t* __restrict__ kin,
                                                         const uint32_t* __restrict__ iin, int64_t n,
-                                                        const uint64_t* __restrict__ rest, int nrest,
-                                                        int runs, uint32_t* __restrict__ part) {
+                                                        const uint64_t* __restrict__ restp, int nrest,
+                                                        const MergeShape* shape, int runs,
+                                                        uint32_t* __restrict__ part) {
     constexpr int kTile = kMsThreads * I;
     __shared__ uint64_t sk[kTile];
     __shared__ uint32_t si[kTile];
     const int t = threadIdx.x, own = blockIdx.x, seg = own / runs * runs, run0 = seg + blockIdx.y;
+    const MsRest rest{restp, nrest, shape};
     const int tiles = min((int)((n + kTile - 1) / kTile), seg + runs);
     MsRec r[I], next[I];
     uint32_t place[I] = {};
@@ -300,7 +322,7 @@ __global__ void __launch_bounds__(kMsThreads) k_ms_rank(const uint64_t* __restri
                 int b = len;
                 while (a < b) {  // records after a of a larger first word compare as such
                     const int mid = (a + b) >> 1;
-                    if (ms_less<REST>(MsRec{sk[mid], si[mid]}, r[j], rest, nrest)) a = mid + 1;
+                    if (ms_less<REST>(MsRec{sk[mid], si[mid]}, r[j], rest)) a = mid + 1;
                     else b = mid;
                 }
             }
@@ -330,17 +352,18 @@ namespace {
 
 template <bool REST, int I>
 MergeSorted run_merge_sort(hipStream_t st, const uint64_t* keys, int64_t n, const uint64_t* rest, int nrest,
-                           uint64_t* const (&kb)[2], uint32_t* const (&ib)[2], uint32_t* part) {
+                           const MergeShape* shape, uint64_t* const (&kb)[2], uint32_t* const (&ib)[2], uint32_t* part) {
     constexpr int64_t kTile = kMsThreads * I;
     const dim3 grid((unsigned)((n + kTile - 1) / kTile));
-    hipLaunchKernelGGL((k_ms_block<REST, I>), grid, dim3(kMsThreads), 0, st, keys, n, rest, nrest, kb[0], ib[0]);
+    hipLaunchKernelGGL((k_ms_block<REST, I>), grid, dim3(kMsThreads), 0, st, keys, n, rest, nrest, shape, kb[0],
+                       ib[0]);
     int at = 0;
     int64_t run = kTile;
     if constexpr (I == 4) {
         if (part) {
             const int runs = (int)ms_rank_runs(n, REST);
             hipLaunchKernelGGL((k_ms_rank<REST, I>), dim3(grid.x, runs / 2), dim3(kMsThreads), 0, st, kb[0], ib[0], n, rest,
-                               nrest, runs, part);
+                               nrest, shape, runs, part);
             run *= runs;
             hipLaunchKernelGGL(k_ms_place, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, kb[0], ib[0], n, part,
                                runs / 2, run, kb[1], ib[1]);
@@ -349,7 +372,7 @@ MergeSorted run_merge_sort(hipStream_t st, const uint64_t* keys, int64_t n, cons
     }
     for (; run < n; run *= 2, at ^= 1)
         hipLaunchKernelGGL((k_ms_merge<REST, I>), grid, dim3(kMsThreads), 0, st, kb[at], ib[at], n, run, rest, nrest,
-                           kb[at ^ 1], ib[at ^ 1]);
+                           shape, kb[at ^ 1], ib[at ^ 1]);
     GP_HIP(hipGetLastError());
     return MergeSorted{kb[at], ib[at]};
 }
@@ -357,7 +380,7 @@ MergeSorted run_merge_sort(hipStream_t st, const uint64_t* keys, int64_t n, cons
 }  // namespace
 
 MergeSorted merge_sort(gp_ctx* ctx, const std::string& name, const uint64_t* keys, int64_t n, const uint64_t* rest,
-                       int nrest) {
+                       int nrest, const MergeShape* shape) {
     if (n > 0xFFFFFFFFll) throw ArgError("sort: more than 2^32 records");
     if (n <= 0) return MergeSorted{nullptr, nullptr};
     uint64_t* const kb[2] = {ctx->dev<uint64_t>(name + ".k0", (size_t)n), ctx->dev<uint64_t>(name + ".k1", (size_t)n)};
@@ -365,10 +388,10 @@ MergeSorted merge_sort(gp_ctx* ctx, const std::string& name, const uint64_t* key
     const int64_t runs = n > 2 * kMsThreads * 4 && n <= kMsSmall ? ms_rank_runs(n, nrest > 0) : 0;  // two tiles: a merge
     uint32_t* const part = runs ? ctx->dev<uint32_t>(name + ".rank", (size_t)(n * runs / 2)) : nullptr;
     if (n <= kMsSmall)
-        return nrest > 0 ? run_merge_sort<true, 4>(ctx->stream, keys, n, rest, nrest, kb, ib, part)
-                         : run_merge_sort<false, 4>(ctx->stream, keys, n, rest, nrest, kb, ib, part);
-    return nrest > 0 ? run_merge_sort<true, 8>(ctx->stream, keys, n, rest, nrest, kb, ib, part)
-                     : run_merge_sort<false, 8>(ctx->stream, keys, n, rest, nrest, kb, ib, part);
+        return nrest > 0 ? run_merge_sort<true, 4>(ctx->stream, keys, n, rest, nrest, shape, kb, ib, part)
+                         : run_merge_sort<false, 4>(ctx->stream, keys, n, rest, nrest, shape, kb, ib, part);
+    return nrest > 0 ? run_merge_sort<true, 8>(ctx->stream, keys, n, rest, nrest, shape, kb, ib, part)
+                     : run_merge_sort<false, 8>(ctx->stream, keys, n, rest, nrest, shape, kb, ib, part);
 }
 
 }  // namespace gp

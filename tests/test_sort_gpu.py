@@ -7,6 +7,7 @@ the gen files."""
 import os
 import subprocess
 import tempfile
+import time
 
 import numpy as np
 import pytest
@@ -93,3 +94,42 @@ def test_sort_ranked_runs(gpu_ctx, m, key_values):
     32 runs of 1024; 2^16: 16 runs and merges), with distinct and equal first words."""
     c = _random_records(np.random.default_rng(m), m, 15, [-3, -1, 1, 3], key_values)
     assert gpu_ctx.sort_candidates(c).lines() == sorted(set(c.lines()))
+
+
+@pytest.mark.parametrize("letters", [[3], [-1, 1], [-2, 0, 2], [-128, 127, 5, 33, -33], list(range(-128, 128))])
+@pytest.mark.parametrize("kind", ["keys", "all but one", "words", "all"])
+@pytest.mark.parametrize("n,m", [(2, 300), (15, 5000), (37, 3000)])
+def test_sort_shared_digits_and_letters(gpu_ctx, n, m, kind, letters):
+    """Records that share their keys (but for the last one), their words or both, over
+    letters of 1 to 8 bits."""
+    rng = np.random.default_rng(n + len(letters))
+    words = rng.choice(letters, size=(m, n)).astype(np.int8)
+    keys = rng.choice([0, 7, 12, 123, 255], size=(m, n // 2)).astype(np.uint8)
+    if kind != "words":
+        keys[:m - (kind == "all but one")] = keys[0]
+    if kind in ("words", "all"):
+        words[:] = words[0]
+    c = g.Cands(words, keys)
+    assert gpu_ctx.sort_candidates(c).lines() == sorted(set(c.lines()))
+
+
+@pytest.mark.parametrize("n,m", [(50, 61000), (25, 400000)])
+def test_sort_repeats_cost_no_more_than_distinct_records(gpu_ctx, n, m):
+    """Records that share their first digits, or all of them, sort no slower than
+    records without ties."""
+    rng = np.random.default_rng(n)
+    words = rng.choice(np.array([-3, -1, 1, 3], np.int8), size=(m, n))
+    keys = rng.integers(0, 100, size=(m, n // 2)).astype(np.uint8)
+    best = {}
+    for kind, (w, k) in {"distinct": (words, keys), "same keys": (words, np.repeat(keys[:1], m, 0)),
+                         "same": (np.repeat(words[:1], m, 0), np.repeat(keys[:1], m, 0))}.items():
+        c = g.Cands(w.copy(), k.copy())
+        for _ in range(6):
+            np.copyto(c.words, w)
+            np.copyto(c.keys, k)
+            s = c.struct()
+            t0 = time.perf_counter()
+            gpu_ctx.check(gpu_ctx.lib.gp_sort_candidates(gpu_ctx.h, g.ctypes.byref(s)), "gp_sort_candidates")
+            best[kind] = min(best.get(kind, 1e9), time.perf_counter() - t0)
+        assert s.count == (1 if kind == "same" else m)
+    assert best["same"] < best["distinct"] and best["same keys"] < 1.3 * best["distinct"], best
