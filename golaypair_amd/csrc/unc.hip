@@ -20,7 +20,6 @@
 #include <array>
 #include <functional>
 #include <numeric>
-#include <queue>
 #include <tuple>
 #include <map>
 #include <stdexcept>
@@ -1138,12 +1137,12 @@ std::shared_ptr<UncPrep> unc_prepare(std::span<const SideHost> sides, std::span<
         const int mtc = SH.mt();
         std::vector<size_t> torder(live.size());
         std::iota(torder.begin(), torder.end(), 0);
-        if (!fp32)
-            std::stable_sort(torder.begin(), torder.end(), [&](size_t x, size_t y) {
-                const int64_t tx = (spl[x].ps + 31) / 32, ty = (spl[y].ps + 31) / 32;
-                if (tx != ty) return tx > ty;
-                return side_suf[x] < side_suf[y];
-            });
+        // (FP32 path: an item is an outer row, so all mid rows times the suffix)
+        auto cost = [&](size_t q) { return fp32 ? spl[q].pm * ((spl[q].ps + 63) / 64) : (spl[q].ps + 31) / 32; };
+        std::stable_sort(torder.begin(), torder.end(), [&](size_t x, size_t y) {
+            if (cost(x) != cost(y)) return cost(x) > cost(y);
+            return side_suf[x] < side_suf[y];
+        });
         std::vector<SideSlot> slot(live.size());
         int64_t n_radix = 0, n_tup = 0, n_pm1 = 0, n_pos = 0, n_olist = 0, n_fix = 0, n_xout = 0;
         for (size_t x = 0; x < torder.size(); ++x) {
