@@ -1328,20 +1328,25 @@ int64_t slot_join_cap(uint64_t leaves) {
 }
 int64_t band_cap(uint64_t leaves) { return (int64_t)std::min<uint64_t>(leaves / 64 + (1 << 16), (uint64_t)1 << 28); }
 
-// Uploads the staged tables into the device buffer `name` (one copy, on the copy
-// stream, which the context's stream then waits for, so that it overlaps earlier
-// kernels), points B's table fields there and returns the filter kernels' view of
-// them.  The staging buffer's event is recorded on the copy stream alone: a thread
-// that takes the buffer for a later batch waits for that event, and a wait for an
-// event of the context's stream while a batch is captured there ends the capture.
+// Uploads the staged tables into the device buffer `name`, points B's table fields there
+// and returns the filter kernels' view of them.  One copy: on the copy stream, which the
+// context's stream then waits for, so that it overlaps earlier kernels; or, without
+// `uploaded`, on the context's stream, and the caller waits for it before U's staging
+// buffer may be released.  (A buffer in the pool waits for events of the copy stream alone:
+// a thread that takes it for a later batch waits for them, and a wait for an event of the
+// context's stream while a batch is captured there ends the capture.)
 UncTabs upload_tables(gp_ctx* ctx, UncPrep& U, const std::string& name, UncBatch& B, const int64_t** d_toff,
-                      hipEvent_t uploaded) {
+                      hipEvent_t uploaded = nullptr) {
     unc_stage(U, ctx->pinned);
     char* base = static_cast<char*>(ctx->buf(name).ensure(U.stage_bytes));
-    GP_HIP(hipMemcpyAsync(base, U.base, U.stage_bytes, hipMemcpyHostToDevice, ctx->copy_stream));
-    GP_HIP(hipEventRecord(uploaded, ctx->copy_stream));
-    GP_HIP(hipStreamWaitEvent(ctx->stream, uploaded, 0));
-    if (U.stage) U.stage->record_upload(ctx->copy_stream);
+    if (uploaded) {
+        GP_HIP(hipMemcpyAsync(base, U.base, U.stage_bytes, hipMemcpyHostToDevice, ctx->copy_stream));
+        GP_HIP(hipEventRecord(uploaded, ctx->copy_stream));
+        GP_HIP(hipStreamWaitEvent(ctx->stream, uploaded, 0));
+        if (U.stage) U.stage->record_upload(ctx->copy_stream);
+    } else {
+        GP_HIP(hipMemcpyAsync(base, U.base, U.stage_bytes, hipMemcpyHostToDevice, ctx->stream));
+    }
     auto at = [&](int i) { return static_cast<void*>(base + U.stage_off[i]); };
     B.d_sides = static_cast<const UncSide*>(at(kStSides));
     B.d_radix = static_cast<const int32_t*>(at(kStRadix));
@@ -1434,10 +1439,11 @@ UncBatch unc_launch(gp_ctx* ctx, UncPrep& U, gp_stats* stats) {
     if (U.T.nsides == 0) return B;
     Phase ph2("unc_filter: upload");
     const int64_t* d_toff = nullptr;
-    // the copy comes after what a call before this one left on the stream
-    GP_HIP(hipEventRecord(ctx->ev3, st));
-    GP_HIP(hipStreamWaitEvent(ctx->copy_stream, ctx->ev3, 0));
-    const UncTabs tb = upload_tables(ctx, U, "u_stage", B, &d_toff, ctx->slot_ev[0][4]);
+    struct Wait {  // for the upload, also where an exception leaves before the first wait below
+        hipStream_t st;
+        ~Wait() { if (st) (void)hipStreamSynchronize(st); }
+    } wait{st};
+    const UncTabs tb = upload_tables(ctx, U, "u_stage", B, &d_toff);
     UncCtl* ctl = ctx->dev<UncCtl>("u_ctl", 1);
     int64_t scap = surv_cap(U.total_leaves);
     int64_t bcap = band_cap(U.total_leaves);
@@ -1453,6 +1459,7 @@ UncBatch unc_launch(gp_ctx* ctx, UncPrep& U, gp_stats* stats) {
         GP_HIP(hipEventRecord(ctx->ev1, st));
         GP_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, st));
         GP_HIP(hipStreamSynchronize(st));
+        wait.st = nullptr;
         GP_HIP(hipEventElapsedTime(&ms_filter, ctx->ev0, ctx->ev1));
         if ((int64_t)h.band > bcap) { bcap = (int64_t)h.band + 1024; continue; }
         if (h.band) {
