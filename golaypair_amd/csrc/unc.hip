@@ -1818,24 +1818,28 @@ CandSet unc_side_cands(gp_ctx* ctx, const UncBatch& B, int input_side, uint64_t 
     unsigned long long m = 0;
     GP_HIP(hipMemcpyAsync(&m, cnt, 8, hipMemcpyDeviceToHost, st));
     GP_HIP(hipStreamSynchronize(st));
-    std::vector<uint64_t> recs(m);
-    if (m) GP_HIP(hipMemcpyAsync(recs.data(), sel, m * 8, hipMemcpyDeviceToHost, st));
-    GP_HIP(hipStreamSynchronize(st));
-    std::sort(recs.begin(), recs.end());  // DFS order
+    if (m == 0) return c;
+    // DFS order (by the records' leaf numbers)
+    const uint64_t* order = merge_sort(ctx, "u_sel_sort", sel, (int64_t)m).key;
     if (proc_num > 1) {
+        std::vector<uint64_t> recs(m);
+        GP_HIP(hipMemcpyAsync(recs.data(), order, m * 8, hipMemcpyDeviceToHost, st));
+        GP_HIP(hipStreamSynchronize(st));
         const uint64_t leaf_mask = ((uint64_t)1 << 40) - 1;
         std::erase_if(recs, [&](uint64_t r) {
             return ((r & leaf_mask) / job_suffix) % (uint64_t)proc_num != (uint64_t)proc_id;
         });
         m = recs.size();
+        if (m == 0) return c;
+        GP_HIP(hipMemcpyAsync(sel, recs.data(), m * 8, hipMemcpyHostToDevice, st));
+        GP_HIP(hipStreamSynchronize(st));  // (recs ends here)
+        order = sel;
     }
-    if (m == 0) return c;
-    GP_HIP(hipMemcpyAsync(sel, recs.data(), m * 8, hipMemcpyHostToDevice, st));
     int8_t* w = ctx->dev<int8_t>("u_cw", (size_t)m * B.N);
     uint8_t* k = ctx->dev<uint8_t>("u_ck", (size_t)m * B.K);
     UncCtl* ctl = ctx->dev<UncCtl>("u_ctl", 1);
     hipLaunchKernelGGL(k_unc_keys, dim3(ctx->num_cus * 4), dim3(128), 0, st, B.d_sides, B.d_radix, B.d_tup, B.d_pos64, B.d_c64,
-                       sel, (int64_t)m, B.bound, w, k, ctl);
+                       order, (int64_t)m, B.bound, w, k, ctl);
     GP_HIP(hipGetLastError());
     c.words.resize((size_t)m * B.N);
     c.keys.resize((size_t)m * B.K);
