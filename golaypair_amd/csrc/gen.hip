@@ -753,7 +753,7 @@ int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, i
             const int ks = k - d0, Js = J - n * d0;
             if (Js < 0 || Js > (n - 1) * (ks - 1)) continue;
             const uint64_t c = cnt[(size_t)(ks - 1) * tsize + (size_t)(n - 1) * cstride + Js];
-            if (c >= cap) throw ArgError("gen: search space too large");
+            if (c >= cap || c > cap - (uint64_t)total) throw ArgError("gen: search space too large");
             total += (int64_t)c;
         }
     }

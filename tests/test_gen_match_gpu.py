@@ -220,3 +220,10 @@ def test_match_many_candidates_few_pairs(gpu_ctx):
     assert st.pair_checks == m * m
     assert (pa == wa[[i for i, _ in want]]).all() and (pb == wb[[j for _, j in want]]).all() and len(pa) == len(want)
     assert held < 1 << 28
+
+
+@pytest.mark.parametrize("order,compress,paf", [(212, 7, 372), (208, 7, 195)])
+def test_gen_refuses_levels_beyond_64_bits(gpu_ctx, order, compress, paf):
+    """Levels whose row sums each have fewer than 2^62 words, but together more than 2^63."""
+    with pytest.raises(g.GolayError, match="search space too large"):
+        gpu_ctx.generate(order, compress, paf, 0, 5)
