@@ -71,7 +71,7 @@ int gp_generate(gp_ctx* ctx, int order, int compress, int paf, int proc_id, int 
         if (!(key == g_gen_key)) {
             GenOutput o;
             gp_stats s{};
-            int rc = generate_level(ctx, order, compress, paf, proc_id, proc_num, o, &s);
+            int rc = generate_level(ctx, order, compress, paf, proc_id, proc_num, o, &s, stats != nullptr);
             if (rc != GP_OK) return rc;
             g_gen_out = std::move(o);
             g_gen_stats = s;

@@ -703,7 +703,7 @@ std::vector<int> units_of(int n) {
 }  // namespace
 
 int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, int proc_num, GenOutput& out,
-                   gp_stats* stats) {
+                   gp_stats* stats, bool timed) {
     hipStream_t st = ctx->stream;
     Phase ph("gen: setup");
     const int n = order / compress;
@@ -856,6 +856,7 @@ int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, i
             const double* t64 = ctx->tables.d_trig64.as<double>() + d.trig_off;
             GP_HIP(hipEventRecord(ctx->ev0, st));
             make_tasks();
+            if (timed) GP_HIP(hipEventRecord(ctx->ev2, st));
             if (tcap) {
                 auto launch = [&](auto kernel) {
                     hipLaunchKernelGGL(kernel, grid(), dim3(256), 0, st, P, F, d_tasks, d_ntasks, tcap, d_cnt.as<uint64_t>(),
@@ -871,9 +872,10 @@ int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, i
             GP_HIP(hipMemcpyAsync(&h, d_fc, sizeof h, hipMemcpyDeviceToHost, st));
             if (tcap) GP_HIP(hipMemcpyAsync(&ntasks, d_ntasks, sizeof ntasks, hipMemcpyDeviceToHost, st));
             GP_HIP(hipStreamSynchronize(st));
-            float ms = 0;
+            float ms = 0, ms_fused = 0;
             GP_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-            if (stats) { stats->kernel_ms += ms; stats->psd_kernel_ms += ms; stats->psd_launches += 1; }
+            if (timed) GP_HIP(hipEventElapsedTime(&ms_fused, ctx->ev2, ctx->ev1));
+            if (stats) { stats->kernel_ms += ms; stats->psd_kernel_ms += ms_fused; stats->psd_launches += 1; }
             if ((int64_t)h.rows <= cap && (int64_t)ntasks <= tcap) break;
             cap = std::max<int64_t>(cap, (int64_t)h.rows + 1024);
             tcap = std::max<int64_t>(tcap, (int64_t)ntasks);

@@ -45,6 +45,7 @@ PairSet import_pairs(const gp_pairs* in);
 
 struct gp_ctx;
 namespace gp {
+// `timed`: the caller wants the PSD kernel's own time (an event between kernels: 3 us).
 int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, int proc_num, GenOutput& out,
-                   gp_stats* stats);
+                   gp_stats* stats, bool timed);
 }

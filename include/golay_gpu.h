@@ -76,7 +76,9 @@ typedef struct gp_stats {
                                 threshold (0 for a parity-grade run)            */
     double kernel_ms;        /* device time of the call's kernels               */
     double psd_kernel_ms;    /* device time of its PSD-filter kernel launches   */
-    double band_kernel_ms;   /* device time of its FP64 band-recheck launches   */
+    double band_kernel_ms;   /* device time of its FP64 band-recheck launches (0 where
+                                the filter's own kernel settles the band: gen and the
+                                two batched filters of caller rows)               */
     uint64_t psd_launches;   /* PSD-filter kernel launches timed above          */
 } gp_stats;
 

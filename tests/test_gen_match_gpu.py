@@ -227,3 +227,14 @@ def test_gen_refuses_levels_beyond_64_bits(gpu_ctx, order, compress, paf):
     """Levels whose row sums each have fewer than 2^62 words, but together more than 2^63."""
     with pytest.raises(g.GolayError, match="search space too large"):
         gpu_ctx.generate(order, compress, paf, 0, 5)
+
+
+@pytest.mark.parametrize("mode", [g.GP_PSD_SPLIT_BF16, g.GP_PSD_FP32])
+def test_gen_device_times(gpu_ctx, mode):
+    """psd_kernel_ms is the time of the kernel with the PSD filter, kernel_ms that of all."""
+    gpu_ctx.set_mode(mode)
+    try:
+        st = gpu_ctx.generate(45, 3, -2, 1, 8)[2]
+    finally:
+        gpu_ctx.set_mode(g.GP_PSD_SPLIT_BF16)
+    assert 0 < st.psd_kernel_ms < st.kernel_ms and st.psd_launches == 1
