@@ -237,3 +237,15 @@ def test_filter_more_than_2_31_pairs(gpu_ctx):
     finally:
         ctx.close()
     assert oa[:out.count, 0].tolist() == [-1, 1, 3] and ob[:out.count, 0].tolist() == [-1, 1, 3]
+
+
+def test_filter_device_time_counts_every_kernel(gpu_ctx):
+    """2e5 pairs of as many classes, which are sorted, against 2e5 pairs of one class, which
+    meet in one slot of the table: the orbit kernel takes as long for both, the call's
+    kernels do not."""
+    rng, m, n = np.random.default_rng(2), 200000, 12
+    a, b = (rng.integers(-7, 8, size=(m, n)).astype(np.int8) for _ in range(2))
+    ms = []
+    for x, y in ((a, b), (np.repeat(a[:1], m, 0), np.repeat(b[:1], m, 0))):
+        ms.append(min(gpu_ctx.filter(2 * n, 2, x, y)[2].kernel_ms for _ in range(4)))
+    assert max(ms) > 1.5 * min(ms) > 0, ms
