@@ -23,9 +23,15 @@ struct Ring {
     PinnedPool& pool;
     std::array<PinnedBuf*, kBufs> b{};
     explicit Ring(PinnedPool& p) : pool(p) {
-        for (auto& x : b) x = pool.acquire(kChunk);
+        try {
+            for (auto& x : b) x = pool.acquire(kChunk);
+        } catch (...) {  // (no destructor runs)
+            give_back();
+            throw;
+        }
     }
-    ~Ring() {
+    ~Ring() { give_back(); }
+    void give_back() {
         for (PinnedBuf* x : b) pool.release(x);  // (a copy from it that still runs is waited for by the next user)
     }
 };

@@ -167,11 +167,11 @@ struct PinnedPool {
             GP_HIP(hipHostMalloc(&pick->p, want, hipHostMallocDefault));
             pick->bytes = want;
         }
-        pick->busy = true;
         if (pick->upload_pending) {  // its last copy to the device must be done before it is refilled
             GP_HIP(hipEventSynchronize(pick->upload));
             pick->upload_pending = false;
         }
+        pick->busy = true;
         return pick;
     }
     void release(PinnedBuf* b) {
