@@ -19,13 +19,16 @@ Per workload (order, compression pair, PAF constant):
   unc_counter_streams/<N>      work counters per filter launch: 1 .. 4
                                (default 8, one per XCD);
 the uncompression candidates timed on a fixed slice of the level's matched
-pairs.  Each candidate runs `reps` times (minimum wall time kept) and its
-output must equal the default setting's, byte for byte; the winner replaces
-the default only if it is at least 3 % faster (run-to-run noise is about 2 %).
+pairs.  The default and the candidates take turns, `reps` times, and every
+output must equal the default setting's, byte for byte.  The fastest candidate by
+median replaces the default only if it gains 2 % and its third quartile still lies
+below the default's first: one that gains less than the runs of one setting differ
+would be chosen by chance.
 """
 import argparse
 import hashlib
 import os
+import statistics
 import sys
 import time
 
@@ -62,36 +65,35 @@ def _set(ctx, key, value):
         raise g.GolayError("gp_set_tuning %s failed" % key)
 
 
-def _time(fn, reps):
-    best, out = None, None
-    for _ in range(reps):
-        t0 = time.perf_counter()
-        out = fn()
-        dt = time.perf_counter() - t0
-        best = dt if best is None else min(best, dt)
-    return best, out
+def choose(times):
+    """The candidate of {None (the default) or value: seconds of its runs} to keep, or None."""
+    med = {v: statistics.median(t) for v, t in times.items()}
+    best = min((v for v in times if v is not None), key=lambda v: med[v], default=None)
+    if best is None:
+        return None
+    quartiles = lambda v: statistics.quantiles(times[v], n=4)
+    return best if med[best] < 0.98 * med[None] and quartiles(best)[2] < quartiles(None)[0] else None
 
 
 def _sweep(ctx, key, candidates, run, reps, log):
-    """Times run() with key unset (the default) and at every candidate; returns
-    (chosen value or None for the default, {value: seconds})."""
-    _set(ctx, key, None)
-    t_def, ref = _time(run, reps)
-    times = {"default": t_def}
-    best_v, best_t = None, t_def
-    for v in candidates:
-        _set(ctx, key, v)
-        t, out = _time(run, reps)
-        if out != ref:
-            raise RuntimeError("%s=%d changed the output" % (key, v))
-        times[v] = t
-        if t < best_t * 0.97:
-            best_v, best_t = v, t
-    _set(ctx, key, best_v)
-    log("%-28s default %.4f s; %s -> %s" % (key, t_def, ", ".join("%s: %.4f" % (k, t) for k, t in times.items()
-                                                                  if k != "default"),
-                                           "default" if best_v is None else best_v))
-    return best_v, times
+    """Times run() with key unset (the default) and at every candidate in turn; returns
+    (chosen value or None for the default, {value: median seconds})."""
+    times = {v: [] for v in [None] + candidates}
+    ref = None
+    for _ in range(reps):
+        for v in times:
+            _set(ctx, key, v)
+            t0 = time.perf_counter()
+            out = run()
+            times[v].append(time.perf_counter() - t0)
+            ref = ref or _digest(out)
+            if _digest(out) != ref:
+                raise RuntimeError("%s=%s changed the output" % (key, v))
+    best = choose(times)
+    _set(ctx, key, best)
+    med = {"default" if v is None else v: round(statistics.median(t), 7) for v, t in times.items()}
+    log("%-28s %s -> %s" % (key, ", ".join("%s: %.6f" % x for x in med.items()), "default" if best is None else best))
+    return best, med
 
 
 def tune(workloads, reps, log):
@@ -105,7 +107,7 @@ def tune(workloads, reps, log):
 
             def gen():
                 a, b, _ = ctx.generate(order, c0, paf)
-                return _digest([a.words, a.keys, b.words, b.keys])
+                return [a.words, a.keys, b.words, b.keys]
 
             key = "gen_ranks_per_lane/%d/%d" % (n0, k)
             v, t = _sweep(ctx, key, GEN_RANKS, gen, reps, log)
@@ -118,7 +120,7 @@ def tune(workloads, reps, log):
 
             def unc():
                 oa, ob, _, _, _ = ctx.uncompress(order, c0, c1, paf, pa, pb)
-                return _digest([oa, ob])
+                return [oa, ob]
 
             for key, cand in (("unc_waves/%d" % N, UNC_WAVES), ("unc_leaf_budget/%d" % N, UNC_BUDGET),
                               ("unc_counter_rounds/%d" % N, UNC_COUNTER_ROUNDS),
@@ -135,8 +137,8 @@ def tune(workloads, reps, log):
 def write(path, chosen, notes, workloads, reps):
     with open(path, "w") as f:
         f.write("# Tuning table of golaypair_amd, written by python -m golaypair_amd.autotune\n")
-        f.write("# workloads %s, %d timed runs per candidate (minimum kept); keys absent here use the\n"
-                "# built-in defaults.  Measured wall times in seconds per candidate:\n" % (" ".join(workloads), reps))
+        f.write("# workloads %s, %d timed runs per candidate in turn; keys absent here use the\n"
+                "# built-in defaults.  Median wall times in seconds per candidate:\n" % (" ".join(workloads), reps))
         for n in notes:
             f.write("#   %s\n" % n)
         for key in sorted(chosen):
@@ -147,7 +149,7 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--out", default=DEFAULT_OUT)
     ap.add_argument("--workloads", nargs="*", default=list(WORKLOADS))
-    ap.add_argument("--reps", type=int, default=5)
+    ap.add_argument("--reps", type=int, default=21)
     args = ap.parse_args()
     os.environ["GOLAY_TUNING"] = os.devnull  # start from the built-in defaults
     chosen, notes = tune(args.workloads, args.reps, lambda s: print(s, file=sys.stderr, flush=True))

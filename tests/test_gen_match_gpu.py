@@ -238,3 +238,29 @@ def test_gen_device_times(gpu_ctx, mode):
     finally:
         gpu_ctx.set_mode(g.GP_PSD_SPLIT_BF16)
     assert 0 < st.psd_kernel_ms < st.kernel_ms and st.psd_launches == 1
+
+
+def _splits(n, k, njobs):
+    """Whether njobs jobs share the necklaces of length n (lyndon.cpp:87-106): some prefix
+    shorter than the words has 10^4 necklaces per job."""
+    count = lambda i: sum(k ** int(np.gcd(i, j)) for j in range(1, i + 1)) // i
+    return njobs > 1 and any(count(i) >= 10000 * njobs for i in range(1, n))
+
+
+@pytest.mark.parametrize("order,compress,paf,njobs,split", [
+    (8, 2, 0, 3, False), (26, 2, 0, 7, False), (26, 1, 0, 2, True), (26, 1, 0, 40, True), (34, 2, 0, 5, True),
+    (34, 2, 0, 40, True), (45, 3, -2, 8, True), (45, 3, -2, 40, True), (50, 5, 0, 3, True), (50, 5, 0, 200, False),
+])
+def test_gen_job_split(gpu_ctx, order, compress, paf, njobs, split):
+    """Where the level is split, its jobs' records are disjoint and together the level's;
+    where it is not, every job has them all."""
+    assert _splits(order // compress, compress + 1, njobs) == split
+    a, b, _ = gpu_ctx.generate(order, compress, paf)
+    parts = [gpu_ctx.generate(order, compress, paf, j, njobs)[:2] for j in range(min(njobs, 40))]
+    for side, level in ((0, a.lines()), (1, b.lines())):
+        jobs = [p[side].lines() for p in parts]
+        if split:
+            assert sorted(sum(jobs, [])) == sorted(level) and len(set(level)) == len(level) > 0
+            assert len(level) < 100 or max(map(len, jobs)) < len(level)
+        else:
+            assert all(j == level for j in jobs)

@@ -23,3 +23,14 @@ def test_tuning_table_format():
         entries += 1
     head = open(TABLE).read()
     assert "golaypair_amd.autotune" in head
+
+
+def test_tuning_choice_is_beyond_the_noise():
+    """A candidate is kept only where its runs lie below the default's, not where a few do."""
+    from golaypair_amd.autotune import choose
+    noisy = [5.37, 5.22, 5.45, 5.31, 5.08, 5.57, 5.40, 5.28]
+    assert choose({None: noisy, 2: [4.99, 5.45, 5.36, 5.30, 5.50, 5.21, 5.33, 5.41]}) is None
+    assert choose({None: noisy, 2: [x - 0.02 for x in noisy], 4: [x + 0.1 for x in noisy]}) is None
+    assert choose({None: noisy, 2: [4.99, 5.45, 5.36, 5.30, 5.50, 5.21, 5.33, 5.41], 3: [4.7] * 7 + [5.9]}) == 3
+    assert choose({None: [5.30, 5.31, 5.30, 5.32], 2: [5.27, 5.28, 5.27, 5.28]}) is None
+    assert choose({None: noisy}) is None
