@@ -389,3 +389,40 @@ def test_uncompress_device_memory(gpu_ctx):
     out, held = _device.held_by(lambda ctx: ctx.uncompress(50, 5, 1, 0, pa[:100], pb[:100]))
     assert out[4].psd_decisions > 1.5e10
     assert held < 17e9
+
+
+@pytest.mark.parametrize("seq,c,paf,passing", [
+    ([1, 3, -3, 1, -1, 1, 3, -1, -3, 3, 3, -1, 1, 1, -3, -3, -3, 1, 1, 3, 1], 3, -129, 57201),  # N = 63: 21 channels
+    ([9, 9, 9, 11, 9], 11, 50, 1170),       # N = 55: 25
+    ([14, 14, 14, 14], 16, 68, 3648),       # N = 64: 30
+])
+def test_uncompress_side_channel_pairs(gpu_ctx, seq, c, paf, passing):
+    """The filter kernels of 11, 13 and 15 channel pairs; DFS candidate lines vs the oracle."""
+    seq = np.array(seq, np.int8)
+    for seqflag in (0, 1):
+        ref_text, ref_leaves = _oracle.uncompress_side(seq, c, 1, paf, seqflag)
+        cands, rot, st = gpu_ctx.uncompress_side(seq, c, 1, paf, seqflag)
+        assert len(cands) == passing and st.psd_decisions == ref_leaves
+        assert "".join(l + "\n" for l in cands.lines()) == ref_text
+
+
+def test_uncompress_fixed_channel_at_the_threshold(gpu_ctx):
+    """Length 64 from a word with a PSD within 1e-6 of the threshold at a frequency that the
+    compressed word fixes: no channel of the batch is then left out of the filter (16 channel
+    pairs), for its sides and for those of the other pair.  Candidate files vs the oracle."""
+    at = np.array([0, 2, 2, 2, -2, 0, -2, -2, 2, 2, 0, 0, 0, -2, 2, 0, -2, 2, 2, 0, 2, -2, 2, 0, 0, 2, 0, 0, 2, 2, -2, 0])
+    other = np.array([-2, 0, 2, 0, 2, 2, -2, 2, 2, 2, 0, 2, 0, 0, 2, 2, 2, 0, 0, 2, 0, 2, 0, 2, 2, 2, 2, 0, 2, 0, 0, 0])
+    paf = 29
+    psd = np.abs(np.fft.fft(at)) ** 2
+    assert np.abs(psd - (2 * 64 - paf + 0.001)).min() < 1e-6
+    pairs = [(at, other), (other, at), (other, other)]
+    want = {(s, f): _oracle.uncompress_side(w, 2, 1, paf, f)[0] for s, w in (("at", at), ("other", other)) for f in (0, 1)}
+    assert len(want["other", 0].splitlines()) == 14
+    for n in (1, 2, 3):
+        pa, pb = (np.array([p[k] for p in pairs[:n]], np.int8) for k in (0, 1))
+        oa, ob, ta, tb, st = gpu_ctx.uncompress(64, 2, 1, paf, pa, pb, want_tmp=True)
+        assert st.psd_pass == sum(len(want["at" if w is at else "other", f].splitlines())
+                                  for p in pairs[:n] for f, w in enumerate(p))
+        for tmp, f in ((ta, 0), (tb, 1)):
+            name = "at" if pairs[n - 1][f] is at else "other"
+            assert "".join(l + "\n" for l in tmp.lines()) == want[name, f]
