@@ -75,12 +75,6 @@ struct FilterThr {
     double thr;
 };
 
-struct TileDesc {
-    int32_t table;
-    int32_t rows;
-    int64_t first_row;
-};
-
 // Host wall-clock phases, printed to stderr when GOLAY_PROFILE is set.
 struct Phase {
     const char* name;
@@ -275,7 +269,7 @@ struct BatchSeg {
 };
 double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nrows,
                       const std::vector<BatchSeg>& segs, const std::vector<FilterThr>& thr_by_table,
-                      uint8_t* d_decision, gp_stats* stats, float* d_maxpsd = nullptr);
+                      uint8_t* d_decision, gp_stats* stats);
 
 // gp_psd_filter_batch on checked, non-empty arguments (host buffers); throws on a
 // word length out of range before anything is written.

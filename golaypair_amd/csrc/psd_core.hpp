@@ -40,23 +40,9 @@ __device__ __forceinline__ uint4 pack8_bf16(uint32_t w0, uint32_t w1) {
     return r;
 }
 
-// Contraction for one tile: NB position blocks, MT M-tiles.  `afrag` points at
-// the table's pre-swizzled A fragments; `bop[b]` is this lane's B operand for
-// block b.  `acc` is initialised by the caller (zero or a prefix sum).
-template <int NB, int MT>
-__device__ __forceinline__ void mfma_tile(const uint4* __restrict__ afrag, const uint4 (&bop)[NB],
-                                          f32x16 (&acc)[MT], int lane) {
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-#pragma unroll
-        for (int s = 0; s < 2 * NB; ++s) {
-            uint4 a = afrag[((t * 2 * NB) + s) * 64 + lane];
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(bop[s % NB]), acc[t], 0, 0, 0);
-        }
-    }
-}
-
-// Same contraction with the A fragments already held in registers.
+// Contraction for one tile: NB position blocks, MT M-tiles.  `a` are the table's
+// pre-swizzled A fragments; `bop[b]` is this lane's B operand for block b.  `acc` is
+// initialised by the caller.
 template <int NB, int MT>
 __device__ __forceinline__ void mfma_tile_reg(const uint4 (&a)[MT][2 * NB], const uint4 (&bop)[NB],
                                               f32x16 (&acc)[MT]) {
@@ -98,11 +84,6 @@ __device__ __forceinline__ float tile_pair_max_psd1(const f32x16& acc0, const f3
     for (int r = 0; r < 8; ++r) m1 = max(m1, __float_as_uint(__builtin_fmaf(acc1[r], acc1[r], acc1[r + 8] * acc1[r + 8])));
     const auto sw = __builtin_amdgcn_permlane32_swap(m0, m1, false, false);
     return __uint_as_float(max((uint32_t)sw[0], (uint32_t)sw[1]));
-}
-
-// The k (1-based) held by register r (< 8) of M-tile t in lane `lane`.
-__device__ __forceinline__ int tile_k(int t, int r, int lane) {
-    return 16 * t + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) + 1;
 }
 
 // FP64 max_{1<=k<=n/2} PSD_k of a word held in memory (direct DFT with the

@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(256) k_psd_mfma(const int8_t* __restrict__ wor
                                                   const PsdTableDesc* __restrict__ tabs,
                                                   const uint4* __restrict__ frags,
                                                   const FilterThr* __restrict__ thr,
-                                                  uint8_t* __restrict__ decision, float* __restrict__ maxpsd) {
+                                                  uint8_t* __restrict__ decision) {
     constexpr int D = NB == 1 ? 8 : NB == 2 ? 4 : 2;
     const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
@@ -257,10 +257,7 @@ __global__ void __launch_bounds__(256) k_psd_mfma(const int8_t* __restrict__ wor
                 const int64_t r = q * 32 + lane;
                 const bool mine = r < rows && (lane < 32 || q + 1 < q1);
                 const uint8_t dec = m > th.hi ? kReject : (m < th.lo ? kAccept : kBand);
-                if (mine) {
-                    decision[row_first + r] = dec;
-                    if (maxpsd) maxpsd[row_first + r] = m;
-                }
+                if (mine) decision[row_first + r] = dec;
             }
         }
         return;
@@ -282,11 +279,7 @@ __global__ void __launch_bounds__(256) k_psd_mfma(const int8_t* __restrict__ wor
             const int64_t r = q * 32 + col;
             const bool mine = half == 0 && r < rows;
             const uint8_t dec = m > th.hi ? kReject : (m < th.lo ? kAccept : kBand);
-            const int64_t row = row_first + r;
-            if (mine) {
-                decision[row] = dec;
-                if (maxpsd) maxpsd[row] = m;
-            }
+            if (mine) decision[row_first + r] = dec;
         }
     }
 }
@@ -295,7 +288,7 @@ __global__ void __launch_bounds__(256) k_psd_mfma(const int8_t* __restrict__ wor
 // (at most every resident wave slot of the class).
 void launch_psd_mfma(const SegTiles& all, const std::vector<PsdTableDesc>& desc, int num_cus, hipStream_t st,
                      const int8_t* words, const PsdTableDesc* tabs, const uint4* frags,
-                     const FilterThr* thr, uint8_t* decision, float* maxpsd) {
+                     const FilterThr* thr, uint8_t* decision) {
     auto cls = [&](int sg) {
         const PsdTableDesc& d = desc[all.table[sg]];
         return d.nb == 1 ? 0 : d.nb == 2 && d.mt == 1 ? 1 : d.nb == 3 && d.mt == 1 ? 2 : d.nb == 3 ? 3 : 4;
@@ -330,8 +323,7 @@ void launch_psd_mfma(const SegTiles& all, const std::vector<PsdTableDesc>& desc,
         const dim3 grid((unsigned)std::max<int64_t>(1, (waves + 3) / 4));
 #define GP_PSD_CASE(C, NB, MT)                                                                                   \
     case C:                                                                                                      \
-        hipLaunchKernelGGL((k_psd_mfma<NB, MT>), grid, dim3(256), 0, st, words, T, tabs, frags, thr, decision,  \
-                           maxpsd);                                                                              \
+        hipLaunchKernelGGL((k_psd_mfma<NB, MT>), grid, dim3(256), 0, st, words, T, tabs, frags, thr, decision); \
         break;
         switch (c) {
             GP_PSD_CASE(0, 1, 1)
@@ -375,7 +367,7 @@ __global__ void __launch_bounds__(256) k_psd_fp32(const int8_t* __restrict__ wor
                                                   const PsdTableDesc* __restrict__ tabs,
                                                   const float* __restrict__ trig32,
                                                   const FilterThr* __restrict__ thr,
-                                                  uint8_t* __restrict__ decision, float* __restrict__ maxpsd) {
+                                                  uint8_t* __restrict__ decision) {
     __shared__ float lds[8][2 * kMaxN];
     __shared__ int seg_table[8];
     if (threadIdx.x < 8 && (int)threadIdx.x < nseg) seg_table[threadIdx.x] = segs[threadIdx.x].table;
@@ -398,7 +390,6 @@ __global__ void __launch_bounds__(256) k_psd_fp32(const int8_t* __restrict__ wor
             const int8_t* w = words + S.byte0 + r * S.stride;
             float m = d.K <= 16 ? fp32_max_psd<16>(w, d.n, d.K, c, s) : fp32_max_psd<32>(w, d.n, d.K, c, s);
             decision[row] = m > th.hi ? kReject : (m < th.lo ? kAccept : kBand);
-            if (maxpsd) maxpsd[row] = m;
         }
     }
 }
@@ -482,7 +473,7 @@ __global__ void __launch_bounds__(256) k_psd_fp64(const int8_t* __restrict__ wor
 
 double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nrows,
                       const std::vector<BatchSeg>& segs_in, const std::vector<FilterThr>& thr_by_table,
-                      uint8_t* d_decision, gp_stats* stats, float* d_maxpsd) {
+                      uint8_t* d_decision, gp_stats* stats) {
     if (segs_in.size() > 8) throw ArgError("at most 8 word lengths per PSD batch");
     std::vector<BatchSeg> segs(segs_in);
     for (BatchSeg& sg : segs) {
@@ -516,13 +507,13 @@ double run_psd_filter(gp_ctx* ctx, const int8_t* d_words, int stride, int64_t nr
     if (ctx->psd_mode == GP_PSD_SPLIT_BF16) {
         if (nrow_total > 0)
             launch_psd_mfma(T, ctx->tables.desc, ctx->num_cus, st, d_words, ctx->tables.d_desc.as<PsdTableDesc>(),
-                            ctx->tables.d_frags.as<uint4>(), d_thr, d_decision, d_maxpsd);
+                            ctx->tables.d_frags.as<uint4>(), d_thr, d_decision);
     } else {
         int blocks = (int)std::min<int64_t>((nrow_total + 255) / 256, (int64_t)ctx->num_cus * 8);
         if (nrow_total > 0)
             hipLaunchKernelGGL(k_psd_fp32, dim3(std::max(blocks, 1)), dim3(256), 0, st, d_words, d_segs,
                                (int)segs.size(), ctx->tables.d_desc.as<PsdTableDesc>(),
-                               ctx->tables.d_trig32.as<float>(), d_thr, d_decision, d_maxpsd);
+                               ctx->tables.d_trig32.as<float>(), d_thr, d_decision);
     }
     GP_HIP(hipGetLastError());
     GP_HIP(hipEventRecord(ctx->ev1, st));
