@@ -321,7 +321,11 @@ JoinResult join_pairs(gp_ctx* ctx, const int8_t* d_wa, const uint8_t* d_ka, int6
     }
     // emission order of the reference: A position outer, B position inner
     std::vector<uint64_t> pairs(h.out);
-    if (h.out) {
+    if (h.out > 0xFFFFFFFFull) {  // (more than the device sort numbers)
+        GP_HIP(hipMemcpyAsync(pairs.data(), out, h.out * 8, hipMemcpyDeviceToHost, st));
+        GP_HIP(hipStreamSynchronize(st));
+        std::sort(pairs.begin(), pairs.end());
+    } else if (h.out) {
         const MergeSorted s = merge_sort(ctx, "j_sort", out, (int64_t)h.out);
         GP_HIP(hipMemcpyAsync(pairs.data(), s.key, h.out * 8, hipMemcpyDeviceToHost, st));
     }

@@ -34,11 +34,14 @@ constexpr int64_t kMsSmall = 1 << 18;
 // Rounds over runs of a few tiles are one step (k_ms_rank, k_ms_place): each record's
 // place among `ms_rank_runs` runs, all searched at once, two per block.  A record is
 // searched in every run where a round of merges passes it once, but the searches do
-// not wait for each other.  Calls of gp_sort_candidates on random records of n = 15,
-// merges against ranks of 32 runs: 18 000 records 190 and 159 us, 32 768 216 and 187;
-// 61 000 283 and 250, and with 16 runs and the rounds over those 257.  Where all first
-// words are equal each search reads further words: 32 768 records 331 and 302 us, but
-// 61 000 408 and 469 (32 runs) or 405 (16 runs), 100 000 553 and 619 (16 runs).  Without
+// not wait for each other.  Calls of gp_sort_candidates on records of n = 15 with merges
+// alone, ranks of 16 and of 32 runs, in us, where the first words differ, and where all but
+// one record have the same first word, so that each search reads further words:
+//   32 768 records  195, 175, 177 and 315, 300, 298
+//   61 000          250, 234, 234     382, 387, 455
+//  100 000          360, 347, 349     516, 578, 720
+//  200 000          580, 567, 581     764, 978, 1230
+// Beyond 2^16 the ranks gain 3 % and lose more where first words tie.  Without
 // further words an equal first word costs nothing more.
 __host__ __device__ constexpr int64_t ms_rank_runs(int64_t n, bool rest) {
     return !rest || n <= 1 << 15 ? 32 : n <= 1 << 16 ? 16 : 0;
