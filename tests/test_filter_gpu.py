@@ -239,7 +239,7 @@ def test_filter_more_than_2_31_pairs(gpu_ctx):
     assert oa[:out.count, 0].tolist() == [-1, 1, 3] and ob[:out.count, 0].tolist() == [-1, 1, 3]
 
 
-def test_filter_device_time_counts_every_kernel(gpu_ctx):
+def test_filter_device_time_counts_classes_and_order(gpu_ctx):
     """2e5 pairs of as many classes, which are sorted, against 2e5 pairs of one class, which
     meet in one slot of the table: the orbit kernel takes as long for both, the call's
     kernels do not."""
