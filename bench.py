@@ -301,7 +301,7 @@ def fp32_parity(order, c0, c1, paf, chunk=200):
     rc, pa, pb, _ = ctx.match(order, c0, paf, ctx.sort_candidates(a), ctx.sort_candidates(b))
     res = {"order": order, "compress": [c0, c1], "paf": paf, "pairs_in": len(pa)}
     texts = {}
-    for mode, name in ((g.GP_PSD_SPLIT_BF16, "split_bf16"), (g.GP_PSD_FP32, "fp32")):
+    for mode, name in ((g.GP_PSD_SPLIT_BF16, "matrix"), (g.GP_PSD_FP32, "fp32")):
         ctx.set_mode(mode)
         parts, leaves, kern, t0 = [], 0, 0.0, time.perf_counter()
         for q in range(0, len(pa), chunk):
@@ -317,8 +317,8 @@ def fp32_parity(order, c0, c1, paf, chunk=200):
                      "sha256": hashlib.sha256(texts[name].encode()).hexdigest(),
                      "candidates_per_s_kernel": leaves / (kern * 1e-3)}
     ctx.close()
-    res["identical"] = texts["split_bf16"] == texts["fp32"]
-    res["fp32_over_split_kernel_time"] = res["fp32"]["psd_kernel_ms"] / res["split_bf16"]["psd_kernel_ms"]
+    res["identical"] = texts["matrix"] == texts["fp32"]
+    res["fp32_over_matrix_kernel_time"] = res["fp32"]["psd_kernel_ms"] / res["matrix"]["psd_kernel_ms"]
     return res
 
 
@@ -422,7 +422,7 @@ def main():
     if not args.no_fp32:
         q0, q1 = FP32_SLICE
         outs, res = {}, {}
-        for mode, name in ((g.GP_PSD_SPLIT_BF16, "split_bf16"), (g.GP_PSD_FP32, "fp32")):
+        for mode, name in ((g.GP_PSD_SPLIT_BF16, "matrix"), (g.GP_PSD_FP32, "fp32")):
             ctx.set_mode(mode)
             t0 = time.perf_counter()
             oa, ob, _, _, s = ctx.uncompress(ORDER, C0, C1, PAF, pa[q0:q1], pb[q0:q1])
@@ -433,10 +433,10 @@ def main():
                          "pairs_out": len(oa)}
         ctx.set_mode(g.GP_PSD_SPLIT_BF16)
         line["fp32_path"] = {"slice": "uncompression 5->1 of the v=50 matched pairs [%d, %d) in file order" % (q0, q1),
-                             "identical_output": outs["split_bf16"] == outs["fp32"],
-                             "split_bf16": res["split_bf16"], "fp32": res["fp32"],
-                             "split_bf16_speedup_kernel": res["fp32"]["psd_kernel_ms"] /
-                             max(res["split_bf16"]["psd_kernel_ms"], 1e-9)}
+                             "identical_output": outs["matrix"] == outs["fp32"],
+                             "matrix": res["matrix"], "fp32": res["fp32"],
+                             "matrix_speedup_kernel": res["fp32"]["psd_kernel_ms"] /
+                             max(res["matrix"]["psd_kernel_ms"], 1e-9)}
     if not args.no_microbench:
         line["microbench"] = {"split_bf16": microbench(ctx, g, g.GP_PSD_SPLIT_BF16),
                               "fp32": microbench(ctx, g, g.GP_PSD_FP32)}
