@@ -758,7 +758,9 @@ int generate_level(gp_ctx* ctx, int order, int compress, int paf, int proc_id, i
         }
     }
     // words per lane of a task: about 8 wave tasks per resident wave (so that the last
-    // round of tasks is short), at least 16 to amortise each lane's unrank
+    // round of tasks is short), at least 16 to amortise each lane's unrank (at n = 15 with 4
+    // letters 4 are better still, 1.10 ms for the level against 1.17, at n = 9 and 10 no better:
+    // the tuning table)
     const int64_t target_tasks = (int64_t)ctx->num_cus * 32 * 8;
     const int heuristic = (int)std::clamp<int64_t>((total + 64 * target_tasks - 1) / (64 * target_tasks), 16, 128);
     const int per_lane = (int)std::clamp<int64_t>(

@@ -2,11 +2,11 @@
 // (stage, word length, alphabet), written by the autotuner
 // (python -m golaypair_amd.autotune) into golaypair_amd/tuning.tsv and read
 // when a context is created.  Keys and their defaults:
-//   unc_waves/<N>                  filter waves per SIMD (capped by each operand
-//                                  class's occupancy)              class maximum
-//   unc_leaf_budget/<N>            leaves per uncompression device batch   2^30
+//   unc_waves/<N>                  filter blocks per CU, one wave per SIMD each (capped
+//                                  by the registers of its channels)    the most
+//   unc_leaf_budget/<N>            leaves per uncompression device batch   2^31
 //   unc_counter_rounds/<N>         filter item rounds handed out by the work
-//                                  counters (the rounds before go by wave
+//                                  counters (the rounds before go by block
 //                                  index)                                   all
 //   unc_counter_streams/<N>        work counters per filter launch (1..8)      8
 //   gen_ranks_per_lane/<n>/<k>     gen ranks per lane, k letters     heuristic
