@@ -151,6 +151,10 @@ struct PinnedPool {
             bufs.emplace_back(new PinnedBuf());
             pick = bufs.back().get();
         }
+        if (pick->upload_pending) {  // its last copy to the device must be done before it is refilled or freed
+            GP_HIP(hipEventSynchronize(pick->upload));
+            pick->upload_pending = false;
+        }
         if (pick->bytes < n) {
             if (pick->p) GP_HIP(hipHostFree(pick->p));
             pick->p = nullptr;
@@ -160,10 +164,6 @@ struct PinnedPool {
             const size_t want = high + high / 4 + 4096;
             GP_HIP(hipHostMalloc(&pick->p, want, hipHostMallocDefault));
             pick->bytes = want;
-        }
-        if (pick->upload_pending) {  // its last copy to the device must be done before it is refilled
-            GP_HIP(hipEventSynchronize(pick->upload));
-            pick->upload_pending = false;
         }
         pick->busy = true;
         return pick;

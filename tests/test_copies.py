@@ -1,6 +1,6 @@
 """Staged copies (golaypair_amd/csrc/copies.hip) over a stand-in of the runtime calls that
-they make: every byte arrives at sizes around the chunks, and a call that fails for want
-of pinned memory hands back what it had taken."""
+they make: every byte arrives at sizes around the chunks, a call that fails for want of
+pinned memory hands back what it had taken, and a buffer is not freed under its last copy."""
 import os
 import subprocess
 
@@ -27,11 +27,12 @@ inline hipError_t hipHostMalloc(void** p, size_t n, int) {
     *p = std::malloc(n);
     return hipSuccess;
 }
-inline hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+inline int recorded = 0, freed_in_flight = 0;  // events recorded and not waited for; buffers freed meanwhile
+inline hipError_t hipHostFree(void* p) { freed_in_flight += recorded; std::free(p); return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, int) { *e = std::malloc(1); return hipSuccess; }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { ++recorded; return hipSuccess; }
+inline hipError_t hipEventSynchronize(hipEvent_t) { recorded = 0; return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t e) { std::free(e); return hipSuccess; }
 '''
 
@@ -60,6 +61,14 @@ int main() {
         host_mallocs_left = 1 << 30;
         gp::copy_to_device(&poor, b.data(), a.data(), a.size());
         if (poor.copy_pinned.bufs.size() > 3) { std::puts("more buffers"); return 1; }
+    }
+    {   // a buffer that grows while its last upload may still run
+        gp::PinnedPool pool;
+        gp::PinnedBuf* b = pool.acquire(100);
+        recorded = freed_in_flight = 0;
+        b->record_upload(nullptr);
+        pool.release(b);
+        if (pool.acquire(1 << 20) != b || freed_in_flight) { std::puts("freed in flight"); return 1; }
     }
     std::puts("ok");
     return 0;
